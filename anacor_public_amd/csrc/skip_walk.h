@@ -1,0 +1,486 @@
+// The skip walk: the tracer's A_h kernel on a field of free distances.
+// Included by trace.hip inside namespace anacor, after the stepping kernels.
+//
+// The reference visits every voxel of a ray, although all that a ray's result
+// depends on is how many of its steps fall on each label, where it stops and
+// its last voxel.  Crystal, loop and liquor are regions tens of voxels thick,
+// so nearly all steps repeat the label of the step before.  Per voxel and
+// direction octant the field holds one byte: the label (bits 0-2) and 8 n (bits
+// 3-7), where n is the side (in voxels, at most 31) of a cube that starts at the
+// voxel, extends into the octant and holds that one label.  A ray of the octant
+// whose steps move at most one voxel per axis stays in that cube for n - 1 more
+// steps, so one gather answers n steps: 13 gathers per ray in place of 101 steps on a
+// 256^3 volume (18 against 117 in a wave's longest lane), with the same step
+// counts per label.
+//
+// Positions are exact without FP64 in the loop.  The reference evaluates
+// rnd(c + RN(inc * d)) per stepped axis, c an integer; that is c + rnd(m),
+// m = RN(inc * d), unless c + m rounds up onto the boundary of rnd, which
+// takes an m within 2^-40 below a boundary.  So the offsets from a ray's
+// origin depend on (ray, exit face, increment) only: each workgroup tabulates
+// them in LDS for its reflection and notes the first increment of each face
+// that is too close to call.  A lane that would use it, or whose geometry the
+// table does not cover in any other way, marks its reflection (kRayRedo), and
+// the host traces such reflections with the stepping kernels.
+//
+// Layout of one octant's field: the volume with a one-voxel replicated shell
+// (the reference clamps a stepped coordinate to the volume), tiles of 8 (x) by
+// 16 (y) bytes, one 128-byte line each, so the 64 rays of a wave (neighbours
+// in Morton order) touch about 15 lines per gather against 29 in rows.  x's
+// high bits follow the tile's 7 bits, y's high bits and then z above them: an
+// offset adds to a position in two words, x and yz, whose gaps the table's
+// words fill with ones so that carries run through, and one bit select merges
+// them.
+//
+// What bounds it: VALU issue (71% of one instruction per SIMD every 4 cycles)
+// and the texture addresser (79% busy, 20 cycles per 64-lane byte gather), at
+// once.  256^3, 25,323 voxels, 20,000 reflections: 62.5 ms stepping, 21.6 ms
+// with the first form of this kernel (507 VALU instructions per wave and ray,
+// five waves per SIMD), 17.7 ms with nine instructions per gather and eight
+// waves, 13.8 ms with the diffracted ray leading the sort and rows of lanes
+// within cubes.  181x203x227, 5,003 voxels, 4,001 reflections, FP64 mean: 5.1
+// and 0.95 ms.
+
+constexpr unsigned kRayRedo = 1u << 30;   // err bit: trace with the stepping kernels
+constexpr int kSkipMaxExtent = 2046;      // coordinates in 16 bits, tables in LDS
+constexpr int kSkipVox = 4;               // voxels per lane between two table builds
+constexpr int kLevels = 12;
+// cubes of k + 1 voxels: n - 1 is quantised down to these
+constexpr int kLevelSide[kLevels] = {1, 2, 3, 4, 5, 6, 7, 8, 12, 16, 24, 30};
+
+struct FieldShape {
+  int Z, Y, X;          // volume
+  int nbx, nby;         // tiles of 8 and 16 along padded x and y
+  int hx;               // bits of the x tile index
+  int zs;               // bytes per z plane
+  long long bytes;      // per octant
+  int wx;               // 32-bit words per padded row of a level plane
+};
+
+__host__ __device__ __forceinline__ unsigned dilate_x(int x) {
+  return (unsigned)((x & 7) + (x >> 3) * 128);
+}
+__host__ __device__ __forceinline__ unsigned dilate_y(int y, int hx) {
+  return (unsigned)(((y & 15) << 3) + (y >> 4) * (1 << (7 + hx)));
+}
+
+// -------------------------------------------------------- building the field
+//
+// Level k of the bit planes: the cube [p, p + k]^3 (its part inside the padded
+// volume) holds one label.  Level 1 compares labels; a level a + s, s <= a, is
+// the AND of level a at the eight offsets {0, s}^3 (cubes that share voxels, so
+// their labels agree), 32 voxels per word operation.  The cube of octant o at v starts at v - k on o's negative axes,
+// so one set of planes serves all eight octants.
+
+__device__ __forceinline__ int padded_label(const uint8_t* __restrict__ vol, int Z, int Y, int X,
+                                            int z, int y, int x) {
+  const int cz = min(max(z, 1), Z), cy = min(max(y, 1), Y), cx = min(max(x, 1), X);
+  return vol[((size_t)cz * (Y + 2) + cy) * (X + 2) + cx];   // the raw layout's zero shell
+}
+
+// flag |= 1 when some listed voxel's label is not 3.
+__global__ void origin_label_kernel(const uint8_t* __restrict__ vol, int Y, int X,
+                                    const int4* __restrict__ coords, int n,
+                                    unsigned* __restrict__ flag) {
+  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  bool other = false;
+  if (i < n) {
+    const int4 c = coords[i];
+    other = vol[((size_t)(c.x + 1) * (Y + 2) + c.y + 1) * (X + 2) + c.z + 1] != 3;
+  }
+  if (__any(other) && (threadIdx.x & (kWave - 1)) == 0) atomicOr(flag, 1u);
+}
+
+// Level 1: one wave per 64 voxels of a padded row; bits past the row are 1.
+__global__ void field_base_kernel(const uint8_t* __restrict__ vol, int Z, int Y, int X, int wx,
+                                  long long waves, uint32_t* __restrict__ out) {
+  const long long w = ((long long)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
+  if (w >= waves) return;               // whole waves
+  const int lane = (int)threadIdx.x & (kWave - 1);
+  const int per_row = (wx + 1) / 2;
+  const long long row = w / per_row;
+  const int x = (int)(w - row * per_row) * kWave + lane;
+  const int z = (int)(row / (Y + 2)), y = (int)(row - (long long)z * (Y + 2));
+  // the label of the 2 x 2 column (z, z + 1) x (y, y + 1) at x, or 255
+  auto column = [&](int cx) {
+    const int a = padded_label(vol, Z, Y, X, z, y, cx);
+    const bool same = padded_label(vol, Z, Y, X, z, y + 1, cx) == a &&
+                      padded_label(vol, Z, Y, X, z + 1, y, cx) == a &&
+                      padded_label(vol, Z, Y, X, z + 1, y + 1, cx) == a;
+    return same ? a : 255;
+  };
+  const int c0 = column(x);
+  int c1 = __shfl_down(c0, 1);
+  if (lane == kWave - 1) c1 = column(x + 1);
+  const unsigned long long b = __ballot(x >= X + 2 || (c0 != 255 && c1 == c0));
+  const int word = (x - lane) / 32 + lane;
+  if (lane < 2 && word < wx) out[row * wx + word] = (uint32_t)(b >> (32 * lane));
+}
+
+struct ErodeArgs {
+  const uint32_t* in;
+  uint32_t* out[4];
+  int s[4];
+  int n;
+  int Z2, Y2, wx;       // padded extents, words per row
+};
+
+// Up to four levels from one: AND over the offsets {0, s}^3, 1 outside.
+__global__ void field_erode_kernel(ErodeArgs a) {
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (long long)a.Z2 * a.Y2 * a.wx) return;
+  const int w = (int)(i % a.wx);
+  const long long row = i / a.wx;
+  const int y = (int)(row % a.Y2), z = (int)(row / a.Y2);
+  for (int k = 0; k < a.n; ++k) {
+    const int s = a.s[k];
+    uint32_t v = ~0u;
+    for (int dz = 0; dz < 2; ++dz)
+      for (int dy = 0; dy < 2; ++dy) {
+        if (z + dz * s >= a.Z2 || y + dy * s >= a.Y2) continue;
+        const uint32_t* p = a.in + ((long long)(z + dz * s) * a.Y2 + (y + dy * s)) * a.wx + w;
+        const uint32_t lo = p[0], hi = w + 1 < a.wx ? p[1] : ~0u;
+        v &= lo & ((lo >> s) | (hi << (32 - s)));     // 1 <= s <= 16
+      }
+    a.out[k][i] = v;
+  }
+}
+
+// Eight x neighbours of one padded (z, y) per thread, all eight octants:
+// n from the highest level whose cube holds, clamped to the padded volume on
+// the negative side (a cube cut off there is only smaller); 1 for label 0.
+__global__ void field_pack_kernel(const uint8_t* __restrict__ vol, FieldShape s,
+                                  const uint32_t* __restrict__ planes, long long plane_words,
+                                  uint8_t* __restrict__ field) {
+  const int Z2 = s.Z + 2, Y2 = s.Y + 2;
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (long long)Z2 * s.nby * s.nbx * 16) return;
+  const int yl = (int)(i & 15);
+  const long long t = i >> 4;
+  const int xb = (int)(t % s.nbx);
+  const long long u = t / s.nbx;
+  const int yb = (int)(u % s.nby), z = (int)(u / s.nby);
+  const int y = yb * 16 + yl, x0 = xb * 8;
+  if (y >= Y2) return;
+  uint32_t lab[2] = {0x08080808u, 0x08080808u}, keep[2] = {0, 0};   // n = 1; where more counts
+  for (int e = 0; e < 8; ++e) {
+    const uint32_t l = (uint32_t)padded_label(vol, s.Z, s.Y, s.X, z, y, x0 + e) & 7u;
+    lab[e >> 2] |= l << (8 * (e & 3));
+    keep[e >> 2] |= (l ? 0xf8u : 0u) << (8 * (e & 3));
+  }
+  const long long at = (long long)z * s.zs + (long long)yb * (1ll << (7 + s.hx)) +
+                       ((long long)xb << 7) + (yl << 3);
+  for (int o = 0; o < 8; ++o) {          // bit 2: z falls, bit 1: y falls, bit 0: x falls
+    uint32_t acc[2] = {0, 0};
+    int prev = 0;
+    for (int l = 0; l < kLevels; ++l) {
+      const int k = kLevelSide[l];
+      const int qz = (o & 4) ? max(z - k, 0) : z;
+      const int qy = (o & 2) ? max(y - k, 0) : y;
+      const uint32_t* row = planes + l * plane_words + ((long long)qz * Y2 + qy) * s.wx;
+      const int xs = (o & 1) ? x0 - k : x0;
+      const int b0 = max(xs, 0), w = b0 >> 5;
+      const uint32_t hi = w + 1 < s.wx ? row[w + 1] : ~0u;
+      uint32_t bits = (uint32_t)((((uint64_t)hi << 32) | row[w]) >> (b0 & 31));
+      if (xs < 0) {                      // positions below 0 take row position 0
+        const int n = min(-xs, 8);
+        bits = (bits << n) | ((bits & 1u) ? (1u << n) - 1u : 0u);
+      }
+      bits &= 0xffu;
+      if (!bits) break;                  // higher levels hold larger cubes
+      const uint32_t add = (uint32_t)(k - prev) << 3;
+      prev = k;
+      acc[0] += (((bits & 15u) * 0x00204081u) & 0x01010101u) * add;
+      acc[1] += (((bits >> 4) * 0x00204081u) & 0x01010101u) * add;
+    }
+    uint2 v;
+    v.x = (acc[0] & keep[0]) + lab[0];
+    v.y = (acc[1] & keep[1]) + lab[1];
+    *(uint2*)(field + (long long)o * s.bytes + at) = v;
+  }
+}
+
+// ------------------------------------------------------------- the kernel
+
+struct SkipArgs {
+  const uint8_t* field;        // eight octants
+  long long oct_bytes;
+  int hx, zs;
+  const int4* vox;             // (z | y << 16, x, x word, yz word), wave-grouped
+  int lo[3], hi[3];            // the listed voxels' box (z, y, x): bounds the tables
+  int at[3];                   // first table entry of each exit axis
+};
+
+// The exit along one axis: the upper plane where the direction's sign bit is
+// clear, else the lower one.  Uniform in a workgroup.
+struct AxisExit {
+  bool up, round;
+  int face;                    // index of the face (0..5)
+  int add;                     // increments tried past the distance to the plane
+  __device__ __forceinline__ AxisExit(const RayRule* __restrict__ rr, int axis) {
+    const unsigned hi =
+        (unsigned)((unsigned long long)__double_as_longlong(rr->dir[axis]) >> 32);
+    up = __builtin_amdgcn_readfirstlane((int)((hi >> 31) ^ rr->neg)) == 0;
+    face = axis == 0 ? (up ? 2 : 1) : axis == 1 ? (up ? 4 : 3) : (up ? 0 : 5);
+    const uint32_t meta = rr->meta[face];
+    round = (meta & kMetaRound) != 0;
+    add = up ? ((meta & kMetaInclusive) ? 1 : 0) : 1;
+  }
+};
+
+// What a lane needs of its exit axis, read from LDS by the axis.
+struct AxisLds {
+  int at;                      // byte offset of its table
+  int near;                    // increments from here on are not tabulated (0: none)
+  int scale, add;
+  int hb, hc;                  // extents - 1 of the two stepped axes
+  int face, up;
+  double db, dc;               // deltas of the two stepped axes
+  double vb, vc, vp, bias;     // voxel edges: stepped axes, exit axis; rounding bias
+};
+static_assert(sizeof(AxisLds) == 80, "AxisLds layout");
+
+// Whether the walk may leave along `axis`: the face's precondition holds, and
+// its deltas agree with the direction that chooses the face, so that every
+// origin leaving there keeps its stepped coordinates within a voxel of the
+// volume (ext: largest extent) and moves into the direction's octant.  A NaN
+// fails its comparison.  scale: 65536 / the largest move of a step along the
+// three axes, rounded down.
+__device__ __forceinline__ bool exit_usable(const RayRule* __restrict__ rr, int axis,
+                                            const AxisExit& e, int ext, int& scale) {
+  const int b = axis == 0 ? 1 : 0, c = axis == 2 ? 1 : 2;
+  const double sg = rr->neg ? -1.0 : 1.0;
+  const double ea = __builtin_fabs(rr->dir[axis]), eb = sg * rr->dir[b], ec = sg * rr->dir[c];
+  const double db = rr->d[e.face][b], dc = rr->d[e.face][c];
+  const double mb = __builtin_fabs(db), mc = __builtin_fabs(dc);
+  const double slack = 0.25 / (double)(ext + 1) * ea;
+  const float most = (float)(mb > mc ? mb : mc);
+  scale = most > 0.99999f ? (int)(65536.0f * 0.9999f / most) : 65536;
+  if (mb <= 1.0 && mc <= 1.0) scale = 65536;
+  return (rr->meta[e.face] & kMetaValid) && ea >= 0x1p-500 && ea <= 0x1p500 && mb <= 0x1p20 &&
+         mc <= 0x1p20 && __builtin_fabs(db * ea - eb) <= slack &&
+         __builtin_fabs(dc * ea - ec) <= slack && db * eb >= 0.0 && dc * ec >= 0.0;
+}
+
+// Offset of a stepped axis at m = RN(inc * d); `near` when some origin's
+// c + m could round onto the boundary above.
+__device__ __forceinline__ int step_offset(double m, bool round, bool& near) {
+  const double f = __builtin_floor(m);
+  const double r = m - f;                       // exact; 1 for a tiny negative m
+  const double gap = round ? 0.5 - r : 1.0 - r; // to the boundary above (or past it)
+  near = near || (round ? (gap > 0.0 && gap < 0x1p-40) : gap < 0x1p-40);
+  return (int)f + ((round && r >= 0.5) ? 1 : 0);
+}
+
+// (m & a) | (~m & b), m uniform
+__device__ __forceinline__ unsigned bit_select(unsigned m, unsigned a, unsigned b) {
+  unsigned r;
+  asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(r) : "s"(m), "v"(a), "v"(b));
+  return r;
+}
+
+// sqrt(S) / D for S zero or well inside the exponent range and D a small positive
+// integer: reciprocal and reciprocal root refined to an ulp or two, a third of
+// the instructions of the correctly rounded pair.  The FP64 mean keeps those.
+template <bool EXACT>
+__device__ __forceinline__ double root_over(double S, double D) {
+  if (EXACT) return __builtin_sqrt(S) / D;
+  double y = __builtin_amdgcn_rsq(S);
+  double g = S * y, h = 0.5 * y;
+  double e = __builtin_fma(-h, g, 0.5);
+  g = __builtin_fma(g, e, g);
+  h = __builtin_fma(h, e, h);
+  g = __builtin_fma(__builtin_fma(-g, g, S), h, g);
+  double q = __builtin_amdgcn_rcp(D);
+  q = __builtin_fma(__builtin_fma(-D, q, 1.0), q, q);
+  q = __builtin_fma(__builtin_fma(-D, q, 1.0), q, q);
+  return S > 0.0 ? g * q : 0.0;       // a ray held on its origin by the clamps
+}
+
+template <bool F64>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(F64 ? 6 : 8)))
+void skip_kernel(TraceArgs a, SkipArgs k) {
+  extern __shared__ uint2 tbl[];                // offsets by increment: z, y, x exits
+  __shared__ uint32_t hist[5 * kBlock];         // 8 x steps per label, one column per lane
+  __shared__ AxisLds axes[3];
+  __shared__ double incident[kSkipVox * kBlock];  // the first ray's exponent per voxel
+  __shared__ ReduceLds red;
+
+  const int lb = xcd_logical_block((int)blockIdx.x, (int)gridDim.x);
+  if (lb >= a.n_blocks) return;
+  int pos, tile;
+  block_work(lb, a.tiles, a.R, a.group, pos, tile);
+  pos += a.pos0;
+  const int refl = a.order[pos];
+  const ReflRule* __restrict__ rule = a.rules + refl;
+  const int tid = (int)threadIdx.x;
+  uint32_t* const col = hist + tid;
+#pragma unroll
+  for (int l = 1; l < 5; ++l) col[l * kBlock] = 0;
+  const unsigned mx = 7u | (((1u << k.hx) - 1u) << 7);
+  const unsigned gap_y = mx & ~7u;              // x's high bits: y's carry runs through
+  TileAcc acc = {0.f, 0.f, 0.0, 0ull, 0u};
+  unsigned steps = 0;
+  const int v_begin = tile * a.vox_per_tile;
+  const int v_end = min(a.N, v_begin + a.vox_per_tile);
+
+  for (int s0 = v_begin; s0 < v_end; s0 += kSkipVox * kBlock) {
+#pragma unroll 1
+    for (int ray = 0; ray < 2; ++ray) {
+      const RayRule* __restrict__ rr = &rule->ray[ray];
+      const AxisExit ez(rr, 0), ey(rr, 1), ex(rr, 2);
+      __syncthreads();                          // the table's last readers are done
+      if (tid < 3) {
+        const AxisExit e = tid == 0 ? ez : tid == 1 ? ey : ex;
+        const double* d = rr->d[e.face];
+        AxisLds& A = axes[tid];
+        A.at = k.at[tid] * (int)sizeof(uint2);
+        A.near = exit_usable(rr, tid, e, max(a.Z, max(a.Y, a.X)), A.scale) ? 0x7fffffff : 0;
+        A.add = e.add;
+        A.hb = (tid == 0 ? a.Y : a.Z) - 1;
+        A.hc = (tid == 2 ? a.Y : a.X) - 1;
+        A.face = e.face;
+        A.up = e.up ? 1 : 0;
+        A.db = d[tid == 0 ? 1 : 0];
+        A.dc = d[tid == 2 ? 1 : 2];
+        A.vb = a.vs[tid == 0 ? 1 : 0];
+        A.vc = a.vs[tid == 2 ? 1 : 2];
+        A.vp = a.vs[tid];
+        A.bias = e.round ? kRoundBias : 0.0;
+      }
+      __syncthreads();
+      // offsets of the increments that any listed voxel takes
+      auto build = [&](const AxisExit& e, int axis, int ext) {
+        const int n = (e.up ? ext - k.lo[axis] : k.hi[axis]) + e.add;
+        uint2* const out = tbl + k.at[axis];
+        const double* d = rr->d[e.face];
+        const double db = axis == 0 ? d[1] : d[0], dc = axis == 2 ? d[1] : d[2];
+        int first = 0x7fffffff;
+        for (int inc = tid; inc < n; inc += kBlock) {
+          bool near = false;
+          const int op = e.up ? inc : -inc;
+          const int ob = step_offset((double)inc * db, e.round, near);
+          const int oc = step_offset((double)inc * dc, e.round, near);
+          const int oz = axis == 0 ? op : ob;
+          const int oy = axis == 0 ? ob : axis == 1 ? op : oc;
+          const int ox = axis == 2 ? op : oc;
+          out[inc] = make_uint2(dilate_x(ox) | 0x78u,
+                                (dilate_y(oy, k.hx) | gap_y) + (unsigned)(oz * k.zs));
+          if (near) first = min(first, inc);
+        }
+        if (first != 0x7fffffff) atomicMin(&axes[axis].near, first);
+      };
+      build(ez, 0, a.Z);
+      build(ey, 1, a.Y);
+      build(ex, 2, a.X);
+      __syncthreads();
+      const int oct = (ez.up ? 0 : 4) | (ey.up ? 0 : 2) | (ex.up ? 0 : 1);
+      const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)(k.field + (long long)oct * k.oct_bytes), (short)0, (int)k.oct_bytes, 0x00020000);
+      const float iz = (float)__builtin_fabs(rr->d[0][3]),
+                  iy = (float)__builtin_fabs(rr->d[1][3]),
+                  ix = (float)__builtin_fabs(rr->d[2][3]);
+      // distance to the exit plane along an axis: off + sgn * c
+      const int sz = ez.up ? -1 : 1, sy = ey.up ? -1 : 1, sx = ex.up ? -1 : 1;
+      const int oz = ez.up ? a.Z : 0, oy = ey.up ? a.Y : 0, ox = ex.up ? a.X : 0;
+      const int s1 = min(v_end, s0 + kSkipVox * kBlock);
+#pragma unroll 1
+      for (int v = s0 + tid; v < s1; v += kBlock) {
+        double r = 0.0;
+        {
+          const int4 q = k.vox[v];
+          const int z = q.x & 0xffff, y = (int)((unsigned)q.x >> 16), x = q.y;
+          // cube_face by FP32 products with the reciprocals; FP64 quotients
+          // decide where two planes are closer than the products' rounding
+          const int kz = mad24(z, sz, oz), ky = mad24(y, sy, oy), kx = mad24(x, sx, ox);
+          const float tz = (float)kz * iz, ty = (float)ky * iy, tx = (float)kx * ix;
+          const bool z_first = tz < ty;
+          const float lo = z_first ? tz : ty, hi = z_first ? ty : tz;
+          const bool x_first = tx < lo;
+          const float t0 = x_first ? tx : lo;
+          const float t1 = x_first ? lo : (hi < tx ? hi : tx);
+          int p = x_first ? 2 : z_first ? 0 : 1;
+          bool use = true;
+          if (!(t1 > t0 * 1.00001f) || min(z, min(y, x)) == 0) {
+            const int face = exit_face<true>(z, y, x, rr->dir[0], rr->dir[1], rr->dir[2],
+                                             rr->d[0][3], rr->d[1][3], rr->d[2][3], a.Z, a.Y, a.X,
+                                             rr->neg != 0);
+            p = (face == 2 || face == 3) ? 0 : (face == 4 || face == 5) ? 1 : 2;
+            use = face - 1 == axes[p].face;
+          }
+          const AxisLds& A = axes[p];
+          const int kp = p == 0 ? kz : p == 1 ? ky : kx;
+          const int limit = kp + A.add;
+          if (!use || limit > A.near) {
+            acc.err |= kRayRedo;
+          } else {
+            const int scale = A.scale;
+            const unsigned xw = (unsigned)q.z, yz = (unsigned)q.w;
+            const char* t = (const char*)tbl + A.at;      // the increment's entry
+            const char* const end = t + (limit << 3);
+            int lab;
+            auto walk = [&](bool unit) {
+              do {
+                const uint2 w = *(const uint2*)t;
+                const unsigned off = bit_select(mx, xw + w.x, yz + w.y);
+                const int b = __builtin_amdgcn_raw_buffer_load_b8(rsrc, (int)off, 0, 0);
+                lab = b & 7;
+                int s8 = b & 0xf8;                        // 8 x steps this label holds for
+                if (!unit) s8 = ((int)(__umul24((unsigned)(s8 - 8), (unsigned)scale) >> 16) & ~7) + 8;
+                atomicAdd(col + lab * kBlock, (unsigned)s8);
+                t += s8;
+              } while (lab != 0 && t < end);
+            };
+            // a wave whose rays all step at most one voxel per axis (most)
+            // skips without scaling
+            if (__all(scale == 65536)) walk(true);
+            else walk(false);
+            // a last label past the end counted the steps beyond it too
+            const int over = (int)(t - end);
+            const int len = lab == 0 ? limit + (over >> 3) - 1 : limit;
+            steps += (unsigned)len;
+            const int n8 = max(lab == 0 ? 0 : over, 0);
+            // sum of mu over the steps, label by label
+            double W = a.mu[0] * (double)(int)(col[1 * kBlock] - (lab == 1 ? n8 : 0));
+            W = __builtin_fma(a.mu[1], (double)(int)(col[2 * kBlock] - (lab == 2 ? n8 : 0)), W);
+            W = __builtin_fma(a.mu[2], (double)(int)(col[3 * kBlock] - (lab == 3 ? n8 : 0)), W);
+            W = __builtin_fma(a.mu[3], (double)(int)(col[4 * kBlock] - (lab == 4 ? n8 : 0)), W);
+#pragma unroll
+            for (int l = 1; l < 5; ++l) col[l * kBlock] = 0;
+            if (len > 1) {
+              const int last = len - 1;
+              const double D = (double)last;
+              const int cb = p == 0 ? y : z, cc = p == 2 ? y : x;
+              const int ib = axis_index<false>((double)cb, D, A.db, A.bias, A.hb);
+              const int ic = axis_index<false>((double)cc, D, A.dc, A.bias, A.hc);
+              const int dp = min(last, kp - A.up);
+              const double b_ = (double)(ib - cb) * A.vb;
+              const double c_ = (double)(ic - cc) * A.vc;
+              const double p_ = (double)dp * A.vp;
+              r = root_over<F64>(b_ * b_ + c_ * c_ + p_ * p_, D) * (W * 0.125);
+            }
+          }
+        }
+        double* const first = incident + (v - s0);
+        if (ray == 0) {
+          *first = r;
+          continue;
+        }
+        r += *first;
+        if (F64) {
+          acc.acc64 += a.is_exp ? exp(-r) : r;
+        } else {
+          const float val = a.is_exp ? exp_neg(r) : (float)r;
+          const float yv = val - acc.kc;
+          const float t = acc.ks + yv;
+          acc.kc = (t - acc.ks) - yv;
+          acc.ks = t;
+        }
+      }
+    }
+  }
+  acc.steps = steps;
+  const int slot = pos * a.tiles + tile;
+  reduce_tile<F64, false>(acc, red, &a.err[refl], a.steps, a.partial32 + slot,
+                          a.partial64 + slot);
+}

@@ -931,6 +931,8 @@ void trace_kernel(TraceArgs a) {
                           a.partial64 + slot);
 }
 
+#include "skip_walk.h"
+
 // Per reflection: combine the tile partials in tile order and divide by N.
 __global__ void finish_kernel(const float2* __restrict__ p32, const double* __restrict__ p64,
                               const unsigned* __restrict__ err, const int* __restrict__ order,
@@ -1313,6 +1315,11 @@ struct Context {
   bool labels_over4 = true;              // some label outside 0..4
   int4* d_coords = nullptr;
   int N = 0;
+  // skip walk: eight octants of free distances, the voxel list in its order
+  uint8_t* d_field = nullptr;
+  FieldShape field{};
+  int4* d_skip_vox = nullptr;
+  int box_lo[3] = {0, 0, 0}, box_hi[3] = {0, 0, 0};   // of the voxel list (z, y, x)
   double vs[3] = {1, 1, 1};
   double mu[4] = {0, 0, 0, 0};
   int full = 0;
@@ -1322,6 +1329,7 @@ struct Context {
                                 // -1: automatic (sort_major_for)
   std::vector<int4> h_coords;   // (z, y, x, index) in the caller's order
   int block[3] = {0, 0, 0};     // voxel grouping in use (0,0,0: Morton)
+  bool auto_block = true;       // not asked for by the caller or the environment
   // reusable per-run buffers
   ReflRule* d_rules = nullptr;
   size_t rules_cap = 0;
@@ -1388,7 +1396,8 @@ static int ensure_run_buffers(Context* c, int64_t R, int64_t n_partials, bool f6
     HIP_TRY(hipMalloc(&c->d_order, (size_t)R * sizeof(int)));
     c->refl_cap = (size_t)R;
   }
-  if (!c->d_steps) HIP_TRY(hipMalloc(&c->d_steps, sizeof(unsigned long long)));
+  // two counters: the call's steps, and those of a repeated reflection's first trace
+  if (!c->d_steps) HIP_TRY(hipMalloc(&c->d_steps, 2 * sizeof(unsigned long long)));
   return ANACOR_OK;
 }
 
@@ -1676,19 +1685,38 @@ static void order_by_direction(Context* c, int64_t R, DirOf dir_of, int major) {
 
 static bool is_bricked(int layout) { return layout == kLayoutBrick2 || layout == kLayoutBrick4; }
 
+// Whether the automatic layout takes the skip walk (a layout that the caller
+// or the environment asks for keeps its stepping kernel).
+static bool skip_ready(const Context* c) {
+  return c->d_field && c->layout_req == ANACOR_LAYOUT_AUTO &&
+         !std::getenv("ANACOR_VOLUME_LAYOUT");
+}
+
+// The skip walk for a call of R reflections.  Its tables and barriers cost a
+// few microseconds per workgroup, which short rays in a call too small to fill
+// the GPU do not earn back: 64^3, 3,149 voxels, 16 reflections 20.3 us against
+// the stepping kernel's 17.3, 256 reflections 61.0 and 61.2, 1,024 107 and 205;
+// 128^3, 3,149 voxels, one reflection 17.2 and 21.8, 256 61 and 110.
+static bool use_skip(const Context* c, int64_t R) {
+  return skip_ready(c) && (R * (int64_t)c->N > (1 << 20) || c->Z + c->Y + c->X > 256);
+}
+
 // The ray whose direction leads the sort key.  Automatic: the incident one in
 // the raw layouts; the diffracted one in the bricked layouts, whose launch
 // groups then share the diffracted rays' bricks (1000x1000x800, 10k
 // reflections, groups of 128, 512-voxel tiles: 1,156 ms led by the incident
-// ray, 1,090 ms by the diffracted one).
-static int sort_major_for(const Context* c, int layout) {
+// ray, 1,090 ms by the diffracted one) and in the skip walk (256^3, 20,000
+// reflections: 17.5 and 15.4 ms; incident directions lie on a cone, so the
+// diffracted ones spread far within any run of them).
+static int sort_major_for(const Context* c, int layout, bool skip) {
   if (c->sort_major >= 0) return c->sort_major;
-  return is_bricked(layout) ? 1 : 0;
+  return is_bricked(layout) || skip ? 1 : 0;
 }
 
-static void order_reflections(Context* c, const ReflRule* rules, int64_t R, int layout) {
+static void order_reflections(Context* c, const ReflRule* rules, int64_t R, int layout,
+                              bool skip) {
   order_by_direction(c, R, [rules](int64_t i, int k) { return rules[i].ray[k].dir; },
-                     sort_major_for(c, layout));
+                     sort_major_for(c, layout, skip));
 }
 
 // Reflections per group of the trace launch order (block_work).  Automatic:
@@ -1703,6 +1731,28 @@ static int launch_group(const Context* c, int layout) {
   return (layout == kLayoutBrick2 || layout == kLayoutBrick4) ? kBrickGroup : 1;
 }
 
+static void launch_skip(const Context* c, const TraceArgs& a, int grid, bool f64, hipStream_t s) {
+  SkipArgs k;
+  k.field = c->d_field;
+  k.oct_bytes = c->field.bytes;
+  k.hx = c->field.hx;
+  k.zs = c->field.zs;
+  k.vox = c->d_skip_vox;
+  const int ext[3] = {c->Z, c->Y, c->X};
+  int entries = 0;
+  for (int i = 0; i < 3; ++i) {
+    k.lo[i] = c->box_lo[i];
+    k.hi[i] = c->box_hi[i];
+    k.at[i] = entries;
+    entries += std::max(ext[i] - k.lo[i], k.hi[i]) + 1;
+  }
+  const unsigned lds = (unsigned)(entries * sizeof(uint2));
+  if (f64)
+    hipLaunchKernelGGL((skip_kernel<true>), dim3((unsigned)grid), dim3(kBlock), lds, s, a, k);
+  else
+    hipLaunchKernelGGL((skip_kernel<false>), dim3((unsigned)grid), dim3(kBlock), lds, s, a, k);
+}
+
 // Device buffers of one trace call: the context's grow-only ones
 // (ensure_run_buffers) or, for anacor_ctx_run_noalloc, parts of the static
 // scratch array.
@@ -1712,7 +1762,7 @@ struct RunBuffers {
   unsigned* err = nullptr;             // [R] per-reflection error bits
   double* out = nullptr;               // [R] means
   void* partial = nullptr;             // [R * tiles] float2 or double
-  unsigned long long* steps = nullptr; // voxel-step counter
+  unsigned long long* steps = nullptr; // [2] voxel-step counter, repeated steps
 };
 
 // Clears what a trace call accumulates into (a fill kernel rather than
@@ -1721,7 +1771,102 @@ __global__ void clear_run_kernel(unsigned* __restrict__ err, int R,
                                  unsigned long long* __restrict__ steps) {
   const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   if (i < R) err[i] = 0u;
-  if (i == 0) *steps = 0ull;
+  if (i == 0 && steps) *steps = 0ull;
+}
+
+// The kernel arguments of a trace in `layout` with vpt voxels per tile; the
+// launch's reflections (R, pos0, n_blocks) are the caller's.
+static TraceArgs trace_args(const Context* c, const RunBuffers& B, int vpt, int layout, int flags,
+                            PathRecord* d_paths) {
+  TraceArgs a;
+  const bool bricked = is_bricked(layout);
+  a.vol = bricked ? c->d_pack : c->d_vol;
+  a.vol_bytes = bricked ? (int)c->pack_bytes : (int)c->vol_bytes;
+  a.cz = 512 * c->NBX * c->NBY - 512;
+  a.cy = 512 * c->NBX - 64;
+  a.Z = c->Z; a.Y = c->Y; a.X = c->X;
+  a.coords = c->d_coords;
+  a.N = c->N;
+  a.rules = B.rules;
+  a.R = 0;
+  a.pos0 = 0;
+  a.tiles = (c->N + vpt - 1) / vpt;
+  a.vox_per_tile = vpt;
+  a.n_blocks = 0;
+  for (int i = 0; i < 3; ++i) a.vs[i] = c->vs[i];
+  for (int i = 0; i < 4; ++i) a.mu[i] = c->mu[i];
+  a.is_exp = (flags & ANACOR_FLAG_NO_EXP) ? 0 : 1;
+  a.partial32 = (float2*)B.partial;
+  a.partial64 = (double*)B.partial;
+  a.err = B.err;
+  a.steps = B.steps;
+  a.paths = d_paths;
+  a.order = B.order;
+  a.incd = c->d_incd;
+  a.incd_last = c->incd_last;
+  a.group = launch_group(c, layout);
+  return a;
+}
+
+// The reflections that the skip walk marked (kRayRedo in h_err[R], downloaded
+// by the caller with their means NaN) once more with the stepping kernel:
+// their means into out, their error words into h_err, and the step count in
+// *steps corrected (the marked reflections' blocks had counted what they
+// walked, which a second skip walk of them alone counts again; *repeated sums
+// those over the calls that share a counter).  h_redo: R words of work space.  Synchronous; nothing to do is the usual case.
+static int retrace_marked(Context* c, const RunBuffers& B, const ReflRule* h_rules, int64_t R,
+                          int vpt, int layout, int flags, double* out, unsigned* h_err,
+                          int* h_redo, unsigned long long* steps,
+                          unsigned long long* repeated) {
+  int n = 0;
+  bool guard = false;
+  for (int64_t i = 0; i < R; ++i)
+    if (h_err[i] & kRayRedo) {
+      h_redo[n++] = (int)i;
+      guard = guard || h_rules[i].ray[0].guard || h_rules[i].ray[1].guard;
+    }
+  if (n == 0) return ANACOR_OK;
+  const bool f64 = (flags & ANACOR_FLAG_F64_MEAN) != 0;
+  const unsigned words = (unsigned)((R + 255) / 256);
+  HIP_TRY(hipMemcpyAsync(B.order, h_redo, (size_t)n * sizeof(int), hipMemcpyHostToDevice,
+                         c->stream));
+  TraceArgs a = trace_args(c, B, vpt, layout, flags, nullptr);
+  const int per_launch = (int)std::max<int64_t>(1, kMaxBlocks / a.tiles);
+  hipLaunchKernelGGL(clear_run_kernel, dim3(words), dim3(256), 0, c->stream, B.err, (int)R,
+                     B.steps + 1);
+  HIP_TRY(hipGetLastError());
+  for (int pass = 0; pass < 2; ++pass) {
+    if (pass == 1) {     // the error words the stepping kernel will set
+      hipLaunchKernelGGL(clear_run_kernel, dim3(words), dim3(256), 0, c->stream, B.err, (int)R,
+                         (unsigned long long*)nullptr);
+      HIP_TRY(hipGetLastError());
+    }
+    a.steps = pass == 0 ? B.steps + 1 : B.steps;
+    for (int p0 = 0; p0 < n; p0 += per_launch) {
+      a.R = std::min(per_launch, n - p0);
+      a.pos0 = p0;
+      a.n_blocks = a.R * a.tiles;
+      const int grid = (a.n_blocks + 7) / 8 * 8;
+      if (pass == 0) launch_skip(c, a, grid, f64, c->stream);
+      else dispatch_trace(a, grid, guard, c->full != 0, layout, f64, false, !c->labels_over4,
+                          c->stream);
+      HIP_TRY(hipGetLastError());
+    }
+  }
+  hipLaunchKernelGGL(finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream,
+                     (const float2*)B.partial, (const double*)B.partial, B.err, B.order, n,
+                     a.tiles, c->N, f64 ? 1 : 0, B.out);
+  HIP_TRY(hipGetLastError());
+  unsigned long long count[2] = {0, 0};
+  HIP_TRY(hipMemcpyAsync(out, B.out, (size_t)R * sizeof(double), hipMemcpyDeviceToHost,
+                         c->stream));
+  HIP_TRY(hipMemcpyAsync(h_err, B.err, (size_t)R * sizeof(unsigned), hipMemcpyDeviceToHost,
+                         c->stream));
+  HIP_TRY(hipMemcpyAsync(count, B.steps, sizeof(count), hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(hipStreamSynchronize(c->stream));
+  *repeated += count[1];
+  *steps = count[0] - *repeated;
+  return ANACOR_OK;
 }
 
 // One trace of R reflections from their host rules h_rules and processing
@@ -1734,13 +1879,14 @@ __global__ void clear_run_kernel(unsigned* __restrict__ err, int R,
 // rules and order of positions [0, first) (reflections [0, first)) go up and
 // their trace is launched, then prepare_rest() fills h_rules and h_order for
 // [first, R) on the host while the GPU traces the first part, and those go
-// up and are traced behind it.
+// up and are traced behind it.  h_redo: R words of host work space.
 static int trace_call(Context* c, const RunBuffers& B, const ReflRule* h_rules,
                       const int* h_order, int64_t R, int vpt, int layout, int flags, double* out,
-                      PathRecord* d_paths, PathRecord* paths_out, unsigned* h_err,
+                      PathRecord* d_paths, PathRecord* paths_out, unsigned* h_err, int* h_redo,
                       int64_t first = -1, const std::function<int()>& prepare_rest = {}) {
   const bool f64 = (flags & ANACOR_FLAG_F64_MEAN) != 0;
   const bool paths = paths_out != nullptr;
+  const bool skip = !paths && use_skip(c, R);
   const int64_t tiles = (c->N + vpt - 1) / vpt;
   const int64_t nblk = R * tiles;
   const int64_t RA = (prepare_rest && first > 0 && first < R) ? first : R;
@@ -1759,32 +1905,7 @@ static int trace_call(Context* c, const RunBuffers& B, const ReflRule* h_rules,
                      B.err, (int)R, B.steps);
   HIP_TRY(hipGetLastError());
 
-  TraceArgs a;
-  const bool bricked = layout == kLayoutBrick2 || layout == kLayoutBrick4;
-  a.vol = bricked ? c->d_pack : c->d_vol;
-  a.vol_bytes = bricked ? (int)c->pack_bytes : (int)c->vol_bytes;
-  a.cz = 512 * c->NBX * c->NBY - 512;
-  a.cy = 512 * c->NBX - 64;
-  a.Z = c->Z; a.Y = c->Y; a.X = c->X;
-  a.coords = c->d_coords;
-  a.N = c->N;
-  a.rules = B.rules;
-  a.R = 0;                     // per launch, below
-  a.tiles = (int)tiles;
-  a.vox_per_tile = vpt;
-  a.n_blocks = 0;
-  for (int i = 0; i < 3; ++i) a.vs[i] = c->vs[i];
-  for (int i = 0; i < 4; ++i) a.mu[i] = c->mu[i];
-  a.is_exp = (flags & ANACOR_FLAG_NO_EXP) ? 0 : 1;
-  a.partial32 = (float2*)B.partial;
-  a.partial64 = (double*)B.partial;
-  a.err = B.err;
-  a.steps = B.steps;
-  a.paths = d_paths;
-  a.order = B.order;
-  a.incd = c->d_incd;
-  a.incd_last = c->incd_last;
-  a.group = launch_group(c, layout);
+  TraceArgs a = trace_args(c, B, vpt, layout, flags, d_paths);
 
   // a dispatch holds at most kMaxBlocks workgroups: a longer call runs as
   // several launches of whole reflections (consecutive processing positions)
@@ -1795,8 +1916,10 @@ static int trace_call(Context* c, const RunBuffers& B, const ReflRule* h_rules,
       a.R = (int)Rc;
       a.pos0 = (int)p0;
       a.n_blocks = (int)(Rc * tiles);
-      dispatch_trace(a, (int)((Rc * tiles + 7) / 8 * 8), guard, c->full != 0, layout, f64,
-                     paths, !c->labels_over4, c->stream);
+      const int grid = (int)((Rc * tiles + 7) / 8 * 8);
+      if (skip) launch_skip(c, a, grid, f64, c->stream);
+      else dispatch_trace(a, grid, guard, c->full != 0, layout, f64, paths, !c->labels_over4,
+                          c->stream);
       HIP_TRY(hipGetLastError());
     }
     return ANACOR_OK;
@@ -1848,6 +1971,12 @@ static int trace_call(Context* c, const RunBuffers& B, const ReflRule* h_rules,
     h_err = tmp.data();
   }
   HIP_TRY(hipMemcpy(h_err, B.err, (size_t)R * sizeof(unsigned), hipMemcpyDeviceToHost));
+  if (skip) {
+    unsigned long long repeated = 0;
+    rc = retrace_marked(c, B, h_rules, R, vpt, layout, flags, out, h_err, h_redo, &c->last_steps,
+                        &repeated);
+    if (rc) return rc;
+  }
   for (int64_t i = 0; i < R; ++i)
     if (h_err[i]) {
       set_error(ANACOR_ERR_GEOMETRY,
@@ -1882,7 +2011,7 @@ static int run_rules(Context* c, const ReflRule* h_rules, int64_t R, int flags, 
     if (rc) return rc;
     layout = c->layout;
   }
-  const int vpt = paths ? kBlock : choose_tile(c, R, layout);
+  const int vpt = paths ? kBlock : choose_tile(c, R, use_skip(c, R) ? -1 : layout);
   const int64_t tiles = (c->N + vpt - 1) / vpt;
   if (R > (int64_t)INT32_MAX / 2 || R * tiles > ((int64_t)1 << 40)) {
     set_error(ANACOR_ERR_ARG, "%lld reflections x %lld tiles in one call", (long long)R,
@@ -1892,7 +2021,7 @@ static int run_rules(Context* c, const ReflRule* h_rules, int64_t R, int flags, 
   rc = ensure_run_buffers(c, R, R * tiles, f64);
   if (rc) return rc;
   const int64_t RA = (!paths && setup_rest && first > 0 && first < R) ? first : R;
-  order_reflections(c, h_rules, RA, layout);
+  order_reflections(c, h_rules, RA, layout, use_skip(c, R));
   HIP_TRY(c->h_order_pin.reserve((size_t)R));
   for (int64_t i = 0; i < RA; ++i) c->h_order_pin[(size_t)i] = c->h_order[(size_t)i];
   // the second part: its setup, then its own direction order, as positions
@@ -1904,7 +2033,8 @@ static int run_rules(Context* c, const ReflRule* h_rules, int64_t R, int flags, 
     std::vector<int> ord((size_t)n);
     std::vector<uint64_t> key((size_t)n), tmp((size_t)n);
     direction_order(n, [&](int64_t i, int k) { return h_rules[RA + i].ray[k].dir; },
-                    ord.data(), key.data(), tmp.data(), sort_major_for(c, layout));
+                    ord.data(), key.data(), tmp.data(),
+                    sort_major_for(c, layout, use_skip(c, R)));
     for (int64_t i = 0; i < n; ++i)
       c->h_order_pin[(size_t)(RA + i)] = (int)RA + ord[(size_t)i];
     return ANACOR_OK;
@@ -1920,9 +2050,10 @@ static int run_rules(Context* c, const ReflRule* h_rules, int64_t R, int flags, 
   B.steps = c->d_steps;
   if (RA < R)
     return trace_call(c, B, h_rules, c->h_order_pin.data(), R, vpt, layout, flags, out,
-                      (PathRecord*)paths_buf.p, paths_out, nullptr, RA, prepare_rest);
+                      (PathRecord*)paths_buf.p, paths_out, nullptr, c->h_order_pin.data(), RA,
+                      prepare_rest);
   return trace_call(c, B, h_rules, c->h_order_pin.data(), R, vpt, layout, flags, out,
-                    (PathRecord*)paths_buf.p, paths_out, nullptr);
+                    (PathRecord*)paths_buf.p, paths_out, nullptr, c->h_order_pin.data());
 }
 
 static void ctx_destroy(Context* c);
@@ -1976,9 +2107,145 @@ static int upload_voxel_order(Context* c, int bz, int by, int bx) {
   return ANACOR_OK;
 }
 
+// The skip walk's voxel list: cubes that hold about one wave's voxels, in
+// Morton order, and rows along x inside a cube, so that the four lanes of an
+// address quad mostly fall into one line of the field; or the grouping that
+// the caller asked for.
+static int upload_skip_voxels(Context* c) {
+  const size_t n = c->h_coords.size();
+  for (int i = 0; i < 3; ++i) {
+    c->box_lo[i] = kSkipMaxExtent;
+    c->box_hi[i] = 0;
+  }
+  for (const int4& q : c->h_coords) {
+    const int p[3] = {q.x, q.y, q.z};
+    for (int i = 0; i < 3; ++i) {
+      c->box_lo[i] = std::min(c->box_lo[i], p[i]);
+      c->box_hi[i] = std::max(c->box_hi[i], p[i]);
+    }
+  }
+  std::vector<int4> v(n);
+  if (c->block[0] > 0 && !c->auto_block) {
+    HIP_TRY(hipMemcpy(v.data(), c->d_coords, n * sizeof(int4), hipMemcpyDeviceToHost));
+  } else {
+    // a crystal fills about half of its box
+    double box = 0.5;
+    for (int i = 0; i < 3; ++i) box *= c->box_hi[i] - c->box_lo[i] + 1;
+    const int e = (int)std::lround(std::log2(std::max(1.0, std::cbrt(kWave * box / (double)n))));
+    auto key_of = [e](const int4& q) {   // coordinates below 2^11: 33 bits
+      const uint64_t low = (1ull << e) - 1;
+      const uint64_t z = (uint64_t)q.x, y = (uint64_t)q.y, x = (uint64_t)q.z;
+      const uint64_t cube = (spread_bits(z >> e) << 2) | (spread_bits(y >> e) << 1) |
+                            spread_bits(x >> e);
+      return (cube << (3 * e)) | ((z & low) << (2 * e)) | ((y & low) << e) | (x & low);
+    };
+    if (n < (size_t(1) << 22)) {
+      std::vector<uint64_t> key(n), tmp(n);
+      for (size_t i = 0; i < n; ++i) key[i] = (key_of(c->h_coords[i]) << 22) | (uint64_t)i;
+      radix_sort_high(key.data(), tmp.data(), (int64_t)n, 22);
+      for (size_t i = 0; i < n; ++i) v[i] = c->h_coords[(size_t)(key[i] & ((1u << 22) - 1))];
+    } else {
+      v = c->h_coords;
+      std::stable_sort(v.begin(), v.end(), [&](const int4& a, const int4& b) {
+        return key_of(a) < key_of(b);
+      });
+    }
+  }
+  const FieldShape& f = c->field;
+  for (int4& q : v) {
+    const int z = q.x, y = q.y, x = q.z;
+    q = make_int4(z | (y << 16), x, (int)dilate_x(x + 1),
+                  (int)(dilate_y(y + 1, f.hx) + (unsigned)((z + 1) * f.zs)));
+  }
+  if (!c->d_skip_vox) HIP_TRY(hipMalloc(&c->d_skip_vox, n * sizeof(int4)));
+  HIP_TRY(hipMemcpy(c->d_skip_vox, v.data(), n * sizeof(int4), hipMemcpyHostToDevice));
+  return ANACOR_OK;
+}
+
+// The skip walk's field, where the walk's rules hold: no full_iteration, every
+// label in 0..4, every listed voxel of label 3, finite coefficients and voxel
+// edges whose squares are normal, extents within the tables and offsets.
+// Without the device memory for it the stepping kernels trace as before.
+static int field_build(Context* c) {
+  FieldShape f;
+  f.Z = c->Z; f.Y = c->Y; f.X = c->X;
+  const int Z2 = c->Z + 2, Y2 = c->Y + 2, X2 = c->X + 2;
+  if (c->N == 0 || c->full || c->labels_over4 ||
+      std::max(c->Z, std::max(c->Y, c->X)) > kSkipMaxExtent)
+    return ANACOR_OK;
+  for (double v : c->mu)
+    if (!(std::fabs(v) < 0x1p300)) return ANACOR_OK;
+  for (double v : c->vs)
+    if (!(std::fabs(v) > 0x1p-300 && std::fabs(v) < 0x1p300)) return ANACOR_OK;
+  f.nbx = (X2 + 7) / 8;
+  f.nby = (Y2 + 15) / 16;
+  f.hx = 0;
+  while ((1 << f.hx) < f.nbx) ++f.hx;
+  const int64_t zs = (int64_t)f.nby << (7 + f.hx);
+  if (zs * Z2 >= (1ll << 31)) return ANACOR_OK;
+  f.zs = (int)zs;
+  f.bytes = zs * Z2;
+  f.wx = (X2 + 31) / 32;
+  const long long plane = (long long)Z2 * Y2 * f.wx;
+  DeviceTemp planes, flag;
+  if (hipMalloc(&planes.p, (size_t)plane * kLevels * sizeof(uint32_t)) != hipSuccess ||
+      hipMalloc(&c->d_field, (size_t)f.bytes * 8) != hipSuccess) {
+    (void)hipGetLastError();
+    c->d_field = nullptr;
+    return ANACOR_OK;
+  }
+  HIP_TRY(hipMalloc(&flag.p, sizeof(unsigned)));
+  HIP_TRY(hipMemsetAsync(flag.p, 0, sizeof(unsigned), c->stream));
+  hipLaunchKernelGGL(origin_label_kernel, dim3((unsigned)((c->N + 255) / 256)), dim3(256), 0,
+                     c->stream, c->d_vol, c->Y, c->X, c->d_coords, c->N, (unsigned*)flag.p);
+  HIP_TRY(hipGetLastError());
+  uint32_t* const P = (uint32_t*)planes.p;
+  const long long waves = (long long)Z2 * Y2 * ((f.wx + 1) / 2);
+  hipLaunchKernelGGL(field_base_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, c->stream,
+                     c->d_vol, c->Z, c->Y, c->X, f.wx, waves, P);
+  HIP_TRY(hipGetLastError());
+  // by index into kLevelSide: 1 -> 2; 2 -> 3, 4; 4 -> 5 .. 8; 8 -> 12, 16; 16 -> 24, 30
+  struct Pass { int from, n, to[4], s[4]; };
+  static const Pass passes[] = {{0, 1, {1}, {1}},
+                                {1, 2, {2, 3}, {1, 2}},
+                                {3, 4, {4, 5, 6, 7}, {1, 2, 3, 4}},
+                                {7, 2, {8, 9}, {4, 8}},
+                                {9, 2, {10, 11}, {8, 14}}};
+  for (const Pass& p : passes) {
+    ErodeArgs e{};
+    e.in = P + p.from * plane;
+    e.n = p.n;
+    for (int i = 0; i < p.n; ++i) {
+      e.out[i] = P + p.to[i] * plane;
+      e.s[i] = p.s[i];
+    }
+    e.Z2 = Z2; e.Y2 = Y2; e.wx = f.wx;
+    hipLaunchKernelGGL(field_erode_kernel, dim3((unsigned)((plane + 255) / 256)), dim3(256), 0,
+                       c->stream, e);
+    HIP_TRY(hipGetLastError());
+  }
+  const long long threads = (long long)Z2 * f.nby * f.nbx * 16;
+  hipLaunchKernelGGL(field_pack_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
+                     c->stream, c->d_vol, f, P, plane, c->d_field);
+  HIP_TRY(hipGetLastError());
+  c->field = f;
+  const int rc = upload_skip_voxels(c);   // host work beside the kernels
+  if (rc) return rc;
+  unsigned other = 0;
+  HIP_TRY(hipMemcpyAsync(&other, flag.p, sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(hipStreamSynchronize(c->stream));
+  if (other) {
+    HIP_TRY(hipFree(c->d_field));
+    c->d_field = nullptr;
+  }
+  return ANACOR_OK;
+}
+
+// reflections: how many the caller is about to trace when the context serves
+// that call only (0: a context that is kept).
 static int ctx_create(const uint8_t* vol, const int64_t shape[3], const int64_t* coords,
                       const int32_t* coords32, int64_t n, const double vs[3], const double mu[4],
-                      int full, int device, Context** out) {
+                      int full, int device, Context** out, int64_t reflections = 0) {
   *out = nullptr;
   if (!vol || !shape) {
     set_error(ANACOR_ERR_ARG, "null volume or shape");
@@ -2078,7 +2345,16 @@ static int ctx_create(const uint8_t* vol, const int64_t shape[3], const int64_t*
     if ((int64_t)nvox > (64ll << 20)) blk[0] = blk[1] = blk[2] = 0;
     if (const char* e = std::getenv("ANACOR_VOXEL_BLOCK"))
       if (std::sscanf(e, "%d,%d,%d", &blk[0], &blk[1], &blk[2]) != 3) blk[0] = blk[1] = blk[2] = 0;
-    return upload_voxel_order(c, blk[0], blk[1], blk[2]);
+    c->auto_block = std::getenv("ANACOR_VOXEL_BLOCK") == nullptr;
+    const int rc = upload_voxel_order(c, blk[0], blk[1], blk[2]);
+    if (rc) return rc;
+    // volumes in bricks keep the bricked walk, whose bytes the L2s hold
+    //; a one-shot call builds the field where its steps
+    // (about a sixth of the extents' sum per ray) cost more than the field does
+    const double steps = (double)reflections * (double)n * (c->Z + c->Y + c->X) / 3.0;
+    if (nvox > (64ull << 20) || (reflections > 0 && steps < 1e9 + 300.0 * (double)nvox))
+      return ANACOR_OK;
+    return field_build(c);
   };
   const int rc = init();
   if (rc != ANACOR_OK) {
@@ -2097,6 +2373,8 @@ static void ctx_destroy(Context* c) {
   if (c->d_incd) (void)hipFree(c->d_incd);
   if (c->d_pack) (void)hipFree(c->d_pack);
   if (c->d_coords) (void)hipFree(c->d_coords);
+  if (c->d_field) (void)hipFree(c->d_field);
+  if (c->d_skip_vox) (void)hipFree(c->d_skip_vox);
   if (c->d_rules) (void)hipFree(c->d_rules);
   if (c->d_partial) (void)hipFree(c->d_partial);
   if (c->d_err) (void)hipFree(c->d_err);
@@ -2250,14 +2528,15 @@ static int ctx_run_noalloc(Context* c, const double* s1, const double* omega, in
   // the tile of anacor_ctx_run, enlarged until R * tiles fits the partials
   rc = ensure_layout(c, /*may_build=*/false);
   if (rc) return rc;
-  int64_t vpt = choose_tile(c, R, c->layout);
+  int64_t vpt = choose_tile(c, R, use_skip(c, R) ? -1 : c->layout);
   const int64_t max_tiles = kNoAllocMaxPartials / R;
   if ((c->N + vpt - 1) / vpt > max_tiles) vpt = (c->N + max_tiles - 1) / max_tiles;
   const auto t0 = std::chrono::steady_clock::now();
   // one host thread: the setup spawns none
   host_setup(s1, omega, R, raw_xray, omega_axis, F, max_dim(c), g_noalloc_rules, nullptr, 1);
   direction_order(R, [](int64_t i, int k) { return g_noalloc_rules[i].ray[k].dir; },
-                  g_noalloc_order, g_noalloc_key, g_noalloc_key2, sort_major_for(c, c->layout));
+                  g_noalloc_order, g_noalloc_key, g_noalloc_key2,
+                  sort_major_for(c, c->layout, use_skip(c, R)));
   c->last_host_ms = ms_since(t0);
   RunBuffers B;
   B.rules = (ReflRule*)(base + kScratchRules);
@@ -2267,7 +2546,7 @@ static int ctx_run_noalloc(Context* c, const double* s1, const double* omega, in
   B.out = (double*)(base + kScratchOut);
   B.steps = (unsigned long long*)(base + kScratchSteps);
   return trace_call(c, B, g_noalloc_rules, g_noalloc_order, R, (int)vpt, c->layout, flags, out,
-                    nullptr, nullptr, g_noalloc_err);
+                    nullptr, nullptr, g_noalloc_err, g_noalloc_order);
 }
 
 // Build a contiguous copy of an int8*** row-pointer table (python_2_c_3d,
@@ -2405,7 +2684,7 @@ static int batch_create(const anacor_sample_t* in, int n, int full, int device, 
   BATCH_TRY(hipEventCreateWithFlags(&b->fork, hipEventDisableTiming));
   BATCH_TRY(hipEventCreate(&b->ev0));
   BATCH_TRY(hipEventCreate(&b->ev1));
-  BATCH_TRY(hipMalloc(&b->d_counters, sizeof(unsigned long long)));
+  BATCH_TRY(hipMalloc(&b->d_counters, 2 * sizeof(unsigned long long)));
 #undef BATCH_TRY
   *out = b;
   return ANACOR_OK;
@@ -2421,7 +2700,7 @@ static void batch_setup_sample(void* p) {
   const auto t0 = std::chrono::steady_clock::now();
   host_setup(j->s1, j->omega, j->R, b->geo, b->geo + 3, b->geo + 6, max_dim(c),
              c->h_rules.data(), nullptr, host_threads(0));
-  order_reflections(c, c->h_rules.data(), j->R, kLayoutRaw);
+  order_reflections(c, c->h_rules.data(), j->R, kLayoutRaw, use_skip(c, j->R));
   bool guard = false;
   for (int64_t r = 0; r < j->R; ++r) {
     c->h_order_pin[(size_t)r] = c->h_order[(size_t)r];
@@ -2489,9 +2768,11 @@ static int batch_enqueue(Batch* b, bool capture, bool f64, int is_exp, long long
     // a graph is captured before any setup has run: it holds the unguarded
     // kernel, and a run whose rays need the guard is traced again without it
     const bool guard = !capture && job.guard;
-    dispatch_trace(t, (t.n_blocks + 7) / 8 * 8, guard, b->full != 0,
-                   raw_needs_wide(c) ? kLayoutWide : kLayoutRaw, f64, false, !c->labels_over4,
-                   b->stream);
+    const int grid = (t.n_blocks + 7) / 8 * 8;
+    if (use_skip(c, job.R)) launch_skip(c, t, grid, f64, b->stream);
+    else dispatch_trace(t, grid, guard, b->full != 0,
+                        raw_needs_wide(c) ? kLayoutWide : kLayoutRaw, f64, false,
+                        !c->labels_over4, b->stream);
     HIP_TRY(hipGetLastError());
   }
   // rejoin copy_stream (a captured fork must end joined)
@@ -2627,6 +2908,7 @@ static int batch_run(Batch* b, const double* const* s1, const double* const* ome
                       (int64_t)(intptr_t)c->d_rules, (int64_t)(intptr_t)c->d_order,
                       (int64_t)(intptr_t)c->d_partial, (int64_t)(intptr_t)c->d_err,
                       (int64_t)(intptr_t)c->d_out, (int64_t)(intptr_t)c->d_coords,
+                      (int64_t)use_skip(c, R[i]), (int64_t)(intptr_t)c->d_skip_vox,
                       (int64_t)(intptr_t)c->h_rules.data(),
                       (int64_t)(intptr_t)c->h_order_pin.data()})
       key.push_back(v);
@@ -2661,8 +2943,9 @@ static int batch_run(Batch* b, const double* const* s1, const double* const* ome
   };
   int rc = launch(use_graph);
   if (rc != ANACOR_OK) return rc;
-  bool guard = false;
-  for (const BatchJob& j : b->jobs) guard = guard || j.guard;
+  bool guard = false;   // a stepping kernel's rays (the skip walk marks its own)
+  for (const BatchJob& j : b->jobs)
+    guard = guard || (j.guard && !use_skip(b->samples[(size_t)j.i], j.R));
   b->last_graph = use_graph;
   if (use_graph && guard) {   // rays beyond the int64 range: the guarded kernels, live
     rc = launch(false);
@@ -2676,6 +2959,30 @@ static int batch_run(Batch* b, const double* const* s1, const double* const* ome
     Context* c = b->samples[(size_t)i];
     if (c->N == 0)
       for (int64_t r = 0; r < R[i]; ++r) out[i][r] = __builtin_nan("");
+  }
+  // reflections the skip walk marked: retraced sample by sample, on the
+  // sample's own stream (the batch's has been waited for)
+  unsigned long long repeated = 0;
+  for (int i = 0; i < S; ++i) {
+    Context* c = b->samples[(size_t)i];
+    if (R[i] == 0 || c->N == 0 || !use_skip(c, R[i])) continue;
+    bool any = false;
+    for (int64_t r = 0; r < R[i] && !any; ++r) any = out[i][r] != out[i][r];
+    if (!any) continue;
+    std::vector<unsigned> err((size_t)R[i]);
+    HIP_TRY(hipMemcpy(err.data(), c->d_err, err.size() * sizeof(unsigned),
+                      hipMemcpyDeviceToHost));
+    RunBuffers B;
+    B.rules = c->d_rules;
+    B.order = c->d_order;
+    B.err = c->d_err;
+    B.out = c->d_out;
+    B.partial = c->d_partial;
+    B.steps = b->d_counters;
+    rc = retrace_marked(c, B, c->h_rules.data(), R[i], b->h_desc[(size_t)i].vpt,
+                        raw_needs_wide(c) ? kLayoutWide : kLayoutRaw, flags, out[i], err.data(),
+                        c->h_order_pin.data(), &b->last_steps, &repeated);
+    if (rc != ANACOR_OK) return rc;
   }
   // report the first reflection the reference would have aborted on
   for (int i = 0; i < S; ++i)
@@ -3460,7 +3767,10 @@ int anacor_ctx_set_voxel_block(anacor_ctx* ctx, int bz, int by, int bx) {
   if (!ctx) return ANACOR_ERR_ARG;
   std::lock_guard<std::mutex> lk(ctx->c->mu_run);
   HIP_TRY(hipSetDevice(ctx->c->device));
-  return upload_voxel_order(ctx->c, bz, by, bx);
+  const int rc = upload_voxel_order(ctx->c, bz, by, bx);
+  if (rc || !ctx->c->d_field) return rc;
+  ctx->c->auto_block = false;
+  return upload_skip_voxels(ctx->c);
 }
 
 int anacor_ctx_set_order(anacor_ctx* ctx, int refl_group, int direction_major) {
@@ -3487,7 +3797,7 @@ int anacor_ctx_get_work_shape(const anacor_ctx* ctx, int block[3], int* tile, in
     for (int i = 0; i < 3; ++i) block[i] = c->block[i];
   if (tile) *tile = c->tile_voxels;
   if (refl_group) *refl_group = launch_group(c, c->layout);
-  if (direction_major) *direction_major = sort_major_for(c, c->layout);
+  if (direction_major) *direction_major = sort_major_for(c, c->layout, skip_ready(c));
   return ANACOR_OK;
 }
 
@@ -3648,7 +3958,7 @@ double* ray_tracing_overall(int64_t low, int64_t up, int64_t* coord_list, int64_
   const uint8_t* vol = flatten_table(label_list, shape, storage);
   Context* c = nullptr;
   if (ctx_create(vol, shape, coord_list, nullptr, len_coord_list, voxel_size, coefficients,
-                 full_iteration, 0, &c) != ANACOR_OK) {
+                 full_iteration, 0, &c, std::max<int64_t>(R, 1)) != ANACOR_OK) {
     fprintf(stderr, "anacor: ray_tracing_overall: %s\n", g_err);
     return result;
   }
@@ -3696,7 +4006,7 @@ float* ray_tracing_gpu_overall(size_t low, size_t up, int* coord_list, size_t le
   for (int i = 0; i < 4; ++i) mu[i] = coefficients[i];
   Context* c = nullptr;
   if (ctx_create(vol, shp, nullptr, coord_list, (int64_t)len_coord_list, vs, mu, full_iteration,
-                 0, &c) != ANACOR_OK) {
+                 0, &c, std::max<int64_t>(R, 1)) != ANACOR_OK) {
     fprintf(stderr, "anacor: ray_tracing_gpu_overall: %s\n", g_err);
     return result;
   }
@@ -3722,7 +4032,7 @@ static double single_impl(int64_t* coord_list, int64_t len_coord_list, const dou
   const uint8_t* vol = flatten_table(label_list, shape, storage);
   Context* c = nullptr;
   if (ctx_create(vol, shape, coord_list, nullptr, len_coord_list, voxel_size, coefficients,
-                 full_iteration, 0, &c) != ANACOR_OK) {
+                 full_iteration, 0, &c, 1) != ANACOR_OK) {
     fprintf(stderr, "anacor: ray_tracing_single: %s\n", g_err);
     return __builtin_nan("");
   }
@@ -3835,7 +4145,7 @@ double ib_test(int64_t* coord_list, int64_t len_coord_list, double* rotated_s1, 
   const uint8_t* vol = flatten_table(label_list, shape, storage);
   Context* c = nullptr;
   if (ctx_create(vol, shape, coord_list, nullptr, len_coord_list, voxel_size, coefficients,
-                 full_iteration, 0, &c) != ANACOR_OK) {
+                 full_iteration, 0, &c, 1) != ANACOR_OK) {
     fprintf(stderr, "anacor: ib_test: %s\n", g_err);
     return __builtin_nan("");
   }
@@ -4020,7 +4330,7 @@ double ray_tracing_single_gridding(int64_t* coord, const double* rotated_s1, dou
   const uint8_t* vol = flatten_table(label_list, shape, storage);
   Context* c = nullptr;
   if (ctx_create(vol, shape, coord, nullptr, 1, voxel_size, coefficients, full_iteration, 0,
-                 &c) != ANACOR_OK) {
+                 &c, 1) != ANACOR_OK) {
     fprintf(stderr, "anacor: ray_tracing_single_gridding: %s\n", g_err);
     return __builtin_nan("");
   }
