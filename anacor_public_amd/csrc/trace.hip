@@ -1425,10 +1425,17 @@ static int fit_tile(int64_t n, int64_t R, int vpt) {
 // 2,048, sort led by the diffracted ray, three workgroups per CU: 939 ms at
 // 512, 864 ms at 384, 894 ms at 256; the same volume with seed 7, 6k
 // reflections: 580, 527, 544 ms; 700x900x900, 80k voxels: 398, 378, 378 ms).
+// The skip walk (kTileSkip) narrows to two voxels per lane where the volume is
+// larger than the caches: 1000x1000x800, 1,500 reflections: 59.1 ms at 1,024,
+// 52.5 at 512, 49.0 at 256; 700x640x680, 3,000: 13.9, 12.4, 12.3 ms.
 static bool is_bricked(int layout);
+constexpr int kTileSkip = -2;
+constexpr long long kCachedVolume = 64ll << 20;   // bytes
 static int choose_tile(const Context* c, int64_t R, int layout = -1) {
   if (c->tile_voxels > 0) return c->tile_voxels;
-  const int64_t cap = is_bricked(layout) ? kBlock + kBlock / 2 : (int64_t)kBlock * 4;
+  const int64_t cap = is_bricked(layout) ? kBlock + kBlock / 2
+                      : layout == kTileSkip && c->vol_bytes > kCachedVolume ? (int64_t)kBlock * 2
+                                                                   : (int64_t)kBlock * 4;
   const int64_t target_blocks = 256 * 16;
   int64_t tiles = (target_blocks + R - 1) / std::max<int64_t>(R, 1);
   tiles = std::max<int64_t>(1, std::min<int64_t>(tiles, (c->N + kBlock - 1) / kBlock));
@@ -2011,7 +2018,7 @@ static int run_rules(Context* c, const ReflRule* h_rules, int64_t R, int flags, 
     if (rc) return rc;
     layout = c->layout;
   }
-  const int vpt = paths ? kBlock : choose_tile(c, R, use_skip(c, R) ? -1 : layout);
+  const int vpt = paths ? kBlock : choose_tile(c, R, use_skip(c, R) ? kTileSkip : layout);
   const int64_t tiles = (c->N + vpt - 1) / vpt;
   if (R > (int64_t)INT32_MAX / 2 || R * tiles > ((int64_t)1 << 40)) {
     set_error(ANACOR_ERR_ARG, "%lld reflections x %lld tiles in one call", (long long)R,
@@ -2187,6 +2194,16 @@ static int field_build(Context* c) {
   f.bytes = zs * Z2;
   f.wx = (X2 + 31) / 32;
   const long long plane = (long long)Z2 * Y2 * f.wx;
+  // a large volume's field (eight bytes per voxel) takes at most a quarter of
+  // the free memory, so that contexts created later still find theirs
+  if (f.bytes >= (32ll << 20)) {
+    size_t free_bytes = 0, total = 0;
+    if (hipMemGetInfo(&free_bytes, &total) != hipSuccess) {
+      (void)hipGetLastError();
+      return ANACOR_OK;
+    }
+    if ((size_t)f.bytes * 8 > free_bytes / 4) return ANACOR_OK;
+  }
   DeviceTemp planes, flag;
   if (hipMalloc(&planes.p, (size_t)plane * kLevels * sizeof(uint32_t)) != hipSuccess ||
       hipMalloc(&c->d_field, (size_t)f.bytes * 8) != hipSuccess) {
@@ -2348,12 +2365,10 @@ static int ctx_create(const uint8_t* vol, const int64_t shape[3], const int64_t*
     c->auto_block = std::getenv("ANACOR_VOXEL_BLOCK") == nullptr;
     const int rc = upload_voxel_order(c, blk[0], blk[1], blk[2]);
     if (rc) return rc;
-    // volumes in bricks keep the bricked walk, whose bytes the L2s hold
-    //; a one-shot call builds the field where its steps
-    // (about a sixth of the extents' sum per ray) cost more than the field does
+    // a one-shot call builds the field where its steps (about a third of the
+    // extents' sum per pair) cost more than the field does
     const double steps = (double)reflections * (double)n * (c->Z + c->Y + c->X) / 3.0;
-    if (nvox > (64ull << 20) || (reflections > 0 && steps < 1e9 + 300.0 * (double)nvox))
-      return ANACOR_OK;
+    if (reflections > 0 && steps < 1e9 + 300.0 * (double)nvox) return ANACOR_OK;
     return field_build(c);
   };
   const int rc = init();
@@ -2528,7 +2543,7 @@ static int ctx_run_noalloc(Context* c, const double* s1, const double* omega, in
   // the tile of anacor_ctx_run, enlarged until R * tiles fits the partials
   rc = ensure_layout(c, /*may_build=*/false);
   if (rc) return rc;
-  int64_t vpt = choose_tile(c, R, use_skip(c, R) ? -1 : c->layout);
+  int64_t vpt = choose_tile(c, R, use_skip(c, R) ? kTileSkip : c->layout);
   const int64_t max_tiles = kNoAllocMaxPartials / R;
   if ((c->N + vpt - 1) / vpt > max_tiles) vpt = (c->N + max_tiles - 1) / max_tiles;
   const auto t0 = std::chrono::steady_clock::now();
