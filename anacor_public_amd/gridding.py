@@ -79,22 +79,36 @@ def dials_2_thetaphi(rotated_s1, L1=False):
     return theta, phi
 
 
+def _squared(v):
+    """v ** 2 with the bits of the scalar expression: one libm pow per value
+    (NumPy's array power multiplies, which rounds differently in about one
+    value in a thousand)."""
+    return np.array([q ** 2 for q in v.tolist()], dtype=np.float64)
+
+
 def grid_directions(n_theta: int, n_phi: int) -> Tuple[np.ndarray, np.ndarray]:
     """(rotated_s1 [D][3], theta_phi [D][2]) of the n_theta x n_phi grid,
     phi-major (utils_gridding.py:254-259 for the grid, :103-112 and :161-163
-    for the vectors and their angles)."""
+    for the vectors and their angles): thetaphi_2_myframe, myframe_2_dials and
+    dials_2_thetaphi of every direction, evaluated on whole columns, bit for
+    bit as one by one (7,200 directions: 62 ms one by one, 2.4 ms so)."""
     theta_list = np.linspace(-180, 180, n_theta, endpoint=False)
     phi_list = np.linspace(-90, 90, n_phi, endpoint=False)
     theta_grid, phi_grid = np.meshgrid(theta_list, phi_list)
-    data = np.stack((theta_grid.ravel(), phi_grid.ravel()), axis=-1)
-    data = data / 180 * np.pi
-    vecs = np.empty((len(data), 3))
-    angles = np.empty((len(data), 2))
-    for i, (theta, phi) in enumerate(data):
-        v = myframe_2_dials(thetaphi_2_myframe(theta, phi))
-        vecs[i] = v
-        angles[i] = dials_2_thetaphi(v)
-    return vecs, angles
+    theta = theta_grid.ravel() / 180 * np.pi
+    phi = phi_grid.ravel() / 180 * np.pi
+    # myframe (z, y, x) with y and z swapped; the matrix product's sum turns -0 into +0
+    a = np.cos(theta) * np.sin(phi) + 0.0
+    b = -np.cos(theta) * np.cos(phi) + 0.0
+    c = -np.sin(theta) + 0.0
+    root = np.sqrt(_squared(a) + _squared(b))
+    flat = b == 0
+    with np.errstate(divide="ignore", invalid="ignore"):
+        t = np.arctan(-c / np.where(flat, -root + 0.001, root))
+        p = np.arctan(-a / np.where(flat, b + 0.001, np.where(b > 0, -b, b)))
+    up = b > 0
+    t = np.where(up, np.where(c < 0, np.pi - t, -np.pi - t), t)
+    return np.stack((a, b, c), axis=1), np.stack((t, np.where(up, -p, p)), axis=1)
 
 
 def padding(n_theta: int, n_phi: int) -> Tuple[int, int]:
