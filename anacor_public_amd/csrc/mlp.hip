@@ -9,9 +9,9 @@
 // gradients stay FP32 and enter the MFMA as a BF16 hi + lo pair (two
 // products), so their rounding puts no input-dependent noise on the output;
 // weight gradients use hi/lo on both operands (three products).  In training
-// the 60 -> 256 input layer and the 256 -> 1 output layer are FP32 VALU
-// kernels; inference runs the input layer on MFMA as hi/lo pairs of both
-// operands.  FP32 master weights, Adam.
+// the 60 -> 256 input layer runs on the FP32 MFMA and the 256 -> 1 output
+// layer on FP32 VALU; inference runs the input layer on MFMA as hi/lo pairs of
+// both operands.  FP32 master weights, Adam.
 //
 // Parameter layout (FP32, ANACOR_MLP_PARAMS values):
 //   W1[256][60] b1[256] W2[256][256] b2[256] W3[256][256] b3[256]
@@ -68,233 +68,9 @@ __device__ __forceinline__ float silu_grad(float z) {
   return s * (1.0f + z * (1.0f - s));
 }
 
-// ------------------------------------------------------------------ GEMM
-//
-// C[M][N] = sum_k A(m,k) B(k,n).  A is stored K-contiguous ([M][K], A_KC) or
-// M-contiguous ([K][M]); B K-contiguous ([N][K], B_KC) or N-contiguous
-// ([K][N]).  FP32 operands (A_F32 / B_F32) are split into BF16 hi + lo in
-// LDS; BF16 operands are used as they are.  Workgroup tile 64x64, 4 waves of
-// 32x32 (2x2 MFMA 16x16x32 blocks), K step 32.
-//
 // MFMA 16x16x32 operand layout: lane l supplies row (A) / column (B) l % 16
 // and the 8 k values 8 (l / 16) .. 8 (l / 16) + 7; the accumulator of lane l
 // holds column l % 16, rows 4 (l / 16) .. 4 (l / 16) + 3.
-
-constexpr int BM = 64, BN = 64, BK = 32, KP = 40;  // KP: padded LDS row (bf16)
-constexpr int kSplitMax = 32;                      // K slices of the weight-gradient GEMMs
-
-enum Epi { kEpiStore = 0, kEpiBiasSilu = 1, kEpiSiluBwd = 2, kEpiSplit = 3 };
-
-struct GemmArgs {
-  int M, N, K;
-  const void* A;
-  int lda;
-  const void* B;
-  int ldb;
-  float* C;      // kEpiStore: C; kEpiBiasSilu: SiLU(z); kEpiSiluBwd: dZ; kEpiSplit: slices [z][M][N]
-  int ldc;
-  float* Z;      // kEpiBiasSilu: pre-activation out (nullable); kEpiSiluBwd: pre-activation in
-  const float* bias;
-  float* colsum; // kEpiSplit, A M-contiguous: per-slice sums of A over k, [z][M] (nullable)
-  int k_chunk;   // kEpiSplit: k per slice (multiple of BK)
-  int vec;       // 1: leading dimensions and bases allow 16-byte loads
-};
-
-// 8 consecutive elements of an FP32 or BF16 matrix as floats (`valid` of
-// them in range; all 8 loaded as 16-byte vectors when valid == 8 and vec).
-template <bool F32>
-__device__ __forceinline__ void load8(const void* base, size_t idx, int valid, bool vec,
-                                      float* v) {
-  if (F32) {
-    const float* p = (const float*)base + idx;
-    if (valid == 8 && vec) {
-      const float4 a = *(const float4*)p, b = *(const float4*)(p + 4);
-      v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-      v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = e < valid ? p[e] : 0.f;
-    }
-  } else {
-    const __bf16* p = (const __bf16*)base + idx;
-    if (valid == 8 && vec) {
-      const bf16x8 a = *(const bf16x8*)p;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = (float)a[e];
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = e < valid ? (float)p[e] : 0.f;
-    }
-  }
-}
-
-// One operand tile (64 rows of the output dimension x 32 k, k < K) into LDS.
-// KC: the operand is K-contiguous in global memory.  With SUM (M-contiguous
-// operands only) the thread adds its 8 values to csum (its 8 rows, one k).
-template <bool KC, bool F32, bool SUM>
-__device__ __forceinline__ void stage(const void* base, int ld, int rows, int K, int r0, int k0,
-                                      bool vec, __bf16 (*hi)[KP], __bf16 (*lo)[KP],
-                                      float* csum) {
-  const int t = (int)threadIdx.x;
-  float v[8];
-  if (KC) {  // thread: one row, 8 consecutive k
-    const int r = t >> 2, kc = (t & 3) * 8;
-    const int gr = r0 + r, gk = k0 + kc;
-    const int valid = (gr < rows) ? min(8, max(0, K - gk)) : 0;
-    if (valid > 0) {
-      load8<F32>(base, (size_t)gr * ld + gk, valid, vec, v);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = 0.f;
-    }
-    bf16x8 h, l;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      h[e] = (__bf16)v[e];
-      l[e] = (__bf16)(v[e] - (float)h[e]);
-    }
-    *(bf16x8*)&hi[r][kc] = h;
-    if (F32) *(bf16x8*)&lo[r][kc] = l;
-  } else {   // thread: one k, 8 consecutive rows
-    const int k = t >> 3, rc = (t & 7) * 8;
-    const int gk = k0 + k, gr = r0 + rc;
-    const int valid = (gk < K) ? min(8, max(0, rows - gr)) : 0;
-    if (valid > 0) {
-      load8<F32>(base, (size_t)gk * ld + gr, valid, vec, v);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = 0.f;
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const __bf16 h = (__bf16)v[e];
-      hi[rc + e][k] = h;
-      if (F32) lo[rc + e][k] = (__bf16)(v[e] - (float)h);
-      if (SUM) csum[e] += v[e];
-    }
-  }
-}
-
-template <bool A_KC, bool B_KC, bool A_F32, bool B_F32, int EPI>
-__global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g) {
-  constexpr bool SUM = (EPI == kEpiSplit) && !A_KC;
-  __shared__ __attribute__((aligned(16))) __bf16 Ah[BM][KP];
-  __shared__ __attribute__((aligned(16))) __bf16 Al[A_F32 ? BM : 1][KP];
-  __shared__ __attribute__((aligned(16))) __bf16 Bh[BN][KP];
-  __shared__ __attribute__((aligned(16))) __bf16 Bl[B_F32 ? BN : 1][KP];
-  const int m0 = (int)blockIdx.y * BM, n0 = (int)blockIdx.x * BN;
-  const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
-  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-  const bool vec = g.vec != 0;
-  int kb = 0, ke = g.K;
-  if (EPI == kEpiSplit) {
-    kb = (int)blockIdx.z * g.k_chunk;
-    ke = min(g.K, kb + g.k_chunk);
-  }
-  const bool do_sum = SUM && g.colsum != nullptr && blockIdx.x == 0;
-  float csum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  floatx4 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-  const int r16 = lane & 15, kg = (lane >> 4) * 8;
-  for (int k0 = kb; k0 < ke; k0 += BK) {
-    if (do_sum)
-      stage<A_KC, A_F32, true>(g.A, g.lda, g.M, ke, m0, k0, vec, Ah, Al, csum);
-    else
-      stage<A_KC, A_F32, false>(g.A, g.lda, g.M, ke, m0, k0, vec, Ah, Al, csum);
-    stage<B_KC, B_F32, false>(g.B, g.ldb, g.N, ke, n0, k0, vec, Bh, Bl, nullptr);
-    __syncthreads();
-    bf16x8 ah[2], al[2], bh[2], bl[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      ah[i] = *(const bf16x8*)&Ah[wm + i * 16 + r16][kg];
-      if (A_F32) al[i] = *(const bf16x8*)&Al[wm + i * 16 + r16][kg];
-      bh[i] = *(const bf16x8*)&Bh[wn + i * 16 + r16][kg];
-      if (B_F32) bl[i] = *(const bf16x8*)&Bl[wn + i * 16 + r16][kg];
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        if (A_F32)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bh[j], acc[i][j], 0, 0, 0);
-        if (B_F32)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bl[j], acc[i][j], 0, 0, 0);
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bh[j], acc[i][j], 0, 0, 0);
-      }
-    __syncthreads();
-  }
-  if (SUM) {   // column sums of A over this slice: 32 k-threads per row group
-    if (do_sum) {
-      __shared__ float red[32][BM + 1];
-      const int k = (int)threadIdx.x >> 3, rc = ((int)threadIdx.x & 7) * 8;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) red[k][rc + e] = csum[e];
-      __syncthreads();
-      if (threadIdx.x < BM && m0 + (int)threadIdx.x < g.M) {
-        float sum = 0.f;
-        for (int q = 0; q < 32; ++q) sum += red[q][threadIdx.x];
-        g.colsum[(size_t)blockIdx.z * g.M + m0 + threadIdx.x] = sum;
-      }
-    }
-  }
-  float* C = g.C;
-  if (EPI == kEpiSplit) C += (size_t)blockIdx.z * g.M * g.ldc;
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = m0 + wm + i * 16 + (lane >> 4) * 4 + r;
-        const int n = n0 + wn + j * 16 + (lane & 15);
-        if (m >= g.M || n >= g.N) continue;
-        const float v = acc[i][j][r];
-        const size_t o = (size_t)m * g.ldc + n;
-        if (EPI == kEpiStore || EPI == kEpiSplit) {
-          C[o] = v;
-        } else if (EPI == kEpiBiasSilu) {
-          const float z = v + g.bias[n];
-          if (g.Z) g.Z[o] = z;
-          C[o] = silu(z);
-        } else {
-          C[o] = v * silu_grad(g.Z[o]);
-        }
-      }
-}
-
-static bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
-
-template <bool A_KC, bool B_KC, bool A_F32, bool B_F32, int EPI>
-static void gemm(GemmArgs g, hipStream_t s, int slices = 1) {
-  const int ea = A_F32 ? 4 : 8, eb = B_F32 ? 4 : 8;   // elements per 16 bytes
-  g.vec = (g.lda % ea == 0 && g.ldb % eb == 0 && aligned16(g.A) && aligned16(g.B)) ? 1 : 0;
-  const dim3 grid((unsigned)((g.N + BN - 1) / BN), (unsigned)((g.M + BM - 1) / BM),
-                  (unsigned)slices);
-  hipLaunchKernelGGL((gemm_kernel<A_KC, B_KC, A_F32, B_F32, EPI>), grid, dim3(256), 0, s, g);
-}
-
-// Sum of the K slices of a split GEMM (fixed order): out[m][n] (row stride
-// ldo) and, when colsum is set, bias_out[m] from the per-slice column sums.
-__global__ void split_reduce(const float* __restrict__ ws, int slices, int M, int N,
-                             float* __restrict__ out, int ldo, const float* __restrict__ colsum,
-                             float* __restrict__ bias_out) {
-  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (i < M * N) {
-    const int m = i / N, n = i % N;
-    float sum = 0.f;
-    for (int z = 0; z < slices; ++z) sum += ws[(size_t)z * M * N + i];
-    out[(size_t)m * ldo + n] = sum;
-  }
-  if (colsum && i < M) {
-    float sum = 0.f;
-    for (int z = 0; z < slices; ++z) sum += colsum[(size_t)z * M + i];
-    bias_out[i] = sum;
-  }
-}
 
 // ------------------------------------------------- fused inference kernel
 //
@@ -311,10 +87,12 @@ __global__ void split_reduce(const float* __restrict__ ws, int slices, int M, in
 // writes A = exp(y std + mean) inside the envelope and NaN outside.
 
 constexpr int kHP = kH + 8;   // padded LDS row of activations (bf16)
-// BF16 weight block: W2, W3, W4 [256][256], then W1 hi and lo [256][kInK].
+// BF16 weight block: W2, W3, W4 [256][256], then W1 hi and lo [256][kInK],
+// then W2, W3, W4 transposed (the backward pass's operand).
 constexpr size_t kWbW1h = (size_t)3 * kH * kH;
 constexpr size_t kWbW1l = kWbW1h + (size_t)kH * kInK;
-constexpr size_t kWbSize = kWbW1l + (size_t)kH * kInK;
+constexpr size_t kWbT = kWbW1l + (size_t)kH * kInK;
+constexpr size_t kWbSize = kWbT + (size_t)3 * kH * kH;
 
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
@@ -442,109 +220,355 @@ __global__ __launch_bounds__(256) void mlp_infer_kernel(
   }
 }
 
-// ------------------------------------------------------- small kernels
+// ------------------------------------------------------- training kernels
+//
+// A training step is three launches: train_tile_kernel (forward and backward
+// through every layer for a tile of rows), weight_grad_kernel (the four weight
+// gradients, split over the rows) and reduce_kernel (the slices' sums, the
+// bias gradients and the loss, with Adam in place).  Layer by layer, with
+// pre-activations, activations and dZ in FP32 through memory, it was 22
+// launches and 270 us at 4,096 rows (67 us now: 42, 16 and 8), 566 us at 16,384
+// (149 us: 97, 44 and 9).
+//
+// Operands of the weight gradients, dW[out][in] = sum_b dZ[b][out] H[b][in],
+// leave the tile kernel as the MFMA reads them: BF16 hi and lo planes in blocks of
+// 32 rows, [block][unit][32], a lane's 8 rows of one unit 16 bytes and a
+// wave's fragment 1 KB in one piece.
 
-// H1 = SiLU(X W1^T + b1), FP32; one thread per (row, unit).  With perm
-// (training) row b reads X[perm[b]] and T[perm[b]] and copies them to
-// Xb[b] / Tb[b] for the backward pass.
-__global__ void layer1_fwd(const float* __restrict__ X, const int* __restrict__ perm,
-                           const float* __restrict__ T, int n, const float* __restrict__ P,
-                           float* __restrict__ Xb, float* __restrict__ Tb,
-                           float* __restrict__ Z1, float* __restrict__ H1) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long long)n * kH) return;
-  const int b = (int)(t / kH), u = (int)(t % kH);
-  const int src = perm ? perm[b] : b;
-  const float* w = P + kOffW1 + u * kIn;
-  const float* x = X + (size_t)src * kIn;
-  float z = P[kOffB1 + u];
-#pragma unroll
-  for (int k = 0; k < kIn; ++k) z = fmaf(x[k], w[k], z);
-  if (Z1) Z1[t] = z;
-  H1[t] = silu(z);
-  if (perm) {
-    if (u < kIn) Xb[(size_t)b * kIn + u] = x[u];
-    if (u == kIn) Tb[b] = T[src];
-  }
+constexpr int kRowBlock = 32;
+constexpr int kSplitMax = 32;             // K slices of the weight gradients
+// Planes of a 32-row block, in elements: the inputs (64 wide) hi and lo, H1-H3
+// hi and lo, dZ1-dZ4 hi and lo.
+constexpr size_t kPlane = (size_t)kH * kRowBlock;
+constexpr size_t kPlaneX = (size_t)kInK * kRowBlock;
+constexpr size_t kActH = 2 * kPlaneX;                 // H(l), l = 0..2: + 2 l kPlane
+constexpr size_t kActD = kActH + 6 * kPlane;          // dZ(l), l = 0..3: + 2 l kPlane
+constexpr size_t kActBlock = kActD + 8 * kPlane;
+// Per-tile partials: column sums of dZ1-dZ4 [4][256], dw5 [256], loss, dy.
+constexpr int kPartW5 = 4 * kH;
+constexpr int kPartLoss = kPartW5 + kH;
+constexpr int kPart = kPartLoss + 2;
+// A slice of weight gradients: W1 [256][64], then W2, W3, W4 [256][256].
+constexpr size_t kWsW2 = (size_t)kH * kInK;
+constexpr size_t kWsStride = kWsW2 + 3 * (size_t)kH * kH;
+
+struct TrainArgs {
+  const float* X;         // rows [kIn], of X[perm[b]] with perm
+  const int* perm;
+  const float* T;
+  int n;
+  const float* P;
+  const __bf16* Wb;
+  __bf16* act;            // [blocks of 32 rows][kActBlock]
+  float* part;            // [tiles][kPart]
+};
+
+__device__ __forceinline__ void split_bf16(float v, __bf16& hi, __bf16& lo) {
+  hi = (__bf16)v;
+  lo = (__bf16)(v - (float)hi);
 }
 
-// y = H4 w5 + b5, FP32; one wave per row.
-__device__ __forceinline__ float head_dot(const float* __restrict__ h, const float* __restrict__ P,
-                                          int lane) {
-  float s = 0.f;
-#pragma unroll
-  for (int k = lane; k < kH; k += 64) s = fmaf(h[k], P[kOffW5 + k], s);
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-  return s + P[kOffB5];
-}
+// Forward and backward of ROWS rows in one workgroup of 8 waves, wave w the
+// units 32 w .. 32 w + 31 of every layer.  MFMA with the rows as M: a lane
+// holds 4 consecutive rows of one unit, which is both a run of a weight-gradient
+// operand plane and, forward and backward, the same (row, unit) pairs of every
+// layer, so SiLU' of the four layers stays in registers.  Activations and dZ
+// pass between layers in LDS as hi/lo [row][unit]; weights come from L2 as
+// 16-byte fragments.  The input layer runs on the FP32 MFMA (k in the order 16
+// s + 4 (l / 16) + e, the same for both operands).
+//
+// What bounds it: the chain of seven layers, each a round of weight fragments
+// from L2 between two barriers (42 us for 256 workgroups of 16 rows, 97 us for
+// 512 of 32).  Rows per workgroup: the weights' 0.86 MB per workgroup ask for
+// more rows, a batch of 4,096 for enough workgroups.
+template <int ROWS>
+__global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
+  constexpr int RT = ROWS / 16;
+  static_assert(ROWS == 16 || ROWS == 32, "row tile");
+  __shared__ __attribute__((aligned(16))) __bf16 Hh[ROWS][kHP];
+  __shared__ __attribute__((aligned(16))) __bf16 Hl[ROWS][kHP];
+  __shared__ float head[8][ROWS];
+  const int t = (int)threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int r16 = lane & 15, quad = lane >> 4, kg = quad * 8, q4 = quad * 4;
+  const int ub = wave * 32;
+  const int r0 = (int)blockIdx.x * ROWS;
+  __bf16* const act = a.act + (size_t)(r0 / kRowBlock) * kActBlock;
+  const int rb = r0 % kRowBlock;                  // this tile's first row in its block
+  float* const part = a.part + (size_t)blockIdx.x * kPart;
 
-__global__ void out_fwd(const float* __restrict__ H4, int n, const float* __restrict__ P,
-                        float* __restrict__ y) {
-  const int row = (int)blockIdx.x * 4 + ((int)threadIdx.x >> 6);
-  const int lane = (int)threadIdx.x & 63;
-  if (row >= n) return;
-  const float s = head_dot(H4 + (size_t)row * kH, P, lane);
-  if (lane == 0) y[row] = s;
-}
-
-// Training head, one wave per row: y, the mean squared error term, dy =
-// 2 (y - t) / n, dZ4 = dy w5 silu'(Z4); per-block partial sums of the loss
-// and of dy (db5) in part[block][2].
-__global__ void head_train(const float* __restrict__ H4, const float* __restrict__ Z4,
-                           const float* __restrict__ T, int n, const float* __restrict__ P,
-                           float* __restrict__ y, float* __restrict__ dy,
-                           float* __restrict__ dZ4, float* __restrict__ part) {
-  __shared__ float red[4][2];
-  const int w = (int)threadIdx.x >> 6;
-  const int row = (int)blockIdx.x * 4 + w;
-  const int lane = (int)threadIdx.x & 63;
-  float l = 0.f, g = 0.f;
-  if (row < n) {
-    const float yv = head_dot(H4 + (size_t)row * kH, P, lane);
-    const float d = yv - T[row];
-    g = 2.f * d / (float)n;
-    l = d * d / (float)n;
-    if (lane == 0) {
-      y[row] = yv;
-      dy[row] = g;
+  floatx4 acc[2][RT];
+  floatx4 sg[4][2][RT];                           // SiLU' of the layers
+  auto clear = [&]() {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < RT; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  };
+  // acc's 4 rows of a unit as hi/lo: into LDS for the next layer, and into the
+  // operand planes at `plane` (hi; lo behind it)
+  auto put = [&](int i, int j, const floatx4& v, __bf16* plane, bool lds) {
+    bf16x4 h, l;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      __bf16 hr, lr;
+      split_bf16(v[r], hr, lr);
+      h[r] = hr;
+      l[r] = lr;
     }
-    const float* z = Z4 + (size_t)row * kH;
-    float* o = dZ4 + (size_t)row * kH;
+    const int u = ub + i * 16 + r16;
+    if (lds) {
 #pragma unroll
-    for (int k = lane; k < kH; k += 64) o[k] = g * P[kOffW5 + k] * silu_grad(z[k]);
+      for (int r = 0; r < 4; ++r) {
+        Hh[j * 16 + q4 + r][u] = h[r];
+        Hl[j * 16 + q4 + r][u] = l[r];
+      }
+    }
+    if (plane) {
+      __bf16* o = plane + (size_t)u * kRowBlock + rb + j * 16 + q4;
+      *(bf16x4*)o = h;
+      *(bf16x4*)(o + kPlane) = l;
+    }
+  };
+  // acc += LDS rows . W^T, W [unit][256] BF16
+  auto product = [&](const __bf16* __restrict__ W) {
+#pragma unroll
+    for (int k0 = 0; k0 < kH; k0 += 32) {
+      bf16x8 w[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        w[i] = *(const bf16x8*)(W + (size_t)(ub + i * 16 + r16) * kH + k0 + kg);
+#pragma unroll
+      for (int j = 0; j < RT; ++j) {
+        const bf16x8 hh = *(const bf16x8*)&Hh[j * 16 + r16][k0 + kg];
+        const bf16x8 hl = *(const bf16x8*)&Hl[j * 16 + r16][k0 + kg];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hl, w[i], acc[i][j], 0, 0, 0);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hh, w[i], acc[i][j], 0, 0, 0);
+        }
+      }
+    }
+  };
+  // column sums of v over the tile's rows (rows past n hold zeros)
+  auto column_sum = [&](int i, const floatx4 (&v)[2][RT], float* out) {
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < RT; ++j) s += (v[i][j][0] + v[i][j][1]) + (v[i][j][2] + v[i][j][3]);
+    s += __shfl_xor(s, 16);
+    s += __shfl_xor(s, 32);
+    if (quad == 0) out[ub + i * 16 + r16] = s;
+  };
+
+  // inputs as operand planes: 8 rows of one column per thread
+  for (int q = t; q < kInK * (ROWS / 8); q += 512) {
+    const int k = q % kInK, rg = q / kInK * 8;
+    bf16x8 h, l;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int row = r0 + rg + e;
+      float v = 0.f;
+      if (k < kIn && row < a.n) v = a.X[(size_t)(a.perm ? a.perm[row] : row) * kIn + k];
+      __bf16 hr, lr;
+      split_bf16(v, hr, lr);
+      h[e] = hr;
+      l[e] = lr;
+    }
+    __bf16* o = act + (size_t)k * kRowBlock + rb + rg;
+    *(bf16x8*)o = h;
+    *(bf16x8*)(o + kPlaneX) = l;
   }
-  if (lane == 0) {
-    red[w][0] = l;
-    red[w][1] = g;
+  // input layer in FP32
+  clear();
+  {
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+    const float* x[RT];
+#pragma unroll
+    for (int j = 0; j < RT; ++j) {
+      const int row = r0 + j * 16 + r16;
+      x[j] = row < a.n ? a.X + (size_t)(a.perm ? a.perm[row] : row) * kIn : nullptr;
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int k = 16 * s + q4;
+      float4 xv[RT], wv[2];
+#pragma unroll
+      for (int j = 0; j < RT; ++j) xv[j] = x[j] && k < kIn ? *(const float4*)(x[j] + k) : zero;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        wv[i] = k < kIn ? *(const float4*)(a.P + kOffW1 + (size_t)(ub + i * 16 + r16) * kIn + k)
+                        : zero;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int j = 0; j < RT; ++j)
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(((const float*)&xv[j])[e],
+                                                             ((const float*)&wv[i])[e],
+                                                             acc[i][j], 0, 0, 0);
+    }
   }
+  constexpr int offb[4] = {kOffB1, kOffB2, kOffB3, kOffB4};
+#pragma unroll
+  for (int l = 0; l < 4; ++l) {
+    if (l > 0) {
+      clear();
+      product(a.Wb + (size_t)(l - 1) * kH * kH);
+      __syncthreads();                            // every wave has read this layer's input
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const float bias = a.P[offb[l] + ub + i * 16 + r16];
+#pragma unroll
+      for (int j = 0; j < RT; ++j) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float z = acc[i][j][r] + bias;
+          const float s = sigmoidf_(z);
+          sg[l][i][j][r] = s * (1.0f + z * (1.0f - s));
+          acc[i][j][r] = r0 + j * 16 + q4 + r < a.n ? z * s : 0.f;
+        }
+        if (l < 3) put(i, j, acc[i][j], act + kActH + 2 * l * kPlane, true);
+      }
+    }
+    if (l < 3) __syncthreads();
+  }
+  // head: y, dy = 2 (y - t) / n, the loss; dw5's partial sums
+  float w5[2], dy[RT][4];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) w5[i] = a.P[kOffW5 + ub + i * 16 + r16];
+#pragma unroll
+  for (int j = 0; j < RT; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float v = fmaf(acc[0][j][r], w5[0], acc[1][j][r] * w5[1]);
+#pragma unroll
+      for (int off = 8; off > 0; off >>= 1) v += __shfl_xor(v, off);
+      if (r16 == 0) head[wave][j * 16 + q4 + r] = v;
+    }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = (red[0][0] + red[1][0]) + (red[2][0] + red[3][0]);
-    part[2 * blockIdx.x + 1] = (red[0][1] + red[1][1]) + (red[2][1] + red[3][1]);
-  }
-}
-
-// loss[0] += sum of the loss partials; G[b5] = sum of the dy partials.
-__global__ void head_finish(const float* __restrict__ part, int nb, float* __restrict__ loss,
-                            float* __restrict__ gb5) {
-  float l = 0.f, g = 0.f;
-  for (int i = (int)threadIdx.x; i < nb; i += 64) {
-    l += part[2 * i];
-    g += part[2 * i + 1];
-  }
+  float loss = 0.f, sum_dy = 0.f;
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    l += __shfl_xor(l, off);
-    g += __shfl_xor(g, off);
+  for (int j = 0; j < RT; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = j * 16 + q4 + r;
+      float y = 0.f;
+#pragma unroll
+      for (int w = 0; w < 8; ++w) y += head[w][row];
+      dy[j][r] = 0.f;
+      if (r0 + row < a.n) {
+        const int src = a.perm ? a.perm[r0 + row] : r0 + row;
+        const float d = (y + a.P[kOffB5]) - a.T[src];
+        dy[j][r] = 2.f * d / (float)a.n;
+        loss += d * d / (float)a.n;
+      }
+      sum_dy += dy[j][r];
+    }
+  loss += __shfl_xor(loss, 16);
+  loss += __shfl_xor(loss, 32);
+  sum_dy += __shfl_xor(sum_dy, 16);
+  sum_dy += __shfl_xor(sum_dy, 32);
+  if (t == 0) {
+    part[kPartLoss] = loss;
+    part[kPartLoss + 1] = sum_dy;
   }
-  if (threadIdx.x == 0) {
-    loss[0] += l;
-    gb5[0] = g;
+  floatx4 dz[2][RT];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+#pragma unroll
+    for (int j = 0; j < RT; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        acc[i][j][r] *= dy[j][r];
+        dz[i][j][r] = dy[j][r] * w5[i] * sg[3][i][j][r];
+      }
+    column_sum(i, acc, part + kPartW5);
+  }
+  // back through the layers; dZ1 feeds the weight gradient only
+#pragma unroll
+  for (int l = 3; l >= 0; --l) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+#pragma unroll
+      for (int j = 0; j < RT; ++j) put(i, j, dz[i][j], act + kActD + 2 * l * kPlane, l > 0);
+      column_sum(i, dz, part + l * kH);
+    }
+    if (l == 0) break;
+    __syncthreads();
+    clear();
+    product(a.Wb + kWbT + (size_t)(l - 1) * kH * kH);
+    __syncthreads();                              // every wave has read dZ of this layer
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < RT; ++j) dz[i][j] = acc[i][j] * sg[l - 1][i][j];
   }
 }
 
-// BF16 copies of W2, W3, W4 (round to nearest even) and W1 as hi/lo pairs
+// One slice of the weight gradients: 13 workgroups per slice, 4 waves of 64 x 64
+// outputs each; W1 [256][64] is one workgroup, W2, W3, W4 four quarters each.
+// Fragments come straight from the operand planes (1 KB per wave and load).
+// hi/lo on both operands, three products.
+struct WeightGradArgs {
+  const __bf16* act;
+  int blocks;             // 32-row blocks
+  int per_slice;          // blocks per slice
+  float* ws;              // [slices][kWsStride]
+};
+
+__global__ __launch_bounds__(256) void weight_grad_kernel(WeightGradArgs g) {
+  const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
+  const int r16 = lane & 15, kg = (lane >> 4) * 8, q4 = (lane >> 4) * 4;
+  const int job = (int)blockIdx.x;                // 0: W1, else quarter (job - 1) % 4 of a layer
+  const bool first = job == 0;
+  const int layer = first ? 0 : (job - 1) / 4 + 1, quarter = (job - 1) & 3;
+  const int m0 = first ? wave * 64 : (quarter >> 1) * 128 + (wave >> 1) * 64;
+  const int n0 = first ? 0 : (quarter & 1) * 128 + (wave & 1) * 64;
+  const size_t A = kActD + 2 * layer * kPlane + (size_t)(m0 + r16) * kRowBlock + kg;
+  const size_t B = (first ? 0 : kActH + 2 * (layer - 1) * kPlane) +
+                   (size_t)(n0 + r16) * kRowBlock + kg;
+  const size_t Blo = first ? kPlaneX : kPlane;
+  floatx4 acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const int b0 = (int)blockIdx.y * g.per_slice, b1 = min(g.blocks, b0 + g.per_slice);
+#pragma unroll 2
+  for (int b = b0; b < b1; ++b) {
+    const __bf16* blk = g.act + (size_t)b * kActBlock;
+    bf16x8 ah[4], al[4], bh[4], bl[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      ah[i] = *(const bf16x8*)(blk + A + i * 16 * kRowBlock);
+      al[i] = *(const bf16x8*)(blk + A + kPlane + i * 16 * kRowBlock);
+      bh[i] = *(const bf16x8*)(blk + B + i * 16 * kRowBlock);
+      bl[i] = *(const bf16x8*)(blk + B + Blo + i * 16 * kRowBlock);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bh[j], acc[i][j], 0, 0, 0);
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bl[j], acc[i][j], 0, 0, 0);
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bh[j], acc[i][j], 0, 0, 0);
+      }
+  }
+  const int ldo = first ? kInK : kH;
+  float* out = g.ws + (size_t)blockIdx.y * kWsStride +
+               (first ? 0 : kWsW2 + (size_t)(layer - 1) * kH * kH);
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        out[(size_t)(m0 + i * 16 + q4 + r) * ldo + n0 + j * 16 + r16] = acc[i][j][r];
+}
+
+// BF16 copies of W2, W3, W4 (round to nearest even), as they are and
+// transposed, and W1 as hi/lo pairs
 // padded to K = kInK (the inference kernel's layout).
 __device__ __forceinline__ void store_bf16_copy(int i, float p, __bf16* __restrict__ Wb) {
   int l = -1, j = 0;
@@ -553,6 +577,7 @@ __device__ __forceinline__ void store_bf16_copy(int i, float p, __bf16* __restri
   else if (i >= kOffW4 && i < kOffB4) { l = 2; j = i - kOffW4; }
   if (l >= 0) {
     Wb[(size_t)l * kH * kH + j] = (__bf16)p;
+    Wb[kWbT + (size_t)l * kH * kH + (size_t)(j % kH) * kH + j / kH] = (__bf16)p;
   } else if (i >= kOffW1 && i < kOffB1) {
     const int u = (i - kOffW1) / kIn, k = (i - kOffW1) % kIn;
     const __bf16 h = (__bf16)p;
@@ -561,20 +586,81 @@ __device__ __forceinline__ void store_bf16_copy(int i, float p, __bf16* __restri
   }
 }
 
-// Adam on every parameter, refreshing the BF16 copies of the weights.
-__global__ void adam_step(float* __restrict__ P, const float* __restrict__ G,
-                          float* __restrict__ m, float* __restrict__ v, __bf16* __restrict__ Wb,
-                          float lr, float b1, float b2, float eps, float c1, float c2) {
-  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (i >= kParams) return;
-  const float g = G[i];
-  const float mi = b1 * m[i] + (1.f - b1) * g;
-  const float vi = b2 * v[i] + (1.f - b2) * g * g;
-  m[i] = mi;
-  v[i] = vi;
-  const float p = P[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-  P[i] = p;
-  store_bf16_copy(i, p, Wb);
+// The gradients' sums in fixed order into G, the batch loss added to loss[0],
+// and with `adam` the update of every parameter, its BF16 copies too.  The
+// first blocks take the weights (one per thread, its slices), the last ones
+// the bias and head partials of the tiles: 64 columns and 4 rows of threads.
+struct ReduceArgs {
+  const float* ws;
+  int slices;
+  const float* part;
+  int tiles;
+  float* G;
+  float* loss;
+  bool adam;
+  float *P, *m, *v;
+  __bf16* Wb;
+  float lr, b1, b2, eps, c1, c2;
+};
+constexpr int kWeightFloats = kH * kIn + 3 * kH * kH;
+constexpr int kWeightBlocks = kWeightFloats / 256;
+static_assert(kWeightFloats % 256 == 0, "whole blocks of weights");
+constexpr int kPartBlocks = (kPart + 63) / 64;
+
+__device__ __forceinline__ void take_gradient(const ReduceArgs& a, int i, float g) {
+  a.G[i] = g;
+  if (!a.adam) return;
+  const float mi = a.b1 * a.m[i] + (1.f - a.b1) * g;
+  const float vi = a.b2 * a.v[i] + (1.f - a.b2) * g * g;
+  a.m[i] = mi;
+  a.v[i] = vi;
+  const float p = a.P[i] - a.lr * (mi / a.c1) / (sqrtf(vi / a.c2) + a.eps);
+  a.P[i] = p;
+  store_bf16_copy(i, p, a.Wb);
+}
+
+__global__ __launch_bounds__(256) void reduce_kernel(ReduceArgs a) {
+  const int t = (int)threadIdx.x;
+  if ((int)blockIdx.x < kWeightBlocks) {
+    const int i = (int)blockIdx.x * 256 + t;
+    int param, at;
+    if (i < kH * kIn) {
+      param = kOffW1 + i;
+      at = i / kIn * kInK + i % kIn;
+    } else {
+      const int l = (i - kH * kIn) / (kH * kH), e = (i - kH * kIn) % (kH * kH);
+      param = (l == 0 ? kOffW2 : l == 1 ? kOffW3 : kOffW4) + e;
+      at = (int)kWsW2 + l * kH * kH + e;
+    }
+    float g = 0.f;
+#pragma unroll 8
+    for (int z = 0; z < a.slices; ++z) g += a.ws[(size_t)z * kWsStride + at];
+    take_gradient(a, param, g);
+    return;
+  }
+  __shared__ float rows[4][64];
+  const int col = ((int)blockIdx.x - kWeightBlocks) * 64 + (t & 63);
+  float s = 0.f;
+  if (col < kPart) {
+#pragma unroll 8
+    for (int w = t >> 6; w < a.tiles; w += 4) s += a.part[(size_t)w * kPart + col];
+  }
+  rows[t >> 6][t & 63] = s;
+  __syncthreads();
+  if (t >= 64 || col >= kPart) return;
+  const float g = (rows[0][t] + rows[1][t]) + (rows[2][t] + rows[3][t]);
+  if (col == kPartLoss) {
+    a.loss[0] += g;
+    return;
+  }
+  int param = kOffB5;
+  if (col < kPartW5) {
+    const int l = col / kH;
+    param = (l == 0 ? kOffB1 : l == 1 ? kOffB2 : l == 2 ? kOffB3 : kOffB4) + col % kH;
+  } else if (col < kPartLoss) {
+    param = kOffW5 + col - kPartW5;
+  }
+  take_gradient(a, param, g);
 }
 
 __global__ void weights_to_bf16(const float* __restrict__ P, __bf16* __restrict__ Wb) {
@@ -910,8 +996,10 @@ struct Model {
   DevBuf<float> P, G, m, v;       // FP32 master parameters, gradients, Adam moments
   DevBuf<__bf16> Wb;              // BF16 copies of W2, W3, W4
   int cap = 0;                    // rows of the activation buffers
-  DevBuf<float> Z[4], H[4], dA, dB, dy, xb, tb, part, loss;
-  DevBuf<float> ws, colws;        // split-K slices [kSplitMax][256][256], [kSplitMax][256]
+  DevBuf<__bf16> act;             // training operands (TrainArgs)
+  DevBuf<float> xb, tb, loss;
+  DevBuf<float> part;             // per training tile: bias and head partials (kPart floats)
+  DevBuf<float> ws;               // weight-gradient slices [kSplitMax][kWsStride]
   // feature / inference / training-set buffers (grown on demand)
   DevBuf<double> s1, omega, inv, A;
   DevBuf<float> X, y, T;
@@ -950,20 +1038,21 @@ struct Model {
 
 static unsigned nblocks(long long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
+// Rows of a training tile: 16 until the batch fills the GPU with them.
+static int train_rows(int n) { return n <= 8192 ? 16 : 32; }
+// Tiles of n rows: whole 32-row blocks, whose rows past n hold zeros.
+static size_t train_tiles(int n) {
+  return (size_t)nblocks(n, kRowBlock) * (size_t)(kRowBlock / train_rows(n));
+}
+
 static int ensure_rows(Model* M, int n) {
   if (n <= M->cap) return ANACOR_OK;
-  for (int l = 0; l < 4; ++l) {
-    MLP_CHECK(M->Z[l].grow((size_t)n * kH));
-    MLP_CHECK(M->H[l].grow((size_t)n * kH));
-  }
-  MLP_CHECK(M->dA.grow((size_t)n * kH));
-  MLP_CHECK(M->dB.grow((size_t)n * kH));
-  MLP_CHECK(M->dy.grow((size_t)n));
+  const size_t blocks = nblocks(n, kRowBlock);
+  MLP_CHECK(M->act.grow(blocks * kActBlock));
   MLP_CHECK(M->xb.grow((size_t)n * kIn));
   MLP_CHECK(M->tb.grow((size_t)n));
-  MLP_CHECK(M->part.grow((size_t)2 * nblocks(n, 4)));
-  MLP_CHECK(M->ws.grow((size_t)kSplitMax * kH * kH));
-  MLP_CHECK(M->colws.grow((size_t)kSplitMax * kH));
+  MLP_CHECK(M->part.grow(blocks * (kRowBlock / 16) * kPart));   // tiles of either size
+  MLP_CHECK(M->ws.grow((size_t)kSplitMax * kWsStride));
   M->cap = n;
   return ANACOR_OK;
 }
@@ -985,87 +1074,46 @@ static void infer(Model* M, const float* X, int64_t n, const uint8_t* flag, floa
                      M->stream, X, n, M->P.p, M->Wb.p, flag, M->y_mean, M->y_std, y, A);
 }
 
-// K slices of a weight-gradient GEMM with K = n rows.
-static void split_shape(int n, int* slices, int* chunk) {
-  int s = std::max(1, std::min(kSplitMax, (n + 63) / 64));
-  int c = ((n + s - 1) / s + BK - 1) / BK * BK;
-  *chunk = c;
-  *slices = (n + c - 1) / c;
-}
-
-// dW[M][N] (row stride ldo) = A^T B over n rows, A [n][M] and B [n][N] FP32,
-// plus bias[M] = column sums of A when bias is set.
-static void weight_grad(Model* M, const float* A, int Mdim, const float* B, int N, int n,
-                        float* dW, int ldo, float* bias) {
-  int slices, chunk;
-  split_shape(n, &slices, &chunk);
-  GemmArgs g{};
-  g.M = Mdim; g.N = N; g.K = n;
-  g.A = A; g.lda = Mdim;
-  g.B = B; g.ldb = N;
-  g.C = M->ws.p; g.ldc = N;
-  g.colsum = bias ? M->colws.p : nullptr;
-  g.k_chunk = chunk;
-  gemm<false, false, true, true, kEpiSplit>(g, M->stream, slices);
-  hipLaunchKernelGGL(split_reduce, dim3(nblocks((long long)Mdim * N, 256)), dim3(256), 0,
-                     M->stream, M->ws.p, slices, Mdim, N, dW, ldo,
-                     bias ? M->colws.p : (const float*)nullptr, bias);
-}
-
-// Forward and backward pass of one batch of n rows: gradients of the mean
-// squared error into G, the batch loss added to loss[0].  With perm the rows
-// are X[perm[b]] / T[perm[b]] (gathered on the way), else X / T themselves.
-static void fwd_bwd(Model* M, const float* X, const int* perm, const float* T, int n) {
+// One batch of n rows: gradients of the mean squared error into G, the batch
+// loss added to loss[0] and, with lr, an Adam step.  With perm the rows are
+// X[perm[b]] / T[perm[b]], else X / T themselves.
+static void train_step(Model* M, const float* X, const int* perm, const float* T, int n,
+                       const float* lr) {
   hipStream_t s = M->stream;
-  float* G = M->G.p;
-  hipLaunchKernelGGL(layer1_fwd, dim3(nblocks((long long)n * kH, 256)), dim3(256), 0, s, X, perm,
-                     T, n, M->P.p, M->xb.p, M->tb.p, M->Z[0].p, M->H[0].p);
-  const float* Xr = perm ? M->xb.p : X;
-  const float* Tr = perm ? M->tb.p : T;
-  const int offw[3] = {kOffW2, kOffW3, kOffW4};
-  const int offb[3] = {kOffB2, kOffB3, kOffB4};
-  for (int l = 0; l < 3; ++l) {
-    GemmArgs g{};
-    g.M = n; g.N = kH; g.K = kH;
-    g.A = M->H[l].p; g.lda = kH;
-    g.B = M->Wb.p + (size_t)l * kH * kH; g.ldb = kH;
-    g.C = M->H[l + 1].p; g.ldc = kH;
-    g.Z = M->Z[l + 1].p;
-    g.bias = M->P.p + offb[l];
-    gemm<true, true, true, false, kEpiBiasSilu>(g, s);
-  }
-  // head: y, loss, dy, dZ4; then db5 and the loss
-  float* dz = M->dA.p;
-  float* dnext = M->dB.p;
-  const unsigned hb = nblocks(n, 4);
-  hipLaunchKernelGGL(head_train, dim3(hb), dim3(256), 0, s, M->H[3].p, M->Z[3].p, Tr, n, M->P.p,
-                     M->y.p, M->dy.p, dz, M->part.p);
-  hipLaunchKernelGGL(head_finish, dim3(1), dim3(64), 0, s, M->part.p, (int)hb, M->loss.p,
-                     G + kOffB5);
-  weight_grad(M, M->H[3].p, kH, M->dy.p, 1, n, G + kOffW5, 1, nullptr);   // dw5 = H4^T dy
-  for (int l = 2; l >= 0; --l) {
-    // dW[out][in] = sum_b dZ[b][out] H[b][in], db = sum_b dZ[b]
-    weight_grad(M, dz, kH, M->H[l].p, kH, n, G + offw[l], kH, G + offb[l]);
-    // dZ_prev = (dZ W) silu'(Z_prev): M = batch, N = in, K = out
-    GemmArgs gd{};
-    gd.M = n; gd.N = kH; gd.K = kH;
-    gd.A = dz; gd.lda = kH;                             // [M][K], K-contiguous
-    gd.B = M->Wb.p + (size_t)l * kH * kH; gd.ldb = kH;  // W[out][in] = [K][N]
-    gd.C = dnext; gd.ldc = kH;
-    gd.Z = M->Z[l].p;
-    gemm<true, false, true, false, kEpiSiluBwd>(gd, s);
-    std::swap(dz, dnext);
-  }
-  weight_grad(M, dz, kH, Xr, kIn, n, G + kOffW1, kIn, G + kOffB1);   // input layer
-}
-
-static void adam(Model* M, float lr) {
+  const int rows = train_rows(n);
+  const unsigned tiles = (unsigned)train_tiles(n);
+  TrainArgs a{X, perm, T, n, M->P.p, M->Wb.p, M->act.p, M->part.p};
+  if (rows == 16)
+    hipLaunchKernelGGL(train_tile_kernel<16>, dim3(tiles), dim3(512), 0, s, a);
+  else
+    hipLaunchKernelGGL(train_tile_kernel<32>, dim3(tiles), dim3(512), 0, s, a);
+  WeightGradArgs w{M->act.p, (int)nblocks(n, kRowBlock), 0, M->ws.p};
+  w.per_slice = (w.blocks + kSplitMax - 1) / kSplitMax;
+  const int slices = (w.blocks + w.per_slice - 1) / w.per_slice;
+  hipLaunchKernelGGL(weight_grad_kernel, dim3(13, (unsigned)slices), dim3(256), 0, s, w);
   const double b1 = 0.9, b2 = 0.999;
-  ++M->adam_t;
-  const float c1 = (float)(1.0 - std::pow(b1, (double)M->adam_t));
-  const float c2 = (float)(1.0 - std::pow(b2, (double)M->adam_t));
-  hipLaunchKernelGGL(adam_step, dim3(nblocks(kParams, 256)), dim3(256), 0, M->stream, M->P.p,
-                     M->G.p, M->m.p, M->v.p, M->Wb.p, lr, (float)b1, (float)b2, 1e-8f, c1, c2);
+  ReduceArgs r{};
+  r.ws = M->ws.p;
+  r.slices = slices;
+  r.part = M->part.p;
+  r.tiles = (int)tiles;
+  r.G = M->G.p;
+  r.loss = M->loss.p;
+  r.adam = lr != nullptr;
+  if (lr) {
+    ++M->adam_t;
+    r.P = M->P.p;
+    r.m = M->m.p;
+    r.v = M->v.p;
+    r.Wb = M->Wb.p;
+    r.lr = *lr;
+    r.b1 = (float)b1;
+    r.b2 = (float)b2;
+    r.eps = 1e-8f;
+    r.c1 = (float)(1.0 - std::pow(b1, (double)M->adam_t));
+    r.c2 = (float)(1.0 - std::pow(b2, (double)M->adam_t));
+  }
+  hipLaunchKernelGGL(reduce_kernel, dim3(kWeightBlocks + kPartBlocks), dim3(256), 0, s, r);
 }
 
 // The goniometer of a call and the model's envelope (if set) for the
@@ -1238,12 +1286,8 @@ void anacor_mlp_destroy(anacor_mlp* mlp) {
     (void)hipSetDevice(M->device);
     if (M->stream) (void)hipStreamSynchronize(M->stream);
     M->P.release(); M->G.release(); M->m.release(); M->v.release(); M->Wb.release();
-    for (int l = 0; l < 4; ++l) {
-      M->Z[l].release();
-      M->H[l].release();
-    }
-    M->dA.release(); M->dB.release(); M->dy.release(); M->xb.release(); M->tb.release();
-    M->part.release(); M->loss.release(); M->ws.release(); M->colws.release();
+    M->act.release(); M->xb.release(); M->tb.release();
+    M->part.release(); M->loss.release(); M->ws.release();
     M->s1.release(); M->omega.release(); M->inv.release(); M->A.release();
     M->X.release(); M->y.release(); M->T.release(); M->flag.release(); M->trust.release();
     M->cell.release();
@@ -1517,13 +1561,12 @@ int anacor_mlp_gradients(anacor_mlp* mlp, const float* x, const float* t, int64_
   std::lock_guard<std::mutex> lk(M->mu);
   MLP_TRY(hipSetDevice(M->device));
   MLP_CHECK(ensure_rows(M, (int)n));
-  MLP_CHECK(M->y.grow((size_t)n));
   MLP_TRY(hipMemcpyAsync(M->xb.p, x, (size_t)n * kIn * sizeof(float), hipMemcpyHostToDevice,
                          M->stream));
   MLP_TRY(hipMemcpyAsync(M->tb.p, t, (size_t)n * sizeof(float), hipMemcpyHostToDevice,
                          M->stream));
   hipLaunchKernelGGL(zero_floats, dim3(1), dim3(64), 0, M->stream, M->loss.p, 1);
-  fwd_bwd(M, M->xb.p, nullptr, M->tb.p, (int)n);
+  train_step(M, M->xb.p, nullptr, M->tb.p, (int)n, nullptr);
   MLP_TRY(hipGetLastError());
   MLP_TRY(hipMemcpyAsync(grad, M->G.p, kParams * sizeof(float), hipMemcpyDeviceToHost,
                          M->stream));
@@ -1545,7 +1588,6 @@ int anacor_mlp_train(anacor_mlp* mlp, const float* x, const float* t, int64_t n,
   std::lock_guard<std::mutex> lk(M->mu);
   MLP_TRY(hipSetDevice(M->device));
   MLP_CHECK(ensure_rows(M, batch));
-  MLP_CHECK(M->y.grow((size_t)batch));
   MLP_CHECK(M->X.grow((size_t)n * kIn));
   MLP_CHECK(M->T.grow((size_t)n));
   DevBuf<int> perm_d;
@@ -1575,10 +1617,10 @@ int anacor_mlp_train(anacor_mlp* mlp, const float* x, const float* t, int64_t n,
       hipLaunchKernelGGL(zero_floats, dim3(1), dim3(64), 0, M->stream, M->loss.p, 1);
       for (int64_t s0 = 0; s0 < n; s0 += batch, ++step) {
         const int c = (int)std::min<int64_t>(batch, n - s0);
-        fwd_bwd(M, M->X.p, perm_d.p + s0, M->T.p, c);
         const double frac = total > 1 ? (double)step / (double)(total - 1) : 1.0;
-        const double cur = lr_min + 0.5 * (lr - lr_min) * (1.0 + std::cos(M_PI * frac));
-        adam(M, (float)cur);
+        const float cur =
+            (float)(lr_min + 0.5 * (lr - lr_min) * (1.0 + std::cos(M_PI * frac)));
+        train_step(M, M->X.p, perm_d.p + s0, M->T.p, c, &cur);
       }
       float l = 0.f;
       if (!hip_ok(hipGetLastError(), "kernel launch") ||
