@@ -207,6 +207,7 @@ struct SkipArgs {
   long long oct_bytes;
   int hx, zs;
   const int4* vox;             // (z | y << 16, x, x word, yz word), wave-grouped
+  const int* index;            // the caller's index of each of them
   int lo[3], hi[3];            // the listed voxels' box (z, y, x): bounds the tables
   int at[3];                   // first table entry of each exit axis
 };
@@ -297,6 +298,165 @@ __device__ __forceinline__ double root_over(double S, double D) {
   return S > 0.0 ? g * q : 0.0;       // a ray held on its origin by the clamps
 }
 
+// One ray direction in a workgroup: its exits, field and table.  Args: the
+// volume's extents Z, Y, X, voxel edges vs and coefficients mu.
+struct SkipRay {
+  AxisExit ez, ey, ex;
+  __amdgpu_buffer_rsrc_t rsrc;
+  float iz, iy, ix;            // 1 / |direction|
+  int sz, sy, sx, oz, oy, ox;  // distance to the exit plane along an axis: o + s * c
+
+  // Builds the tables; every thread of the workgroup, behind a barrier after
+  // the last reader of the previous ray's.
+  template <class Args>
+  __device__ __forceinline__ SkipRay(const RayRule* __restrict__ rr, const Args& a,
+                                     const SkipArgs& k, AxisLds* axes, uint2* tbl)
+      : ez(rr, 0), ey(rr, 1), ex(rr, 2) {
+    const int tid = (int)threadIdx.x;
+    const unsigned mx = 7u | (((1u << k.hx) - 1u) << 7);
+    const unsigned gap_y = mx & ~7u;              // x's high bits: y's carry runs through
+    if (tid < 3) {
+      const AxisExit e = tid == 0 ? ez : tid == 1 ? ey : ex;
+      const double* d = rr->d[e.face];
+      AxisLds& A = axes[tid];
+      A.at = k.at[tid] * (int)sizeof(uint2);
+      A.near = exit_usable(rr, tid, e, max(a.Z, max(a.Y, a.X)), A.scale) ? 0x7fffffff : 0;
+      A.add = e.add;
+      A.hb = (tid == 0 ? a.Y : a.Z) - 1;
+      A.hc = (tid == 2 ? a.Y : a.X) - 1;
+      A.face = e.face;
+      A.up = e.up ? 1 : 0;
+      A.db = d[tid == 0 ? 1 : 0];
+      A.dc = d[tid == 2 ? 1 : 2];
+      A.vb = a.vs[tid == 0 ? 1 : 0];
+      A.vc = a.vs[tid == 2 ? 1 : 2];
+      A.vp = a.vs[tid];
+      A.bias = e.round ? kRoundBias : 0.0;
+    }
+    __syncthreads();
+    // offsets of the increments that any listed voxel takes
+    auto build = [&](const AxisExit& e, int axis, int ext) {
+      const int n = (e.up ? ext - k.lo[axis] : k.hi[axis]) + e.add;
+      uint2* const out = tbl + k.at[axis];
+      const double* d = rr->d[e.face];
+      const double db = axis == 0 ? d[1] : d[0], dc = axis == 2 ? d[1] : d[2];
+      int first = 0x7fffffff;
+      for (int inc = tid; inc < n; inc += kBlock) {
+        bool near = false;
+        const int op = e.up ? inc : -inc;
+        const int ob = step_offset((double)inc * db, e.round, near);
+        const int oc = step_offset((double)inc * dc, e.round, near);
+        const int oz = axis == 0 ? op : ob;
+        const int oy = axis == 0 ? ob : axis == 1 ? op : oc;
+        const int ox = axis == 2 ? op : oc;
+        out[inc] = make_uint2(dilate_x(ox) | 0x78u,
+                              (dilate_y(oy, k.hx) | gap_y) + (unsigned)(oz * k.zs));
+        if (near) first = min(first, inc);
+      }
+      if (first != 0x7fffffff) atomicMin(&axes[axis].near, first);
+    };
+    build(ez, 0, a.Z);
+    build(ey, 1, a.Y);
+    build(ex, 2, a.X);
+    __syncthreads();
+    const int oct = (ez.up ? 0 : 4) | (ey.up ? 0 : 2) | (ex.up ? 0 : 1);
+    rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(k.field + (long long)oct * k.oct_bytes),
+                                             (short)0, (int)k.oct_bytes, 0x00020000);
+    iz = (float)__builtin_fabs(rr->d[0][3]);
+    iy = (float)__builtin_fabs(rr->d[1][3]);
+    ix = (float)__builtin_fabs(rr->d[2][3]);
+    sz = ez.up ? -1 : 1;
+    sy = ey.up ? -1 : 1;
+    sx = ex.up ? -1 : 1;
+    oz = ez.up ? a.Z : 0;
+    oy = ey.up ? a.Y : 0;
+    ox = ex.up ? a.X : 0;
+  }
+
+  // mu * length of one voxel's ray; kRayRedo in err where the walk does not
+  // cover it.  col: this lane's step counters (zero before and after).
+  template <bool EXACT, class Args>
+  __device__ __forceinline__ double trace(const RayRule* __restrict__ rr, const int4 q,
+                                          const Args& a, const SkipArgs& k, const AxisLds* axes,
+                                          const uint2* tbl, uint32_t* col, unsigned& err,
+                                          unsigned& steps) const {
+    double r = 0.0;
+    const unsigned mx = 7u | (((1u << k.hx) - 1u) << 7);
+    const int z = q.x & 0xffff, y = (int)((unsigned)q.x >> 16), x = q.y;
+    // cube_face by FP32 products with the reciprocals; FP64 quotients
+    // decide where two planes are closer than the products' rounding
+    const int kz = mad24(z, sz, oz), ky = mad24(y, sy, oy), kx = mad24(x, sx, ox);
+    const float tz = (float)kz * iz, ty = (float)ky * iy, tx = (float)kx * ix;
+    const bool z_first = tz < ty;
+    const float lo = z_first ? tz : ty, hi = z_first ? ty : tz;
+    const bool x_first = tx < lo;
+    const float t0 = x_first ? tx : lo;
+    const float t1 = x_first ? lo : (hi < tx ? hi : tx);
+    int p = x_first ? 2 : z_first ? 0 : 1;
+    bool use = true;
+    if (!(t1 > t0 * 1.00001f) || min(z, min(y, x)) == 0) {
+      const int face = exit_face<true>(z, y, x, rr->dir[0], rr->dir[1], rr->dir[2],
+                                       rr->d[0][3], rr->d[1][3], rr->d[2][3], a.Z, a.Y, a.X,
+                                       rr->neg != 0);
+      p = (face == 2 || face == 3) ? 0 : (face == 4 || face == 5) ? 1 : 2;
+      use = face - 1 == axes[p].face;
+    }
+    const AxisLds& A = axes[p];
+    const int kp = p == 0 ? kz : p == 1 ? ky : kx;
+    const int limit = kp + A.add;
+    if (!use || limit > A.near) {
+      err |= kRayRedo;
+    } else {
+      const int scale = A.scale;
+      const unsigned xw = (unsigned)q.z, yz = (unsigned)q.w;
+      const char* t = (const char*)tbl + A.at;      // the increment's entry
+      const char* const end = t + (limit << 3);
+      int lab;
+      auto walk = [&](bool unit) {
+        do {
+          const uint2 w = *(const uint2*)t;
+          const unsigned off = bit_select(mx, xw + w.x, yz + w.y);
+          const int b = __builtin_amdgcn_raw_buffer_load_b8(rsrc, (int)off, 0, 0);
+          lab = b & 7;
+          int s8 = b & 0xf8;                        // 8 x steps this label holds for
+          if (!unit) s8 = ((int)(__umul24((unsigned)(s8 - 8), (unsigned)scale) >> 16) & ~7) + 8;
+          atomicAdd(col + lab * kBlock, (unsigned)s8);
+          t += s8;
+        } while (lab != 0 && t < end);
+      };
+      // a wave whose rays all step at most one voxel per axis (most)
+      // skips without scaling
+      if (__all(scale == 65536)) walk(true);
+      else walk(false);
+      // a last label past the end counted the steps beyond it too
+      const int over = (int)(t - end);
+      const int len = lab == 0 ? limit + (over >> 3) - 1 : limit;
+      steps += (unsigned)len;
+      const int n8 = max(lab == 0 ? 0 : over, 0);
+      // sum of mu over the steps, label by label
+      double W = a.mu[0] * (double)(int)(col[1 * kBlock] - (lab == 1 ? n8 : 0));
+      W = __builtin_fma(a.mu[1], (double)(int)(col[2 * kBlock] - (lab == 2 ? n8 : 0)), W);
+      W = __builtin_fma(a.mu[2], (double)(int)(col[3 * kBlock] - (lab == 3 ? n8 : 0)), W);
+      W = __builtin_fma(a.mu[3], (double)(int)(col[4 * kBlock] - (lab == 4 ? n8 : 0)), W);
+#pragma unroll
+      for (int l = 1; l < 5; ++l) col[l * kBlock] = 0;
+      if (len > 1) {
+        const int last = len - 1;
+        const double D = (double)last;
+        const int cb = p == 0 ? y : z, cc = p == 2 ? y : x;
+        const int ib = axis_index<false>((double)cb, D, A.db, A.bias, A.hb);
+        const int ic = axis_index<false>((double)cc, D, A.dc, A.bias, A.hc);
+        const int dp = min(last, kp - A.up);
+        const double b_ = (double)(ib - cb) * A.vb;
+        const double c_ = (double)(ic - cc) * A.vc;
+        const double p_ = (double)dp * A.vp;
+        r = root_over<EXACT>(b_ * b_ + c_ * c_ + p_ * p_, D) * (W * 0.125);
+      }
+    }
+    return r;
+  }
+};
+
 template <bool F64>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(F64 ? 6 : 8)))
 void skip_kernel(TraceArgs a, SkipArgs k) {
@@ -317,8 +477,6 @@ void skip_kernel(TraceArgs a, SkipArgs k) {
   uint32_t* const col = hist + tid;
 #pragma unroll
   for (int l = 1; l < 5; ++l) col[l * kBlock] = 0;
-  const unsigned mx = 7u | (((1u << k.hx) - 1u) << 7);
-  const unsigned gap_y = mx & ~7u;              // x's high bits: y's carry runs through
   TileAcc acc = {0.f, 0.f, 0.0, 0ull, 0u};
   unsigned steps = 0;
   const int v_begin = tile * a.vox_per_tile;
@@ -328,139 +486,12 @@ void skip_kernel(TraceArgs a, SkipArgs k) {
 #pragma unroll 1
     for (int ray = 0; ray < 2; ++ray) {
       const RayRule* __restrict__ rr = &rule->ray[ray];
-      const AxisExit ez(rr, 0), ey(rr, 1), ex(rr, 2);
       __syncthreads();                          // the table's last readers are done
-      if (tid < 3) {
-        const AxisExit e = tid == 0 ? ez : tid == 1 ? ey : ex;
-        const double* d = rr->d[e.face];
-        AxisLds& A = axes[tid];
-        A.at = k.at[tid] * (int)sizeof(uint2);
-        A.near = exit_usable(rr, tid, e, max(a.Z, max(a.Y, a.X)), A.scale) ? 0x7fffffff : 0;
-        A.add = e.add;
-        A.hb = (tid == 0 ? a.Y : a.Z) - 1;
-        A.hc = (tid == 2 ? a.Y : a.X) - 1;
-        A.face = e.face;
-        A.up = e.up ? 1 : 0;
-        A.db = d[tid == 0 ? 1 : 0];
-        A.dc = d[tid == 2 ? 1 : 2];
-        A.vb = a.vs[tid == 0 ? 1 : 0];
-        A.vc = a.vs[tid == 2 ? 1 : 2];
-        A.vp = a.vs[tid];
-        A.bias = e.round ? kRoundBias : 0.0;
-      }
-      __syncthreads();
-      // offsets of the increments that any listed voxel takes
-      auto build = [&](const AxisExit& e, int axis, int ext) {
-        const int n = (e.up ? ext - k.lo[axis] : k.hi[axis]) + e.add;
-        uint2* const out = tbl + k.at[axis];
-        const double* d = rr->d[e.face];
-        const double db = axis == 0 ? d[1] : d[0], dc = axis == 2 ? d[1] : d[2];
-        int first = 0x7fffffff;
-        for (int inc = tid; inc < n; inc += kBlock) {
-          bool near = false;
-          const int op = e.up ? inc : -inc;
-          const int ob = step_offset((double)inc * db, e.round, near);
-          const int oc = step_offset((double)inc * dc, e.round, near);
-          const int oz = axis == 0 ? op : ob;
-          const int oy = axis == 0 ? ob : axis == 1 ? op : oc;
-          const int ox = axis == 2 ? op : oc;
-          out[inc] = make_uint2(dilate_x(ox) | 0x78u,
-                                (dilate_y(oy, k.hx) | gap_y) + (unsigned)(oz * k.zs));
-          if (near) first = min(first, inc);
-        }
-        if (first != 0x7fffffff) atomicMin(&axes[axis].near, first);
-      };
-      build(ez, 0, a.Z);
-      build(ey, 1, a.Y);
-      build(ex, 2, a.X);
-      __syncthreads();
-      const int oct = (ez.up ? 0 : 4) | (ey.up ? 0 : 2) | (ex.up ? 0 : 1);
-      const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-          (void*)(k.field + (long long)oct * k.oct_bytes), (short)0, (int)k.oct_bytes, 0x00020000);
-      const float iz = (float)__builtin_fabs(rr->d[0][3]),
-                  iy = (float)__builtin_fabs(rr->d[1][3]),
-                  ix = (float)__builtin_fabs(rr->d[2][3]);
-      // distance to the exit plane along an axis: off + sgn * c
-      const int sz = ez.up ? -1 : 1, sy = ey.up ? -1 : 1, sx = ex.up ? -1 : 1;
-      const int oz = ez.up ? a.Z : 0, oy = ey.up ? a.Y : 0, ox = ex.up ? a.X : 0;
+      const SkipRay walk(rr, a, k, axes, tbl);
       const int s1 = min(v_end, s0 + kSkipVox * kBlock);
 #pragma unroll 1
       for (int v = s0 + tid; v < s1; v += kBlock) {
-        double r = 0.0;
-        {
-          const int4 q = k.vox[v];
-          const int z = q.x & 0xffff, y = (int)((unsigned)q.x >> 16), x = q.y;
-          // cube_face by FP32 products with the reciprocals; FP64 quotients
-          // decide where two planes are closer than the products' rounding
-          const int kz = mad24(z, sz, oz), ky = mad24(y, sy, oy), kx = mad24(x, sx, ox);
-          const float tz = (float)kz * iz, ty = (float)ky * iy, tx = (float)kx * ix;
-          const bool z_first = tz < ty;
-          const float lo = z_first ? tz : ty, hi = z_first ? ty : tz;
-          const bool x_first = tx < lo;
-          const float t0 = x_first ? tx : lo;
-          const float t1 = x_first ? lo : (hi < tx ? hi : tx);
-          int p = x_first ? 2 : z_first ? 0 : 1;
-          bool use = true;
-          if (!(t1 > t0 * 1.00001f) || min(z, min(y, x)) == 0) {
-            const int face = exit_face<true>(z, y, x, rr->dir[0], rr->dir[1], rr->dir[2],
-                                             rr->d[0][3], rr->d[1][3], rr->d[2][3], a.Z, a.Y, a.X,
-                                             rr->neg != 0);
-            p = (face == 2 || face == 3) ? 0 : (face == 4 || face == 5) ? 1 : 2;
-            use = face - 1 == axes[p].face;
-          }
-          const AxisLds& A = axes[p];
-          const int kp = p == 0 ? kz : p == 1 ? ky : kx;
-          const int limit = kp + A.add;
-          if (!use || limit > A.near) {
-            acc.err |= kRayRedo;
-          } else {
-            const int scale = A.scale;
-            const unsigned xw = (unsigned)q.z, yz = (unsigned)q.w;
-            const char* t = (const char*)tbl + A.at;      // the increment's entry
-            const char* const end = t + (limit << 3);
-            int lab;
-            auto walk = [&](bool unit) {
-              do {
-                const uint2 w = *(const uint2*)t;
-                const unsigned off = bit_select(mx, xw + w.x, yz + w.y);
-                const int b = __builtin_amdgcn_raw_buffer_load_b8(rsrc, (int)off, 0, 0);
-                lab = b & 7;
-                int s8 = b & 0xf8;                        // 8 x steps this label holds for
-                if (!unit) s8 = ((int)(__umul24((unsigned)(s8 - 8), (unsigned)scale) >> 16) & ~7) + 8;
-                atomicAdd(col + lab * kBlock, (unsigned)s8);
-                t += s8;
-              } while (lab != 0 && t < end);
-            };
-            // a wave whose rays all step at most one voxel per axis (most)
-            // skips without scaling
-            if (__all(scale == 65536)) walk(true);
-            else walk(false);
-            // a last label past the end counted the steps beyond it too
-            const int over = (int)(t - end);
-            const int len = lab == 0 ? limit + (over >> 3) - 1 : limit;
-            steps += (unsigned)len;
-            const int n8 = max(lab == 0 ? 0 : over, 0);
-            // sum of mu over the steps, label by label
-            double W = a.mu[0] * (double)(int)(col[1 * kBlock] - (lab == 1 ? n8 : 0));
-            W = __builtin_fma(a.mu[1], (double)(int)(col[2 * kBlock] - (lab == 2 ? n8 : 0)), W);
-            W = __builtin_fma(a.mu[2], (double)(int)(col[3 * kBlock] - (lab == 3 ? n8 : 0)), W);
-            W = __builtin_fma(a.mu[3], (double)(int)(col[4 * kBlock] - (lab == 4 ? n8 : 0)), W);
-#pragma unroll
-            for (int l = 1; l < 5; ++l) col[l * kBlock] = 0;
-            if (len > 1) {
-              const int last = len - 1;
-              const double D = (double)last;
-              const int cb = p == 0 ? y : z, cc = p == 2 ? y : x;
-              const int ib = axis_index<false>((double)cb, D, A.db, A.bias, A.hb);
-              const int ic = axis_index<false>((double)cc, D, A.dc, A.bias, A.hc);
-              const int dp = min(last, kp - A.up);
-              const double b_ = (double)(ib - cb) * A.vb;
-              const double c_ = (double)(ic - cc) * A.vc;
-              const double p_ = (double)dp * A.vp;
-              r = root_over<F64>(b_ * b_ + c_ * c_ + p_ * p_, D) * (W * 0.125);
-            }
-          }
-        }
+        double r = walk.trace<F64>(rr, k.vox[v], a, k, axes, tbl, col, acc.err, steps);
         double* const first = incident + (v - s0);
         if (ray == 0) {
           *first = r;
@@ -483,4 +514,33 @@ void skip_kernel(TraceArgs a, SkipArgs k) {
   const int slot = pos * a.tiles + tile;
   reduce_tile<F64, false>(acc, red, &a.err[refl], a.steps, a.partial32 + slot,
                           a.partial64 + slot);
+}
+
+// The absorption map (grid_map_kernel) by the skip walk: one direction per
+// workgroup and tile, whose table serves every voxel of the tile.  A direction
+// that the walk does not cover is marked and mapped by the stepping kernel.
+// 150x201x187, 4,000 voxels, 7,200 directions: 3.97 ms stepping, 1.22 ms so,
+// marked directions included; bound as skip_kernel is.
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6)))
+void skip_map_kernel(GridArgs a, SkipArgs k) {
+  extern __shared__ uint2 tbl[];
+  __shared__ uint32_t hist[5 * kBlock];
+  __shared__ AxisLds axes[3];
+  const int lb = xcd_logical_block((int)blockIdx.x, (int)gridDim.x);
+  if (lb >= a.n_blocks) return;
+  const int d = lb / a.tiles;
+  const int tile = lb - d * a.tiles;
+  uint32_t* const col = hist + threadIdx.x;
+#pragma unroll
+  for (int l = 1; l < 5; ++l) col[l * kBlock] = 0;
+  const RayRule* __restrict__ rr = a.rays + d;
+  const SkipRay walk(rr, a, k, axes, tbl);
+  unsigned err = 0, steps = 0;
+  const int v_end = min(a.N, (tile + 1) * a.vox_per_tile);
+#pragma unroll 1
+  for (int v = tile * a.vox_per_tile + (int)threadIdx.x; v < v_end; v += kBlock) {
+    const double r = walk.trace<true>(rr, k.vox[v], a, k, axes, tbl, col, err, steps);
+    a.map[(size_t)d * a.N + k.index[v]] = (float)(a.is_exp ? exp(-r) : r);
+  }
+  if (err) atomicOr(&a.err[d], err);
 }

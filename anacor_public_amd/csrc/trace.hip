@@ -931,6 +931,26 @@ void trace_kernel(TraceArgs a) {
                           a.partial64 + slot);
 }
 
+// The absorption-map kernels' arguments (grid_map_kernel, skip_map_kernel).
+struct GridArgs {
+  const uint8_t* vol;
+  int vol_bytes, cz, cy;
+  int Z, Y, X;
+  const int4* coords;          // (z, y, x, caller index)
+  int N;
+  const RayRule* rays;         // [D] one ray per direction
+  const int* dirs;             // directions of this launch (null: all, in order)
+  int D, tiles, vox_per_tile, n_blocks;
+  double vs[3];
+  double mu[4];
+  int is_exp;
+  float* map;                  // [D][N], voxels in the caller's order
+  double* map64;               // same, unrounded (nullable)
+  unsigned* err;               // [D]
+  const double* incd;          // (double)i for i = 0 .. incd_last
+  int incd_last;
+};
+
 #include "skip_walk.h"
 
 // Per reflection: combine the tile partials in tile order and divide by N.
@@ -1027,24 +1047,6 @@ __global__ void batch_finish_kernel(const BatchSample* __restrict__ samples, int
 // IsExp = 0, stored as float), then per reflection a look-up of the incident
 // and the diffracted direction and the mean of exp(-(m1 + m2)).
 
-struct GridArgs {
-  const uint8_t* vol;
-  int vol_bytes, cz, cy;
-  int Z, Y, X;
-  const int4* coords;          // (z, y, x, caller index)
-  int N;
-  const RayRule* rays;         // [D] one ray per direction
-  int D, tiles, vox_per_tile, n_blocks;
-  double vs[3];
-  double mu[4];
-  int is_exp;
-  float* map;                  // [D][N], voxels in the caller's order
-  double* map64;               // same, unrounded (nullable)
-  unsigned* err;               // [D]
-  const double* incd;          // (double)i for i = 0 .. incd_last
-  int incd_last;
-};
-
 template <int CAP, int U, bool GUARD, bool FULL, int LAYOUT>
 __global__ __launch_bounds__(kBlock)
 __attribute__((amdgpu_waves_per_eu(LAYOUT >= kLayoutBrick2 ? 1 : 5)))
@@ -1052,8 +1054,9 @@ void grid_map_kernel(GridArgs a) {
   __shared__ uint32_t seg_lds[seg_slots(CAP, U) * kBlock];
   const int lb = xcd_logical_block((int)blockIdx.x, (int)gridDim.x);
   if (lb >= a.n_blocks) return;
-  const int d = lb / a.tiles;
-  const int tile = lb - d * a.tiles;
+  const int row = lb / a.tiles;
+  const int tile = lb - row * a.tiles;
+  const int d = a.dirs ? a.dirs[row] : row;
   const Volume V = make_volume(a.vol, a.Z, a.Y, a.X, a.vol_bytes, a.cz, a.cy, a.incd,
                                a.incd_last);
   lds_u32* seg = (lds_u32*)(seg_lds + threadIdx.x);
@@ -1319,6 +1322,7 @@ struct Context {
   uint8_t* d_field = nullptr;
   FieldShape field{};
   int4* d_skip_vox = nullptr;
+  int* d_skip_index = nullptr;           // the caller's index of each
   int box_lo[3] = {0, 0, 0}, box_hi[3] = {0, 0, 0};   // of the voxel list (z, y, x)
   double vs[3] = {1, 1, 1};
   double mu[4] = {0, 0, 0, 0};
@@ -1738,13 +1742,15 @@ static int launch_group(const Context* c, int layout) {
   return (layout == kLayoutBrick2 || layout == kLayoutBrick4) ? kBrickGroup : 1;
 }
 
-static void launch_skip(const Context* c, const TraceArgs& a, int grid, bool f64, hipStream_t s) {
+// The skip walk's arguments and the bytes of its tables.
+static SkipArgs skip_args(const Context* c, unsigned* lds) {
   SkipArgs k;
   k.field = c->d_field;
   k.oct_bytes = c->field.bytes;
   k.hx = c->field.hx;
   k.zs = c->field.zs;
   k.vox = c->d_skip_vox;
+  k.index = c->d_skip_index;
   const int ext[3] = {c->Z, c->Y, c->X};
   int entries = 0;
   for (int i = 0; i < 3; ++i) {
@@ -1753,7 +1759,13 @@ static void launch_skip(const Context* c, const TraceArgs& a, int grid, bool f64
     k.at[i] = entries;
     entries += std::max(ext[i] - k.lo[i], k.hi[i]) + 1;
   }
-  const unsigned lds = (unsigned)(entries * sizeof(uint2));
+  *lds = (unsigned)(entries * sizeof(uint2));
+  return k;
+}
+
+static void launch_skip(const Context* c, const TraceArgs& a, int grid, bool f64, hipStream_t s) {
+  unsigned lds;
+  const SkipArgs k = skip_args(c, &lds);
   if (f64)
     hipLaunchKernelGGL((skip_kernel<true>), dim3((unsigned)grid), dim3(kBlock), lds, s, a, k);
   else
@@ -2159,13 +2171,18 @@ static int upload_skip_voxels(Context* c) {
     }
   }
   const FieldShape& f = c->field;
-  for (int4& q : v) {
+  std::vector<int> index(n);
+  for (size_t i = 0; i < n; ++i) {
+    int4& q = v[i];
     const int z = q.x, y = q.y, x = q.z;
+    index[i] = q.w;
     q = make_int4(z | (y << 16), x, (int)dilate_x(x + 1),
                   (int)(dilate_y(y + 1, f.hx) + (unsigned)((z + 1) * f.zs)));
   }
   if (!c->d_skip_vox) HIP_TRY(hipMalloc(&c->d_skip_vox, n * sizeof(int4)));
   HIP_TRY(hipMemcpy(c->d_skip_vox, v.data(), n * sizeof(int4), hipMemcpyHostToDevice));
+  if (!c->d_skip_index) HIP_TRY(hipMalloc(&c->d_skip_index, n * sizeof(int)));
+  HIP_TRY(hipMemcpy(c->d_skip_index, index.data(), n * sizeof(int), hipMemcpyHostToDevice));
   return ANACOR_OK;
 }
 
@@ -2390,6 +2407,7 @@ static void ctx_destroy(Context* c) {
   if (c->d_coords) (void)hipFree(c->d_coords);
   if (c->d_field) (void)hipFree(c->d_field);
   if (c->d_skip_vox) (void)hipFree(c->d_skip_vox);
+  if (c->d_skip_index) (void)hipFree(c->d_skip_index);
   if (c->d_rules) (void)hipFree(c->d_rules);
   if (c->d_partial) (void)hipFree(c->d_partial);
   if (c->d_err) (void)hipFree(c->d_err);
@@ -3062,6 +3080,14 @@ static void grid_free(Grid* g) {
   delete g;
 }
 
+// Voxels per workgroup of the map by the skip walk: up to 16 per lane, to build
+// a direction's table once, while 4,096 workgroups remain.
+static int skip_map_tile(int N, int D) {
+  const int64_t tiles = std::max<int64_t>(1, (4096 + D - 1) / D);
+  const int64_t vpt = ((N + tiles - 1) / tiles + kBlock - 1) / kBlock * kBlock;
+  return (int)std::min<int64_t>(vpt, 16 * kBlock);
+}
+
 // Absorption maps of every crystal voxel of c for D directions.
 static int grid_build(Context* c, int64_t n_theta, int64_t n_phi, const double* rotated_s1,
                       const double* theta_phi, int is_exp, Grid** out,
@@ -3085,6 +3111,8 @@ static int grid_build(Context* c, int64_t n_theta, int64_t n_phi, const double* 
   if (rc) { grid_free(g); return rc; }
   RayRule* d_rays = nullptr;
   unsigned* d_err = nullptr;
+  std::vector<int> marked;     // directions that the skip walk leaves to the stepping kernel
+  DeviceTemp marked_buf;
   auto fail = [&](hipError_t e, const char* what) {
     set_error(ANACOR_ERR_HIP, "gridding: %s failed: %s", what, hipGetErrorString(e));
     if (d_rays) (void)hipFree(d_rays);
@@ -3105,8 +3133,10 @@ static int grid_build(Context* c, int64_t n_theta, int64_t n_phi, const double* 
   if ((e = hipMemsetAsync(d_err, 0, (size_t)D * sizeof(unsigned), c->stream)) != hipSuccess)
     return fail(e, "hipMemsetAsync");
   std::vector<unsigned> h_err((size_t)D, 0u);
+  // the skip walk as in use_skip; the unrounded map keeps the stepping kernel
+  const bool skip = skip_ready(c) && !d_map64 && (int64_t)D * N > (1 << 20);
   if (N > 0) {
-    const int vpt = fit_tile(N, D, choose_tile(c, D));
+    const int vpt = fit_tile(N, D, skip ? skip_map_tile(N, D) : choose_tile(c, D));
     if (vpt == 0) {
       (void)hipFree(d_rays);
       (void)hipFree(d_err);
@@ -3126,6 +3156,7 @@ static int grid_build(Context* c, int64_t n_theta, int64_t n_phi, const double* 
     a.coords = c->d_coords;
     a.N = N;
     a.rays = d_rays;
+    a.dirs = nullptr;
     a.D = D;
     a.tiles = (int)tiles;
     a.vox_per_tile = vpt;
@@ -3140,8 +3171,34 @@ static int grid_build(Context* c, int64_t n_theta, int64_t n_phi, const double* 
     a.incd_last = c->incd_last;
     if ((e = hipEventRecord(c->ev0, c->stream)) != hipSuccess) return fail(e, "event");
     const int i = (guard ? 1 : 0) | (c->full ? 2 : 0) | (c->layout << 2);
-    kLaunchGrid[i](a, (int)((nblk + 7) / 8 * 8), c->stream);
-    if ((e = hipGetLastError()) != hipSuccess) return fail(e, "grid_map_kernel");
+    if (skip) {
+      unsigned lds;
+      const SkipArgs k = skip_args(c, &lds);
+      hipLaunchKernelGGL(skip_map_kernel, dim3((unsigned)((nblk + 7) / 8 * 8)), dim3(kBlock), lds,
+                         c->stream, a, k);
+      if ((e = hipGetLastError()) != hipSuccess) return fail(e, "skip_map_kernel");
+      if ((e = hipMemcpyAsync(h_err.data(), d_err, (size_t)D * sizeof(unsigned),
+                              hipMemcpyDeviceToHost, c->stream)) != hipSuccess ||
+          (e = hipStreamSynchronize(c->stream)) != hipSuccess)
+        return fail(e, "skip_map_kernel");
+      for (int d = 0; d < D; ++d)
+        if (h_err[(size_t)d]) marked.push_back(d);
+      if (!marked.empty()) {       // these directions by the stepping kernel
+        if ((e = hipMalloc(&marked_buf.p, marked.size() * sizeof(int))) != hipSuccess ||
+            (e = hipMemcpyAsync(marked_buf.p, marked.data(), marked.size() * sizeof(int),
+                                hipMemcpyHostToDevice, c->stream)) != hipSuccess ||
+            (e = hipMemsetAsync(d_err, 0, (size_t)D * sizeof(unsigned), c->stream)) != hipSuccess)
+          return fail(e, "marked directions");
+        a.dirs = (const int*)marked_buf.p;
+        a.vox_per_tile = fit_tile(N, D, choose_tile(c, (int64_t)marked.size()));
+        a.tiles = (N + a.vox_per_tile - 1) / a.vox_per_tile;
+        a.n_blocks = (int)marked.size() * a.tiles;
+      }
+    }
+    if (!skip || !marked.empty()) {
+      kLaunchGrid[i](a, (a.n_blocks + 7) / 8 * 8, c->stream);
+      if ((e = hipGetLastError()) != hipSuccess) return fail(e, "grid_map_kernel");
+    }
     if ((e = hipEventRecord(c->ev1, c->stream)) != hipSuccess) return fail(e, "event");
   }
   if ((e = hipMemcpyAsync(h_err.data(), d_err, (size_t)D * sizeof(unsigned),
