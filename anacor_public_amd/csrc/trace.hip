@@ -1324,6 +1324,9 @@ struct Context {
   // skip walk: eight octants of free distances, the voxel list in its order
   uint8_t* d_field = nullptr;
   FieldShape field{};
+  uint8_t* d_fine = nullptr;             // by cells: single labels; null: by voxels
+  size_t fine_bytes = 0;
+  CellShape cells{};
   int4* d_skip_vox = nullptr;
   int* d_skip_index = nullptr;           // the caller's index of each
   int box_lo[3] = {0, 0, 0}, box_hi[3] = {0, 0, 0};   // of the voxel list (z, y, x)
@@ -1442,8 +1445,8 @@ static int fit_tile(int64_t n, int64_t R, int vpt) {
 // 512, 864 ms at 384, 894 ms at 256; the same volume with seed 7, 6k
 // reflections: 580, 527, 544 ms; 700x900x900, 80k voxels: 398, 378, 378 ms).
 // The skip walk (kTileSkip) narrows to two voxels per lane where the volume is
-// larger than the caches: 1000x1000x800, 1,500 reflections: 59.1 ms at 1,024,
-// 52.5 at 512, 49.0 at 256; 700x640x680, 3,000: 13.9, 12.4, 12.3 ms.
+// larger than the caches (by voxels, 1000x1000x800, 1,500 reflections: 59.1 ms
+// at 1,024, 52.5 at 512; by cells 29.5, 29.0 and 32.5 at 256).
 static bool is_bricked(int layout);
 constexpr int kTileSkip = -2;
 constexpr long long kCachedVolume = 64ll << 20;   // bytes
@@ -1757,10 +1760,14 @@ static int launch_group(const Context* c, int layout) {
 // The skip walk's arguments and the bytes of its tables.
 static SkipArgs skip_args(const Context* c, unsigned* lds) {
   SkipArgs k;
+  const bool cells = c->d_fine != nullptr;
   k.field = c->d_field;
   k.oct_bytes = c->field.bytes;
-  k.hx = c->field.hx;
-  k.zs = c->field.zs;
+  k.hx = cells ? c->cells.hx : c->field.hx;
+  k.zs = cells ? c->cells.tiles : c->field.zs;
+  k.fine = c->d_fine;
+  k.fine_bytes = (unsigned)c->fine_bytes;
+  k.fine_shift = c->cells.shift;
   k.vox = c->d_skip_vox;
   k.index = c->d_skip_index;
   const int ext[3] = {c->Z, c->Y, c->X};
@@ -1771,17 +1778,17 @@ static SkipArgs skip_args(const Context* c, unsigned* lds) {
     k.at[i] = entries;
     entries += std::max(ext[i] - k.lo[i], k.hi[i]) + 1;
   }
-  *lds = (unsigned)(entries * sizeof(uint2));
+  *lds = (unsigned)(entries * (cells ? sizeof(CellField::Words) : sizeof(VoxelField::Words)));
   return k;
 }
 
 static void launch_skip(const Context* c, const TraceArgs& a, int grid, bool f64, hipStream_t s) {
   unsigned lds;
   const SkipArgs k = skip_args(c, &lds);
-  if (f64)
-    hipLaunchKernelGGL((skip_kernel<true>), dim3((unsigned)grid), dim3(kBlock), lds, s, a, k);
-  else
-    hipLaunchKernelGGL((skip_kernel<false>), dim3((unsigned)grid), dim3(kBlock), lds, s, a, k);
+  auto* const kernel =
+      c->d_fine ? (f64 ? skip_kernel<CellField, true> : skip_kernel<CellField, false>)
+                : (f64 ? skip_kernel<VoxelField, true> : skip_kernel<VoxelField, false>);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kBlock), lds, s, a, k);
 }
 
 // A call of few reflections as one record, in page-locked memory and on the
@@ -2244,6 +2251,11 @@ static int upload_skip_voxels(Context* c) {
     int4& q = v[i];
     const int z = q.x, y = q.y, x = q.z;
     index[i] = q.w;
+    if (c->d_fine) {
+      const CellField::Words w = CellField::dilate(z + 1, y + 1, x + 1, c->cells.hx);
+      q = make_int4(z | (y << 16), x, (int)w.x, (int)w.y);
+      continue;
+    }
     q = make_int4(z | (y << 16), x, (int)dilate_x(x + 1),
                   (int)(dilate_y(y + 1, f.hx) + (unsigned)((z + 1) * f.zs)));
   }
@@ -2254,57 +2266,14 @@ static int upload_skip_voxels(Context* c) {
   return ANACOR_OK;
 }
 
-// The skip walk's field, where the walk's rules hold: no full_iteration, every
-// label in 0..4, every listed voxel of label 3, finite coefficients and voxel
-// edges whose squares are normal, extents within the tables and offsets.
-// Without the device memory for it the stepping kernels trace as before.
-static int field_build(Context* c) {
-  FieldShape f;
-  f.Z = c->Z; f.Y = c->Y; f.X = c->X;
-  const int Z2 = c->Z + 2, Y2 = c->Y + 2, X2 = c->X + 2;
-  if (c->N == 0 || c->full || c->labels_over4 ||
-      std::max(c->Z, std::max(c->Y, c->X)) > kSkipMaxExtent)
-    return ANACOR_OK;
-  for (double v : c->mu)
-    if (!(std::fabs(v) < 0x1p300)) return ANACOR_OK;
-  for (double v : c->vs)
-    if (!(std::fabs(v) > 0x1p-300 && std::fabs(v) < 0x1p300)) return ANACOR_OK;
-  f.nbx = (X2 + 7) / 8;
-  f.nby = (Y2 + 15) / 16;
-  f.hx = 0;
-  while ((1 << f.hx) < f.nbx) ++f.hx;
-  const int64_t zs = (int64_t)f.nby << (7 + f.hx);
-  if (zs * Z2 >= (1ll << 31)) return ANACOR_OK;
-  f.zs = (int)zs;
-  f.bytes = zs * Z2;
-  f.wx = (X2 + 31) / 32;
-  const long long plane = (long long)Z2 * Y2 * f.wx;
-  // a large volume's field (eight bytes per voxel) takes at most a quarter of
-  // the free memory, so that contexts created later still find theirs
-  if (f.bytes >= (32ll << 20)) {
-    size_t free_bytes = 0, total = 0;
-    if (hipMemGetInfo(&free_bytes, &total) != hipSuccess) {
-      (void)hipGetLastError();
-      return ANACOR_OK;
-    }
-    if ((size_t)f.bytes * 8 > free_bytes / 4) return ANACOR_OK;
-  }
-  DeviceTemp planes, flag;
-  if (hipMalloc(&planes.p, (size_t)plane * kLevels * sizeof(uint32_t)) != hipSuccess ||
-      hipMalloc(&c->d_field, (size_t)f.bytes * 8) != hipSuccess) {
-    (void)hipGetLastError();
-    c->d_field = nullptr;
-    return ANACOR_OK;
-  }
-  HIP_TRY(hipMalloc(&flag.p, sizeof(unsigned)));
-  HIP_TRY(hipMemsetAsync(flag.p, 0, sizeof(unsigned), c->stream));
-  hipLaunchKernelGGL(origin_label_kernel, dim3((unsigned)((c->N + 255) / 256)), dim3(256), 0,
-                     c->stream, c->d_vol, c->Y, c->X, c->d_coords, c->N, (unsigned*)flag.p);
-  HIP_TRY(hipGetLastError());
-  uint32_t* const P = (uint32_t*)planes.p;
-  const long long waves = (long long)Z2 * Y2 * ((f.wx + 1) / 2);
+// Bit planes of the cubes of one label (kLevels of them into P) over the
+// volume vol of Z x Y x X with its zero shell, wx words per padded row.
+static int field_planes(Context* c, const uint8_t* vol, int Z, int Y, int X, int wx, uint32_t* P) {
+  const int Z2 = Z + 2, Y2 = Y + 2;
+  const long long plane = (long long)Z2 * Y2 * wx;
+  const long long waves = (long long)Z2 * Y2 * ((wx + 1) / 2);
   hipLaunchKernelGGL(field_base_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, c->stream,
-                     c->d_vol, c->Z, c->Y, c->X, f.wx, waves, P);
+                     vol, Z, Y, X, wx, waves, P);
   HIP_TRY(hipGetLastError());
   // by index into kLevelSide: 1 -> 2; 2 -> 3, 4; 4 -> 5 .. 8; 8 -> 12, 16; 16 -> 24, 30
   struct Pass { int from, n, to[4], s[4]; };
@@ -2321,22 +2290,133 @@ static int field_build(Context* c) {
       e.out[i] = P + p.to[i] * plane;
       e.s[i] = p.s[i];
     }
-    e.Z2 = Z2; e.Y2 = Y2; e.wx = f.wx;
+    e.Z2 = Z2; e.Y2 = Y2; e.wx = wx;
     hipLaunchKernelGGL(field_erode_kernel, dim3((unsigned)((plane + 255) / 256)), dim3(256), 0,
                        c->stream, e);
     HIP_TRY(hipGetLastError());
   }
+  return ANACOR_OK;
+}
+
+// The field of voxels (planes in P) or, with its labels, of cells; false when
+// the offsets or the device memory do not allow it.
+static int voxel_field(Context* c, DeviceTemp& planes, bool* built) {
+  FieldShape f;
+  f.Z = c->Z; f.Y = c->Y; f.X = c->X;
+  const int Z2 = c->Z + 2, Y2 = c->Y + 2, X2 = c->X + 2;
+  f.nbx = (X2 + 7) / 8;
+  f.nby = (Y2 + 15) / 16;
+  f.hx = 0;
+  while ((1 << f.hx) < f.nbx) ++f.hx;
+  const int64_t zs = (int64_t)f.nby << (7 + f.hx);
+  if (zs * Z2 >= (1ll << 31)) return ANACOR_OK;
+  f.zs = (int)zs;
+  f.bytes = zs * Z2;
+  f.wx = (X2 + 31) / 32;
+  const long long plane = (long long)Z2 * Y2 * f.wx;
+  if (hipMalloc(&planes.p, (size_t)plane * kLevels * sizeof(uint32_t)) != hipSuccess ||
+      hipMalloc(&c->d_field, (size_t)f.bytes * 8) != hipSuccess) {
+    (void)hipGetLastError();
+    c->d_field = nullptr;
+    return ANACOR_OK;
+  }
+  uint32_t* const P = (uint32_t*)planes.p;
+  const int rc = field_planes(c, c->d_vol, c->Z, c->Y, c->X, f.wx, P);
+  if (rc) return rc;
   const long long threads = (long long)Z2 * f.nby * f.nbx * 16;
   hipLaunchKernelGGL(field_pack_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
                      c->stream, c->d_vol, f, P, plane, c->d_field);
   HIP_TRY(hipGetLastError());
   c->field = f;
-  const int rc = upload_skip_voxels(c);   // host work beside the kernels
+  *built = true;
+  return ANACOR_OK;
+}
+
+static int cell_field(Context* c, DeviceTemp& planes, DeviceTemp& labels, bool* built) {
+  CellShape s;
+  s.Z = (c->Z + 5) / 4; s.Y = (c->Y + 5) / 4; s.X = (c->X + 5) / 4;   // of the padded volume
+  s.shift = c->labels_over3 ? 1 : 2;
+  const int nxt = (s.X + 7) / 8, nyt = (s.Y + 3) / 4, nzt = (s.Z + 3) / 4;
+  s.hx = 0;
+  while ((1 << s.hx) < nxt) ++s.hx;
+  s.tiles = nyt << s.hx;
+  const int64_t slots = (int64_t)nzt * s.tiles << 13;
+  if (slots >= (1ll << 32)) return ANACOR_OK;
+  FieldShape f{};
+  f.bytes = slots >> 6;
+  f.wx = (s.X + 2 + 31) / 32;
+  const long long ncell = (long long)(s.Z + 2) * (s.Y + 2) * (s.X + 2);
+  const long long plane = (long long)(s.Z + 2) * (s.Y + 2) * f.wx;
+  uint8_t* fine = nullptr;
+  if (hipMalloc(&planes.p, (size_t)plane * kLevels * sizeof(uint32_t)) != hipSuccess ||
+      hipMalloc(&labels.p, (size_t)ncell) != hipSuccess ||
+      hipMalloc(&c->d_field, (size_t)f.bytes * 8) != hipSuccess ||
+      hipMalloc(&fine, (size_t)(slots >> s.shift)) != hipSuccess) {
+    (void)hipGetLastError();
+    if (c->d_field) (void)hipFree(c->d_field);
+    c->d_field = nullptr;
+    return ANACOR_OK;
+  }
+  c->d_fine = fine;
+  c->fine_bytes = (size_t)(slots >> s.shift);
+  hipLaunchKernelGGL(cell_label_kernel, dim3((unsigned)((ncell + 255) / 256)), dim3(256), 0,
+                     c->stream, c->d_vol, c->Z, c->Y, c->X, s, (uint8_t*)labels.p,
+                     (uint32_t*)c->d_fine);
+  HIP_TRY(hipGetLastError());
+  uint32_t* const P = (uint32_t*)planes.p;
+  const int rc = field_planes(c, (const uint8_t*)labels.p, s.Z, s.Y, s.X, f.wx, P);
+  if (rc) return rc;
+  const long long threads = (long long)s.Z * s.Y * s.X;
+  hipLaunchKernelGGL(cell_pack_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
+                     c->stream, (const uint8_t*)labels.p, s, f.wx, P, plane, c->d_field, f.bytes);
+  HIP_TRY(hipGetLastError());
+  c->field = f;
+  c->cells = s;
+  *built = true;
+  return ANACOR_OK;
+}
+
+// The skip walk's field, where the walk's rules hold: no full_iteration, every
+// label in 0..4, every listed voxel of label 3, finite coefficients and voxel
+// edges whose squares are normal, extents within the tables and offsets.
+// Without the device memory for it the stepping kernels trace as before.
+// By cells in volumes past 160 MB, whose voxel field outgrows the caches by too
+// much (450x460x440, 20,000 voxels, 3,000 reflections: 6.3 ms by voxels, 7.6 by
+// cells; 700x640x680: 12.4 and 9.7 ms; 1000x1000x800: 53.9 and 29.7 ms).
+constexpr long long kCellVolume = 160ll << 20;
+static int field_build(Context* c) {
+  if (c->N == 0 || c->full || c->labels_over4 ||
+      std::max(c->Z, std::max(c->Y, c->X)) > kSkipMaxExtent)
+    return ANACOR_OK;
+  for (double v : c->mu)
+    if (!(std::fabs(v) < 0x1p300)) return ANACOR_OK;
+  for (double v : c->vs)
+    if (!(std::fabs(v) > 0x1p-300 && std::fabs(v) < 0x1p300)) return ANACOR_OK;
+  // at most a quarter of the free memory (eight bytes per voxel, or a cell's
+  // eight and its labels), so that contexts created later still find theirs
+  size_t free_bytes = 0, total = 0;
+  if (hipMemGetInfo(&free_bytes, &total) != hipSuccess) {
+    (void)hipGetLastError();
+    return ANACOR_OK;
+  }
+  const bool by_cells = c->vol_bytes > kCellVolume;
+  if ((size_t)c->vol_bytes * (by_cells ? 1 : 10) > free_bytes / 4) return ANACOR_OK;
+  DeviceTemp planes, labels, flag;
+  HIP_TRY(hipMalloc(&flag.p, sizeof(unsigned)));
+  HIP_TRY(hipMemsetAsync(flag.p, 0, sizeof(unsigned), c->stream));
+  hipLaunchKernelGGL(origin_label_kernel, dim3((unsigned)((c->N + 255) / 256)), dim3(256), 0,
+                     c->stream, c->d_vol, c->Y, c->X, c->d_coords, c->N, (unsigned*)flag.p);
+  HIP_TRY(hipGetLastError());
+  bool built = false;
+  int rc = by_cells ? cell_field(c, planes, labels, &built) : voxel_field(c, planes, &built);
+  if (!rc && built) rc = upload_skip_voxels(c);   // host work beside the kernels
   if (rc) return rc;
   unsigned other = 0;
   HIP_TRY(hipMemcpyAsync(&other, flag.p, sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
-  if (other) {
+  unsigned lds = 0;
+  if (built) (void)skip_args(c, &lds);
+  if (built && (other || lds > kSkipTableBytes)) {
     HIP_TRY(hipFree(c->d_field));
     c->d_field = nullptr;
   }
@@ -2474,6 +2554,7 @@ static void ctx_destroy(Context* c) {
   if (c->d_pack) (void)hipFree(c->d_pack);
   if (c->d_coords) (void)hipFree(c->d_coords);
   if (c->d_field) (void)hipFree(c->d_field);
+  if (c->d_fine) (void)hipFree(c->d_fine);
   if (c->d_skip_vox) (void)hipFree(c->d_skip_vox);
   if (c->d_skip_index) (void)hipFree(c->d_skip_index);
   if (c->d_rules) (void)hipFree(c->d_rules);
@@ -3240,7 +3321,8 @@ static int grid_build(Context* c, int64_t n_theta, int64_t n_phi, const double* 
     if (skip) {
       unsigned lds;
       const SkipArgs k = skip_args(c, &lds);
-      hipLaunchKernelGGL(skip_map_kernel, dim3((unsigned)((nblk + 7) / 8 * 8)), dim3(kBlock), lds,
+      auto* const kernel = c->d_fine ? skip_map_kernel<CellField> : skip_map_kernel<VoxelField>;
+      hipLaunchKernelGGL(kernel, dim3((unsigned)((nblk + 7) / 8 * 8)), dim3(kBlock), lds,
                          c->stream, a, k);
       if ((e = hipGetLastError()) != hipSuccess) return fail(e, "skip_map_kernel");
       if ((e = hipMemcpyAsync(h_err.data(), d_err, (size_t)D * sizeof(unsigned),
