@@ -87,12 +87,25 @@ __device__ __forceinline__ float silu_grad(float z) {
 // writes A = exp(y std + mean) inside the envelope and NaN outside.
 
 constexpr int kHP = kH + 8;   // padded LDS row of activations (bf16)
-// BF16 weight block: W2, W3, W4 [256][256], then W1 hi and lo [256][kInK],
-// then W2, W3, W4 transposed (the backward pass's operand).
+// BF16 weight block: W2, W3, W4, then W1 hi and lo [256][kInK], then W2, W3, W4
+// transposed (the backward pass's operand).  The 256x256 ones lie in the order
+// of the MFMA's fragments, [16 units][32 k][lane][8]: a wave's load is 1 KB in
+// one piece, where rows of 256 give it half of 16 lines that the L1 loses before
+// the other half is asked for (training tiles,
+// 4,096 rows: 41 us in rows, 32 so; inference, a million rows: 1.29 and 1.04 ms).
 constexpr size_t kWbW1h = (size_t)3 * kH * kH;
 constexpr size_t kWbW1l = kWbW1h + (size_t)kH * kInK;
 constexpr size_t kWbT = kWbW1l + (size_t)kH * kInK;
 constexpr size_t kWbSize = kWbT + (size_t)3 * kH * kH;
+// element (unit, k) of a 256x256 block
+__device__ __forceinline__ int frag_index(int unit, int k) {
+  return (((unit >> 4) * 8 + (k >> 5)) * 64 + ((k >> 3) & 3) * 16 + (unit & 15)) * 8 + (k & 7);
+}
+// a lane's fragment of 16 units at `unit` and 32 k at `k`
+__device__ __forceinline__ const __bf16* frag(const __bf16* __restrict__ W, int unit, int k,
+                                              int lane) {
+  return W + (((unit >> 4) * 8 + (k >> 5)) * 64 + lane) * 8;
+}
 
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
@@ -158,7 +171,7 @@ __global__ __launch_bounds__(256) void mlp_infer_kernel(
         bf16x8 w[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          w[i] = *(const bf16x8*)(W + (size_t)(ub + i * 16 + r16) * kH + k0 + kg);
+          w[i] = *(const bf16x8*)frag(W, ub + i * 16, k0, lane);
 #pragma unroll
         for (int j = 0; j < RT; ++j) {
           const bf16x8 hh = *(const bf16x8*)&Hh[j * 16 + r16][k0 + kg];
@@ -227,8 +240,8 @@ __global__ __launch_bounds__(256) void mlp_infer_kernel(
 // gradients, split over the rows) and reduce_kernel (the slices' sums, the
 // bias gradients and the loss, with Adam in place).  Layer by layer, with
 // pre-activations, activations and dZ in FP32 through memory, it was 22
-// launches and 270 us at 4,096 rows (67 us now: 42, 16 and 8), 566 us at 16,384
-// (149 us: 97, 44 and 9).
+// launches and 270 us at 4,096 rows (56 us now: 32, 16 and 8), 566 us at 16,384
+// (126 us: 74, 43 and 9).
 //
 // Operands of the weight gradients, dW[out][in] = sum_b dZ[b][out] H[b][in],
 // leave the tile kernel as the MFMA reads them: BF16 hi and lo planes in blocks of
@@ -268,25 +281,34 @@ __device__ __forceinline__ void split_bf16(float v, __bf16& hi, __bf16& lo) {
   lo = (__bf16)(v - (float)hi);
 }
 
+// A barrier for data in LDS: unlike __syncthreads() it leaves global loads and
+// stores in flight.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 // Forward and backward of ROWS rows in one workgroup of 8 waves, wave w the
 // units 32 w .. 32 w + 31 of every layer.  MFMA with the rows as M: a lane
 // holds 4 consecutive rows of one unit, which is both a run of a weight-gradient
 // operand plane and, forward and backward, the same (row, unit) pairs of every
-// layer, so SiLU' of the four layers stays in registers.  Activations and dZ
+// layer, so SiLU' waits in LDS at the thread's own place.  Activations and dZ
 // pass between layers in LDS as hi/lo [row][unit]; weights come from L2 as
 // 16-byte fragments.  The input layer runs on the FP32 MFMA (k in the order 16
 // s + 4 (l / 16) + e, the same for both operands).
 //
-// What bounds it: the chain of seven layers, each a round of weight fragments
-// from L2 between two barriers (42 us for 256 workgroups of 16 rows, 97 us for
-// 512 of 32).  Rows per workgroup: the weights' 0.86 MB per workgroup ask for
-// more rows, a batch of 4,096 for enough workgroups.
+// What bounds it: the weights' 0.86 MB per workgroup out of L2 (32 us for 256
+// workgroups of 16 rows, 74 us for 512 of 32: 7 and 6 TB/s), in rounds between two
+// barriers per layer.  SiLU' in registers and the layers unrolled: 43 us at the
+// fragments of then (41 rolled); fetching a layer's fragments ahead of its barrier
+// changed nothing.  Rows per workgroup: the weights ask for more rows, a batch of
+// 4,096 for enough workgroups.
 template <int ROWS>
 __global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
   constexpr int RT = ROWS / 16;
   static_assert(ROWS == 16 || ROWS == 32, "row tile");
   __shared__ __attribute__((aligned(16))) __bf16 Hh[ROWS][kHP];
   __shared__ __attribute__((aligned(16))) __bf16 Hl[ROWS][kHP];
+  __shared__ floatx4 slope[3][2 * RT][512];       // SiLU' of layers 1-3, by thread
   __shared__ float head[8][ROWS];
   const int t = (int)threadIdx.x, lane = t & 63, wave = t >> 6;
   const int r16 = lane & 15, quad = lane >> 4, kg = quad * 8, q4 = quad * 4;
@@ -297,7 +319,7 @@ __global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
   float* const part = a.part + (size_t)blockIdx.x * kPart;
 
   floatx4 acc[2][RT];
-  floatx4 sg[4][2][RT];                           // SiLU' of the layers
+  floatx4 sg[2][RT];                              // SiLU' of a layer
   auto clear = [&]() {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -329,14 +351,15 @@ __global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
       *(bf16x4*)(o + kPlane) = l;
     }
   };
-  // acc += LDS rows . W^T, W [unit][256] BF16
+  // acc = LDS rows . W^T, W [unit][256] BF16
   auto product = [&](const __bf16* __restrict__ W) {
+    clear();
 #pragma unroll
     for (int k0 = 0; k0 < kH; k0 += 32) {
       bf16x8 w[2];
 #pragma unroll
       for (int i = 0; i < 2; ++i)
-        w[i] = *(const bf16x8*)(W + (size_t)(ub + i * 16 + r16) * kH + k0 + kg);
+        w[i] = *(const bf16x8*)frag(W, ub + i * 16, k0, lane);
 #pragma unroll
       for (int j = 0; j < RT; ++j) {
         const bf16x8 hh = *(const bf16x8*)&Hh[j * 16 + r16][k0 + kg];
@@ -347,6 +370,22 @@ __global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hh, w[i], acc[i][j], 0, 0, 0);
         }
       }
+    }
+  };
+  // acc (z without its bias) to SiLU(z), 0 in rows past n, and sg
+  auto activate = [&](const float* __restrict__ bias) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const float b = bias[ub + i * 16 + r16];
+#pragma unroll
+      for (int j = 0; j < RT; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float z = acc[i][j][r] + b;
+          const float s = sigmoidf_(z);
+          sg[i][j][r] = s * (1.0f + z * (1.0f - s));
+          acc[i][j][r] = r0 + j * 16 + q4 + r < a.n ? z * s : 0.f;
+        }
     }
   };
   // column sums of v over the tile's rows (rows past n hold zeros)
@@ -380,7 +419,7 @@ __global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
   // input layer in FP32
   clear();
   {
-    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+    const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
     const float* x[RT];
 #pragma unroll
     for (int j = 0; j < RT; ++j) {
@@ -390,12 +429,12 @@ __global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       const int k = 16 * s + q4;
-      float4 xv[RT], wv[2];
+      floatx4 xv[RT], wv[2];
 #pragma unroll
-      for (int j = 0; j < RT; ++j) xv[j] = x[j] && k < kIn ? *(const float4*)(x[j] + k) : zero;
+      for (int j = 0; j < RT; ++j) xv[j] = x[j] && k < kIn ? *(const floatx4*)(x[j] + k) : zero;
 #pragma unroll
       for (int i = 0; i < 2; ++i)
-        wv[i] = k < kIn ? *(const float4*)(a.P + kOffW1 + (size_t)(ub + i * 16 + r16) * kIn + k)
+        wv[i] = k < kIn ? *(const floatx4*)(a.P + kOffW1 + (size_t)(ub + i * 16 + r16) * kIn + k)
                         : zero;
 #pragma unroll
       for (int e = 0; e < 4; ++e)
@@ -403,36 +442,28 @@ __global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
         for (int j = 0; j < RT; ++j)
 #pragma unroll
           for (int i = 0; i < 2; ++i)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(((const float*)&xv[j])[e],
-                                                             ((const float*)&wv[i])[e],
-                                                             acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[j][e], wv[i][e], acc[i][j],
+                                                             0, 0, 0);
     }
   }
-  constexpr int offb[4] = {kOffB1, kOffB2, kOffB3, kOffB4};
+  // layers 1-3: activations for the next layer; W2-W4 and their biases lie at
+  // one stride
+  static_assert(kOffB3 - kOffB2 == kOffB4 - kOffB3, "bias stride");
+#pragma unroll 1
+  for (int l = 0; l < 3; ++l) {
+    activate(a.P + (l == 0 ? kOffB1 : kOffB2 + (l - 1) * (kOffB3 - kOffB2)));
 #pragma unroll
-  for (int l = 0; l < 4; ++l) {
-    if (l > 0) {
-      clear();
-      product(a.Wb + (size_t)(l - 1) * kH * kH);
-      __syncthreads();                            // every wave has read this layer's input
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const float bias = a.P[offb[l] + ub + i * 16 + r16];
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int j = 0; j < RT; ++j) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float z = acc[i][j][r] + bias;
-          const float s = sigmoidf_(z);
-          sg[l][i][j][r] = s * (1.0f + z * (1.0f - s));
-          acc[i][j][r] = r0 + j * 16 + q4 + r < a.n ? z * s : 0.f;
-        }
-        if (l < 3) put(i, j, acc[i][j], act + kActH + 2 * l * kPlane, true);
+        slope[l][i * RT + j][t] = sg[i][j];
+        put(i, j, acc[i][j], act + kActH + 2 * l * kPlane, true);
       }
-    }
-    if (l < 3) __syncthreads();
+    lds_barrier();
+    product(a.Wb + (size_t)l * kH * kH);
+    lds_barrier();                                // every wave has read this layer's input
   }
+  activate(a.P + kOffB4);
   // head: y, dy = 2 (y - t) / n, the loss; dw5's partial sums
   float w5[2], dy[RT][4];
 #pragma unroll
@@ -446,7 +477,7 @@ __global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
       for (int off = 8; off > 0; off >>= 1) v += __shfl_xor(v, off);
       if (r16 == 0) head[wave][j * 16 + q4 + r] = v;
     }
-  __syncthreads();
+  lds_barrier();
   float loss = 0.f, sum_dy = 0.f;
 #pragma unroll
   for (int j = 0; j < RT; ++j)
@@ -481,12 +512,12 @@ __global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         acc[i][j][r] *= dy[j][r];
-        dz[i][j][r] = dy[j][r] * w5[i] * sg[3][i][j][r];
+        dz[i][j][r] = dy[j][r] * w5[i] * sg[i][j][r];
       }
     column_sum(i, acc, part + kPartW5);
   }
   // back through the layers; dZ1 feeds the weight gradient only
-#pragma unroll
+#pragma unroll 1
   for (int l = 3; l >= 0; --l) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -495,14 +526,13 @@ __global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
       column_sum(i, dz, part + l * kH);
     }
     if (l == 0) break;
-    __syncthreads();
-    clear();
+    lds_barrier();
     product(a.Wb + kWbT + (size_t)(l - 1) * kH * kH);
-    __syncthreads();                              // every wave has read dZ of this layer
+    lds_barrier();                                // every wave has read dZ of this layer
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int j = 0; j < RT; ++j) dz[i][j] = acc[i][j] * sg[l - 1][i][j];
+      for (int j = 0; j < RT; ++j) dz[i][j] = acc[i][j] * slope[l - 1][i * RT + j][t];
   }
 }
 
@@ -576,8 +606,8 @@ __device__ __forceinline__ void store_bf16_copy(int i, float p, __bf16* __restri
   else if (i >= kOffW3 && i < kOffB3) { l = 1; j = i - kOffW3; }
   else if (i >= kOffW4 && i < kOffB4) { l = 2; j = i - kOffW4; }
   if (l >= 0) {
-    Wb[(size_t)l * kH * kH + j] = (__bf16)p;
-    Wb[kWbT + (size_t)l * kH * kH + (size_t)(j % kH) * kH + j / kH] = (__bf16)p;
+    Wb[(size_t)l * kH * kH + frag_index(j / kH, j % kH)] = (__bf16)p;
+    Wb[kWbT + (size_t)l * kH * kH + frag_index(j % kH, j / kH)] = (__bf16)p;
   } else if (i >= kOffW1 && i < kOffB1) {
     const int u = (i - kOffW1) / kIn, k = (i - kOffW1) % kIn;
     const __bf16 h = (__bf16)p;
