@@ -2531,9 +2531,12 @@ static int ctx_create(const uint8_t* vol, const int64_t shape[3], const int64_t*
     const int rc = upload_voxel_order(c, blk[0], blk[1], blk[2]);
     if (rc) return rc;
     // a one-shot call builds the field where its steps (about a third of the
-    // extents' sum per pair) cost more than the field does
+    // extents' sum per pair) cost more than the field and its allocations do,
+    // some 1.3 ms: 150x201x187, 6.5e8 steps 1.6 ms per call without it and 2.4
+    // with it, 1.6e9 steps 3.0 and 2.7; 100^3, 2e8 steps 0.67 and 0.84; 256^3,
+    // 1.3e9 steps 4.0 and 2.4, 5.1e9 steps 14.2 and 3.9
     const double steps = (double)reflections * (double)n * (c->Z + c->Y + c->X) / 3.0;
-    if (reflections > 0 && steps < 1e9 + 300.0 * (double)nvox) return ANACOR_OK;
+    if (reflections > 0 && steps < 1e9 + 30.0 * (double)nvox) return ANACOR_OK;
     return field_build(c);
   };
   const int rc = init();
