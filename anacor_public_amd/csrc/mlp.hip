@@ -9,8 +9,8 @@
 // gradients stay FP32 and enter the MFMA as a BF16 hi + lo pair (two
 // products), so their rounding puts no input-dependent noise on the output;
 // weight gradients use hi/lo on both operands (three products).  In training
-// the 60 -> 256 input layer runs on the FP32 MFMA and the 256 -> 1 output
-// layer on FP32 VALU; inference runs the input layer on MFMA as hi/lo pairs of
+// the 60 -> 256 input layer and the 256 -> 1 output layer run on FP32 VALU;
+// inference runs the input layer on MFMA as hi/lo pairs of
 // both operands.  FP32 master weights, Adam.
 //
 // Parameter layout (FP32, ANACOR_MLP_PARAMS values):
@@ -240,8 +240,12 @@ __global__ __launch_bounds__(256) void mlp_infer_kernel(
 // gradients, split over the rows) and reduce_kernel (the slices' sums, the
 // bias gradients and the loss, with Adam in place).  Layer by layer, with
 // pre-activations, activations and dZ in FP32 through memory, it was 22
-// launches and 270 us at 4,096 rows (56 us now: 32, 16 and 8), 566 us at 16,384
-// (126 us: 74, 43 and 9).
+// launches and 270 us at 4,096 rows (66 us now: 38, 19 and 9), 566 us at 16,384
+// (162 us: 98, 57 and 7).  Every sum keeps the order it had there, so gradients
+// and trained parameters carry the same bits: a training run multiplies a
+// difference of one rounding a hundredfold in 400 steps.  (In the orders that
+// suit the tiles, the input layer on the FP32 MFMA, bias and output gradients
+// summed in the tiles: 32, 16 and 8 us, 74, 43 and 9.)
 //
 // Operands of the weight gradients, dW[out][in] = sum_b dZ[b][out] H[b][in],
 // leave the tile kernel as the MFMA reads them: BF16 hi and lo planes in blocks of
@@ -250,20 +254,20 @@ __global__ __launch_bounds__(256) void mlp_infer_kernel(
 
 constexpr int kRowBlock = 32;
 constexpr int kSplitMax = 32;             // K slices of the weight gradients
-// Planes of a 32-row block, in elements: the inputs (64 wide) hi and lo, H1-H3
-// hi and lo, dZ1-dZ4 hi and lo.
+// Planes of a 32-row block, in elements: the inputs (64 wide) hi and lo, H1-H4
+// hi and lo, dZ1-dZ4 hi and lo, dy hi and lo.
 constexpr size_t kPlane = (size_t)kH * kRowBlock;
 constexpr size_t kPlaneX = (size_t)kInK * kRowBlock;
-constexpr size_t kActH = 2 * kPlaneX;                 // H(l), l = 0..2: + 2 l kPlane
-constexpr size_t kActD = kActH + 6 * kPlane;          // dZ(l), l = 0..3: + 2 l kPlane
-constexpr size_t kActBlock = kActD + 8 * kPlane;
-// Per-tile partials: column sums of dZ1-dZ4 [4][256], dw5 [256], loss, dy.
-constexpr int kPartW5 = 4 * kH;
-constexpr int kPartLoss = kPartW5 + kH;
-constexpr int kPart = kPartLoss + 2;
-// A slice of weight gradients: W1 [256][64], then W2, W3, W4 [256][256].
+constexpr size_t kActH = 2 * kPlaneX;                 // H(l), l = 0..3: + 2 l kPlane
+constexpr size_t kActD = kActH + 8 * kPlane;          // dZ(l), l = 0..3: + 2 l kPlane
+constexpr size_t kActY = kActD + 8 * kPlane;
+constexpr size_t kActBlock = kActY + 2 * kRowBlock;
+constexpr size_t kDzBlock = 4 * kPlane;               // dZ1-dZ4 in FP32, for the biases
+// A slice of gradients: W1 [256][64], W2, W3, W4 [256][256], b1-b4, w5.
 constexpr size_t kWsW2 = (size_t)kH * kInK;
-constexpr size_t kWsStride = kWsW2 + 3 * (size_t)kH * kH;
+constexpr size_t kWsB = kWsW2 + 3 * (size_t)kH * kH;
+constexpr size_t kWsW5 = kWsB + 4 * kH;
+constexpr size_t kWsStride = kWsW5 + kH;
 
 struct TrainArgs {
   const float* X;         // rows [kIn], of X[perm[b]] with perm
@@ -273,7 +277,8 @@ struct TrainArgs {
   const float* P;
   const __bf16* Wb;
   __bf16* act;            // [blocks of 32 rows][kActBlock]
-  float* part;            // [tiles][kPart]
+  float* dz;              // [blocks of 32 rows][kDzBlock]
+  float* part;            // [groups of 4 rows][2]: loss, dy
 };
 
 __device__ __forceinline__ void split_bf16(float v, __bf16& hi, __bf16& lo) {
@@ -293,30 +298,31 @@ __device__ __forceinline__ void lds_barrier() {
 // operand plane and, forward and backward, the same (row, unit) pairs of every
 // layer, so SiLU' waits in LDS at the thread's own place.  Activations and dZ
 // pass between layers in LDS as hi/lo [row][unit]; weights come from L2 as
-// 16-byte fragments.  The input layer runs on the FP32 MFMA (k in the order 16
-// s + 4 (l / 16) + e, the same for both operands).
+// 16-byte fragments.  The input layer runs on FP32 VALU.
 //
-// What bounds it: the weights' 0.86 MB per workgroup out of L2 (32 us for 256
-// workgroups of 16 rows, 74 us for 512 of 32: 7 and 6 TB/s), in rounds between two
-// barriers per layer.  SiLU' in registers and the layers unrolled: 43 us at the
-// fragments of then (41 rolled); fetching a layer's fragments ahead of its barrier
+// What bounds it: the weights' 0.86 MB per workgroup out of L2, in rounds between
+// two barriers per layer (38 us for 256 workgroups of 16 rows, 98 us for 512 of
+// 32, some 6 and 24 us of it the input layer's chains).  SiLU' in registers and
+// the layers unrolled, or a layer's fragments fetched ahead of its barrier,
 // changed nothing.  Rows per workgroup: the weights ask for more rows, a batch of
 // 4,096 for enough workgroups.
 template <int ROWS>
 __global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
   constexpr int RT = ROWS / 16;
   static_assert(ROWS == 16 || ROWS == 32, "row tile");
-  __shared__ __attribute__((aligned(16))) __bf16 Hh[ROWS][kHP];
-  __shared__ __attribute__((aligned(16))) __bf16 Hl[ROWS][kHP];
+  __shared__ __attribute__((aligned(16))) __bf16 hilo[2][ROWS][kHP];
+  __bf16 (*const Hh)[kHP] = hilo[0];
+  __bf16 (*const Hl)[kHP] = hilo[1];
+  float (*const h4)[kHP] = (float(*)[kHP])hilo;   // H4 in FP32, between two layers
   __shared__ floatx4 slope[3][2 * RT][512];       // SiLU' of layers 1-3, by thread
-  __shared__ float head[8][ROWS];
+  __shared__ float loss[ROWS], dys[ROWS];
   const int t = (int)threadIdx.x, lane = t & 63, wave = t >> 6;
   const int r16 = lane & 15, quad = lane >> 4, kg = quad * 8, q4 = quad * 4;
   const int ub = wave * 32;
   const int r0 = (int)blockIdx.x * ROWS;
   __bf16* const act = a.act + (size_t)(r0 / kRowBlock) * kActBlock;
   const int rb = r0 % kRowBlock;                  // this tile's first row in its block
-  float* const part = a.part + (size_t)blockIdx.x * kPart;
+  float* const dzs = a.dz + (size_t)(r0 / kRowBlock) * kDzBlock;
 
   floatx4 acc[2][RT];
   floatx4 sg[2][RT];                              // SiLU' of a layer
@@ -372,11 +378,11 @@ __global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
       }
     }
   };
-  // acc (z without its bias) to SiLU(z), 0 in rows past n, and sg
+  // acc (z, or without its bias) to SiLU(z), 0 in rows past n, and sg
   auto activate = [&](const float* __restrict__ bias) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      const float b = bias[ub + i * 16 + r16];
+      const float b = bias ? bias[ub + i * 16 + r16] : 0.f;
 #pragma unroll
       for (int j = 0; j < RT; ++j)
 #pragma unroll
@@ -388,16 +394,6 @@ __global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
         }
     }
   };
-  // column sums of v over the tile's rows (rows past n hold zeros)
-  auto column_sum = [&](int i, const floatx4 (&v)[2][RT], float* out) {
-    float s = 0.f;
-#pragma unroll
-    for (int j = 0; j < RT; ++j) s += (v[i][j][0] + v[i][j][1]) + (v[i][j][2] + v[i][j][3]);
-    s += __shfl_xor(s, 16);
-    s += __shfl_xor(s, 32);
-    if (quad == 0) out[ub + i * 16 + r16] = s;
-  };
-
   // inputs as operand planes: 8 rows of one column per thread
   for (int q = t; q < kInK * (ROWS / 8); q += 512) {
     const int k = q % kInK, rg = q / kInK * 8;
@@ -416,34 +412,39 @@ __global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
     *(bf16x8*)o = h;
     *(bf16x8*)(o + kPlaneX) = l;
   }
-  // input layer in FP32
-  clear();
+  // input layer in FP32, one chain of multiply-adds per (row, unit)
   {
-    const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
-    const float* x[RT];
+    const float* x[RT][4];
 #pragma unroll
-    for (int j = 0; j < RT; ++j) {
-      const int row = r0 + j * 16 + r16;
-      x[j] = row < a.n ? a.X + (size_t)(a.perm ? a.perm[row] : row) * kIn : nullptr;
+    for (int j = 0; j < RT; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {     // rows past n: any row's, and zero below
+        const int row = min(r0 + j * 16 + q4 + r, a.n - 1);
+        x[j][r] = a.X + (size_t)(a.perm ? a.perm[row] : row) * kIn;
+      }
+    const float* const w = a.P + kOffW1 + (size_t)(ub + r16) * kIn;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const float bias = a.P[kOffB1 + ub + i * 16 + r16];
+#pragma unroll
+      for (int j = 0; j < RT; ++j) acc[i][j] = floatx4{bias, bias, bias, bias};
     }
+#pragma unroll 3
+    for (int k = 0; k < kIn; k += 4) {
+      floatx4 wv[2];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const int k = 16 * s + q4;
-      floatx4 xv[RT], wv[2];
+      for (int i = 0; i < 2; ++i) wv[i] = *(const floatx4*)(w + i * 16 * kIn + k);
 #pragma unroll
-      for (int j = 0; j < RT; ++j) xv[j] = x[j] && k < kIn ? *(const floatx4*)(x[j] + k) : zero;
+      for (int j = 0; j < RT; ++j)
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
-        wv[i] = k < kIn ? *(const floatx4*)(a.P + kOffW1 + (size_t)(ub + i * 16 + r16) * kIn + k)
-                        : zero;
+        for (int r = 0; r < 4; ++r) {
+          const floatx4 xv = *(const floatx4*)(x[j][r] + k);
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
+          for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int j = 0; j < RT; ++j)
-#pragma unroll
-          for (int i = 0; i < 2; ++i)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[j][e], wv[i][e], acc[i][j],
-                                                             0, 0, 0);
+            for (int i = 0; i < 2; ++i)
+              acc[i][j][r] = fmaf(xv[e], wv[i][e], acc[i][j][r]);
+        }
     }
   }
   // layers 1-3: activations for the next layer; W2-W4 and their biases lie at
@@ -451,7 +452,7 @@ __global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
   static_assert(kOffB3 - kOffB2 == kOffB4 - kOffB3, "bias stride");
 #pragma unroll 1
   for (int l = 0; l < 3; ++l) {
-    activate(a.P + (l == 0 ? kOffB1 : kOffB2 + (l - 1) * (kOffB3 - kOffB2)));
+    activate(l == 0 ? nullptr : a.P + kOffB2 + (l - 1) * (kOffB3 - kOffB2));
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -464,67 +465,65 @@ __global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
     lds_barrier();                                // every wave has read this layer's input
   }
   activate(a.P + kOffB4);
-  // head: y, dy = 2 (y - t) / n, the loss; dw5's partial sums
-  float w5[2], dy[RT][4];
+  // head, a wave per row: y, dy = 2 (y - t) / n, the loss
 #pragma unroll
-  for (int i = 0; i < 2; ++i) w5[i] = a.P[kOffW5 + ub + i * 16 + r16];
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-  for (int j = 0; j < RT; ++j)
+    for (int j = 0; j < RT; ++j) {
+      put(i, j, acc[i][j], act + kActH + 6 * kPlane, false);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float v = fmaf(acc[0][j][r], w5[0], acc[1][j][r] * w5[1]);
-#pragma unroll
-      for (int off = 8; off > 0; off >>= 1) v += __shfl_xor(v, off);
-      if (r16 == 0) head[wave][j * 16 + q4 + r] = v;
+      for (int r = 0; r < 4; ++r) h4[j * 16 + q4 + r][ub + i * 16 + r16] = acc[i][j][r];
     }
   lds_barrier();
-  float loss = 0.f, sum_dy = 0.f;
+  for (int row = wave; row < ROWS; row += 8) {
+    float y = 0.f;
 #pragma unroll
-  for (int j = 0; j < RT; ++j)
+    for (int k = lane; k < kH; k += 64) y = fmaf(h4[row][k], a.P[kOffW5 + k], y);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = j * 16 + q4 + r;
-      float y = 0.f;
-#pragma unroll
-      for (int w = 0; w < 8; ++w) y += head[w][row];
-      dy[j][r] = 0.f;
+    for (int off = 32; off > 0; off >>= 1) y += __shfl_xor(y, off);
+    if (lane == 0) {
+      float l = 0.f, g = 0.f;
       if (r0 + row < a.n) {
-        const int src = a.perm ? a.perm[r0 + row] : r0 + row;
-        const float d = (y + a.P[kOffB5]) - a.T[src];
-        dy[j][r] = 2.f * d / (float)a.n;
-        loss += d * d / (float)a.n;
+        const float d = (y + a.P[kOffB5]) - a.T[a.perm ? a.perm[r0 + row] : r0 + row];
+        g = 2.f * d / (float)a.n;
+        l = d * d / (float)a.n;
       }
-      sum_dy += dy[j][r];
+      loss[row] = l;
+      dys[row] = g;
     }
-  loss += __shfl_xor(loss, 16);
-  loss += __shfl_xor(loss, 32);
-  sum_dy += __shfl_xor(sum_dy, 16);
-  sum_dy += __shfl_xor(sum_dy, 32);
-  if (t == 0) {
-    part[kPartLoss] = loss;
-    part[kPartLoss + 1] = sum_dy;
+  }
+  lds_barrier();
+  if (t < ROWS / 4) {
+    float* const o = a.part + 2 * ((size_t)r0 / 4 + t);
+    o[0] = (loss[4 * t] + loss[4 * t + 1]) + (loss[4 * t + 2] + loss[4 * t + 3]);
+    o[1] = (dys[4 * t] + dys[4 * t + 1]) + (dys[4 * t + 2] + dys[4 * t + 3]);
+  }
+  if (t < ROWS) {
+    __bf16 h, l;
+    split_bf16(dys[t], h, l);
+    act[kActY + rb + t] = h;
+    act[kActY + kRowBlock + rb + t] = l;
   }
   floatx4 dz[2][RT];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
+    const float w5 = a.P[kOffW5 + ub + i * 16 + r16];
 #pragma unroll
     for (int j = 0; j < RT; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        acc[i][j][r] *= dy[j][r];
-        dz[i][j][r] = dy[j][r] * w5[i] * sg[i][j][r];
-      }
-    column_sum(i, acc, part + kPartW5);
+      for (int r = 0; r < 4; ++r) dz[i][j][r] = dys[j * 16 + q4 + r] * w5 * sg[i][j][r];
   }
   // back through the layers; dZ1 feeds the weight gradient only
 #pragma unroll 1
   for (int l = 3; l >= 0; --l) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int j = 0; j < RT; ++j) put(i, j, dz[i][j], act + kActD + 2 * l * kPlane, l > 0);
-      column_sum(i, dz, part + l * kH);
-    }
+      for (int j = 0; j < RT; ++j) {
+        put(i, j, dz[i][j], act + kActD + 2 * l * kPlane, l > 0);
+        *(floatx4*)(dzs + l * kPlane + (size_t)(ub + i * 16 + r16) * kRowBlock + rb + j * 16 +
+                    q4) = dz[i][j];
+      }
     if (l == 0) break;
     lds_barrier();
     product(a.Wb + kWbT + (size_t)(l - 1) * kH * kH);
@@ -536,12 +535,15 @@ __global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
   }
 }
 
-// One slice of the weight gradients: 13 workgroups per slice, 4 waves of 64 x 64
-// outputs each; W1 [256][64] is one workgroup, W2, W3, W4 four quarters each.
+// One slice of the gradients: 18 workgroups per slice. 13 are 4 waves of 64 x 64
+// outputs each; W1 [256][64] is one of them, W2, W3, W4 four quarters each. One
+// takes w5 (dw5 = H4^T dy, a wave 64 units), four the biases: a thread per unit
+// sums dZ in FP32, first each of the 32 rows over the slice's blocks, then those.
 // Fragments come straight from the operand planes (1 KB per wave and load).
 // hi/lo on both operands, three products.
 struct WeightGradArgs {
   const __bf16* act;
+  const float* dz;
   int blocks;             // 32-row blocks
   int per_slice;          // blocks per slice
   float* ws;              // [slices][kWsStride]
@@ -550,7 +552,54 @@ struct WeightGradArgs {
 __global__ __launch_bounds__(256) void weight_grad_kernel(WeightGradArgs g) {
   const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
   const int r16 = lane & 15, kg = (lane >> 4) * 8, q4 = (lane >> 4) * 4;
-  const int job = (int)blockIdx.x;                // 0: W1, else quarter (job - 1) % 4 of a layer
+  const int job = (int)blockIdx.x;                // 0: W1, to 12: quarter (job - 1) % 4 of a layer
+  const int b0 = (int)blockIdx.y * g.per_slice, b1 = min(g.blocks, b0 + g.per_slice);
+  float* const ws = g.ws + (size_t)blockIdx.y * kWsStride;
+  if (job >= 14) {
+    const int layer = job - 14, unit = (int)threadIdx.x;
+    floatx4 s[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) s[q] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int b = b0; b < b1; ++b) {
+      const float* d = g.dz + (size_t)b * kDzBlock + layer * kPlane + (size_t)unit * kRowBlock;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) s[q] += *(const floatx4*)(d + 4 * q);
+    }
+    float sum = 0.f;
+#pragma unroll
+    for (int q = 0; q < 32; ++q) sum += s[q >> 2][q & 3];
+    ws[kWsB + layer * kH + unit] = sum;
+    return;
+  }
+  if (job == 13) {
+    floatx4 acc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int b = b0; b < b1; ++b) {
+      const __bf16* blk = g.act + (size_t)b * kActBlock;
+      bf16x8 yh = {}, yl = {};
+      if (r16 == 0) {                               // the one column
+        yh = *(const bf16x8*)(blk + kActY + kg);
+        yl = *(const bf16x8*)(blk + kActY + kRowBlock + kg);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const __bf16* h = blk + kActH + 6 * kPlane +
+                          (size_t)(wave * 64 + i * 16 + r16) * kRowBlock + kg;
+        const bf16x8 ah = *(const bf16x8*)h, al = *(const bf16x8*)(h + kPlane);
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, yh, acc[i], 0, 0, 0);
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, yl, acc[i], 0, 0, 0);
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, yh, acc[i], 0, 0, 0);
+      }
+    }
+    if (r16 == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) ws[kWsW5 + wave * 64 + i * 16 + q4 + r] = acc[i][r];
+    }
+    return;
+  }
   const bool first = job == 0;
   const int layer = first ? 0 : (job - 1) / 4 + 1, quarter = (job - 1) & 3;
   const int m0 = first ? wave * 64 : (quarter >> 1) * 128 + (wave >> 1) * 64;
@@ -564,7 +613,6 @@ __global__ __launch_bounds__(256) void weight_grad_kernel(WeightGradArgs g) {
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const int b0 = (int)blockIdx.y * g.per_slice, b1 = min(g.blocks, b0 + g.per_slice);
 #pragma unroll 2
   for (int b = b0; b < b1; ++b) {
     const __bf16* blk = g.act + (size_t)b * kActBlock;
@@ -586,8 +634,7 @@ __global__ __launch_bounds__(256) void weight_grad_kernel(WeightGradArgs g) {
       }
   }
   const int ldo = first ? kInK : kH;
-  float* out = g.ws + (size_t)blockIdx.y * kWsStride +
-               (first ? 0 : kWsW2 + (size_t)(layer - 1) * kH * kH);
+  float* out = ws + (first ? 0 : kWsW2 + (size_t)(layer - 1) * kH * kH);
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -617,14 +664,13 @@ __device__ __forceinline__ void store_bf16_copy(int i, float p, __bf16* __restri
 }
 
 // The gradients' sums in fixed order into G, the batch loss added to loss[0],
-// and with `adam` the update of every parameter, its BF16 copies too.  The
-// first blocks take the weights (one per thread, its slices), the last ones
-// the bias and head partials of the tiles: 64 columns and 4 rows of threads.
+// and with `adam` the update of every parameter, its BF16 copies too.  One
+// parameter per thread, its slices; the last block takes b5 and the loss.
 struct ReduceArgs {
   const float* ws;
   int slices;
   const float* part;
-  int tiles;
+  int groups;             // of 4 rows
   float* G;
   float* loss;
   bool adam;
@@ -632,10 +678,8 @@ struct ReduceArgs {
   __bf16* Wb;
   float lr, b1, b2, eps, c1, c2;
 };
-constexpr int kWeightFloats = kH * kIn + 3 * kH * kH;
-constexpr int kWeightBlocks = kWeightFloats / 256;
-static_assert(kWeightFloats % 256 == 0, "whole blocks of weights");
-constexpr int kPartBlocks = (kPart + 63) / 64;
+constexpr int kReduceBlocks = (kParams - 1) / 256;
+static_assert((kParams - 1) % 256 == 0 && kOffB5 == kParams - 1, "whole blocks, b5 last");
 
 __device__ __forceinline__ void take_gradient(const ReduceArgs& a, int i, float g) {
   a.G[i] = g;
@@ -651,46 +695,38 @@ __device__ __forceinline__ void take_gradient(const ReduceArgs& a, int i, float 
 
 __global__ __launch_bounds__(256) void reduce_kernel(ReduceArgs a) {
   const int t = (int)threadIdx.x;
-  if ((int)blockIdx.x < kWeightBlocks) {
+  if ((int)blockIdx.x < kReduceBlocks) {
     const int i = (int)blockIdx.x * 256 + t;
-    int param, at;
-    if (i < kH * kIn) {
-      param = kOffW1 + i;
-      at = i / kIn * kInK + i % kIn;
-    } else {
-      const int l = (i - kH * kIn) / (kH * kH), e = (i - kH * kIn) % (kH * kH);
-      param = (l == 0 ? kOffW2 : l == 1 ? kOffW3 : kOffW4) + e;
-      at = (int)kWsW2 + l * kH * kH + e;
+    int at;
+    if (i < kOffB1) at = i / kIn * kInK + i % kIn;
+    else if (i < kOffW2) at = (int)kWsB + i - kOffB1;
+    else if (i >= kOffW5) at = (int)kWsW5 + i - kOffW5;
+    else {
+      const int l = (i - kOffW2) / (kOffW3 - kOffW2), e = (i - kOffW2) % (kOffW3 - kOffW2);
+      at = e < kH * kH ? (int)kWsW2 + l * kH * kH + e : (int)kWsB + (l + 1) * kH + e - kH * kH;
     }
     float g = 0.f;
 #pragma unroll 8
     for (int z = 0; z < a.slices; ++z) g += a.ws[(size_t)z * kWsStride + at];
-    take_gradient(a, param, g);
+    take_gradient(a, i, g);
     return;
   }
-  __shared__ float rows[4][64];
-  const int col = ((int)blockIdx.x - kWeightBlocks) * 64 + (t & 63);
-  float s = 0.f;
-  if (col < kPart) {
+  if (t >= 64) return;
+  float l = 0.f, g = 0.f;
 #pragma unroll 8
-    for (int w = t >> 6; w < a.tiles; w += 4) s += a.part[(size_t)w * kPart + col];
+  for (int i = t; i < a.groups; i += 64) {
+    l += a.part[2 * i];
+    g += a.part[2 * i + 1];
   }
-  rows[t >> 6][t & 63] = s;
-  __syncthreads();
-  if (t >= 64 || col >= kPart) return;
-  const float g = (rows[0][t] + rows[1][t]) + (rows[2][t] + rows[3][t]);
-  if (col == kPartLoss) {
-    a.loss[0] += g;
-    return;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    l += __shfl_xor(l, off);
+    g += __shfl_xor(g, off);
   }
-  int param = kOffB5;
-  if (col < kPartW5) {
-    const int l = col / kH;
-    param = (l == 0 ? kOffB1 : l == 1 ? kOffB2 : l == 2 ? kOffB3 : kOffB4) + col % kH;
-  } else if (col < kPartLoss) {
-    param = kOffW5 + col - kPartW5;
+  if (t == 0) {
+    a.loss[0] += l;
+    take_gradient(a, kOffB5, g);
   }
-  take_gradient(a, param, g);
 }
 
 __global__ void weights_to_bf16(const float* __restrict__ P, __bf16* __restrict__ Wb) {
@@ -1028,7 +1064,8 @@ struct Model {
   int cap = 0;                    // rows of the activation buffers
   DevBuf<__bf16> act;             // training operands (TrainArgs)
   DevBuf<float> xb, tb, loss;
-  DevBuf<float> part;             // per training tile: bias and head partials (kPart floats)
+  DevBuf<float> dz;               // dZ1-dZ4 in FP32 (TrainArgs)
+  DevBuf<float> part;             // per 4 rows: loss and dy
   DevBuf<float> ws;               // weight-gradient slices [kSplitMax][kWsStride]
   // feature / inference / training-set buffers (grown on demand)
   DevBuf<double> s1, omega, inv, A;
@@ -1081,7 +1118,8 @@ static int ensure_rows(Model* M, int n) {
   MLP_CHECK(M->act.grow(blocks * kActBlock));
   MLP_CHECK(M->xb.grow((size_t)n * kIn));
   MLP_CHECK(M->tb.grow((size_t)n));
-  MLP_CHECK(M->part.grow(blocks * (kRowBlock / 16) * kPart));   // tiles of either size
+  MLP_CHECK(M->dz.grow(blocks * kDzBlock));
+  MLP_CHECK(M->part.grow(blocks * (kRowBlock / 4) * 2));
   MLP_CHECK(M->ws.grow((size_t)kSplitMax * kWsStride));
   M->cap = n;
   return ANACOR_OK;
@@ -1112,21 +1150,23 @@ static void train_step(Model* M, const float* X, const int* perm, const float* T
   hipStream_t s = M->stream;
   const int rows = train_rows(n);
   const unsigned tiles = (unsigned)train_tiles(n);
-  TrainArgs a{X, perm, T, n, M->P.p, M->Wb.p, M->act.p, M->part.p};
+  TrainArgs a{X, perm, T, n, M->P.p, M->Wb.p, M->act.p, M->dz.p, M->part.p};
   if (rows == 16)
     hipLaunchKernelGGL(train_tile_kernel<16>, dim3(tiles), dim3(512), 0, s, a);
   else
     hipLaunchKernelGGL(train_tile_kernel<32>, dim3(tiles), dim3(512), 0, s, a);
-  WeightGradArgs w{M->act.p, (int)nblocks(n, kRowBlock), 0, M->ws.p};
-  w.per_slice = (w.blocks + kSplitMax - 1) / kSplitMax;
+  WeightGradArgs w{M->act.p, M->dz.p, (int)nblocks(n, kRowBlock), 0, M->ws.p};
+  // slices of at least 64 rows
+  const int most = std::max(1, std::min(kSplitMax, (n + 63) / 64));
+  w.per_slice = (int)nblocks((n + most - 1) / most, kRowBlock);
   const int slices = (w.blocks + w.per_slice - 1) / w.per_slice;
-  hipLaunchKernelGGL(weight_grad_kernel, dim3(13, (unsigned)slices), dim3(256), 0, s, w);
+  hipLaunchKernelGGL(weight_grad_kernel, dim3(18, (unsigned)slices), dim3(256), 0, s, w);
   const double b1 = 0.9, b2 = 0.999;
   ReduceArgs r{};
   r.ws = M->ws.p;
   r.slices = slices;
   r.part = M->part.p;
-  r.tiles = (int)tiles;
+  r.groups = (int)nblocks(n, 4);
   r.G = M->G.p;
   r.loss = M->loss.p;
   r.adam = lr != nullptr;
@@ -1143,7 +1183,7 @@ static void train_step(Model* M, const float* X, const int* perm, const float* T
     r.c1 = (float)(1.0 - std::pow(b1, (double)M->adam_t));
     r.c2 = (float)(1.0 - std::pow(b2, (double)M->adam_t));
   }
-  hipLaunchKernelGGL(reduce_kernel, dim3(kWeightBlocks + kPartBlocks), dim3(256), 0, s, r);
+  hipLaunchKernelGGL(reduce_kernel, dim3(kReduceBlocks + 1), dim3(256), 0, s, r);
 }
 
 // The goniometer of a call and the model's envelope (if set) for the
@@ -1317,7 +1357,7 @@ void anacor_mlp_destroy(anacor_mlp* mlp) {
     if (M->stream) (void)hipStreamSynchronize(M->stream);
     M->P.release(); M->G.release(); M->m.release(); M->v.release(); M->Wb.release();
     M->act.release(); M->xb.release(); M->tb.release();
-    M->part.release(); M->loss.release(); M->ws.release();
+    M->dz.release(); M->part.release(); M->loss.release(); M->ws.release();
     M->s1.release(); M->omega.release(); M->inv.release(); M->A.release();
     M->X.release(); M->y.release(); M->T.release(); M->flag.release(); M->trust.release();
     M->cell.release();
