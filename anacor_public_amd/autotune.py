@@ -7,8 +7,8 @@ Three knobs change speed but never a path length:
   wave's 64 parallel rays touch per step;
 * the tile size (voxels per workgroup), which trades partial sums and
   scheduling granularity against load balance;
-* the volume layout (raw uint8 or 8x8x8 bricks of 2-/4-bit labels) of a
-  single-sample tracer (the batched kernel reads the raw layout).
+* the volume layout (the library's choice, raw uint8 or 8x8x8 bricks of
+  2-/4-bit labels) of a single-sample tracer (a batch's samples keep theirs).
 
 ``tune(tracer, ...)`` times every candidate on a slice of the sample's own
 reflections with the trace kernel's HIP-event duration and keeps the fastest.
@@ -27,7 +27,9 @@ import numpy as np
 BLOCKS: Tuple[Tuple[int, int, int], ...] = ((1, 2, 64), (1, 1, 128), (2, 2, 32), (1, 4, 32),
                                              (2, 4, 16), (0, 0, 0))
 TILES: Tuple[int, ...] = (0, 512, 2048)       # 0 = the library's automatic choice (1,024 max)
-LAYOUTS: Tuple[int, ...] = (0, 1)             # raw, bricks (_lib.LAYOUT_RAW, _lib.LAYOUT_BRICK)
+# The library's automatic choice, which walks by free distances where it can; the stepping
+# kernel on the raw volume and on bricks (_lib.LAYOUT_AUTO, LAYOUT_RAW, LAYOUT_BRICK).
+LAYOUTS: Tuple[int, ...] = (-1, 0, 1)
 
 _lock = threading.Lock()
 

@@ -498,7 +498,7 @@ def measure_plain(config: str, steps: int, warmup: int, cpu_budget: float,
     every reflection's A_h.  Returns the record (value in A_h/s, roofline of
     the trace kernel, CPU baseline on a bounded sample of the same
     workload)."""
-    from anacor_public_amd import autotune
+    from anacor_public_amd import _lib, autotune
     from anacor_public_amd import workload as W
     from anacor_public_amd.ray_tracing import Batch, Tracer
     t0 = time.perf_counter()
@@ -515,6 +515,9 @@ def measure_plain(config: str, steps: int, warmup: int, cpu_budget: float,
     log(f"# workload {name}: volumes {[w.volume.shape for w in wls]}, N={N}, R={R} "
         f"(built in {time.perf_counter() - t0:.1f}s)")
     extra = {}
+    # the automatic layout walks by free distances (skip_kernel), for which no
+    # traffic per voxel step is on record
+    skip = "ANACOR_VOLUME_LAYOUT" not in os.environ
     if config == "batched":
         runner = Batch(wls)
         if autotune_on:
@@ -537,6 +540,7 @@ def measure_plain(config: str, steps: int, warmup: int, cpu_budget: float,
                                  trial=512, layouts=autotune.LAYOUTS, use_cache=False)
             extra["autotune"] = {"layout": pick["layout"], "block": pick["block"],
                                  "tile": pick["tile"]}
+            skip = skip and pick["layout"] == _lib.LAYOUT_AUTO
             log(f"# autotune ({time.perf_counter() - t1:.1f}s): {extra['autotune']}")
 
         def call():
@@ -580,8 +584,9 @@ def measure_plain(config: str, steps: int, warmup: int, cpu_budget: float,
     if config != "batched":
         shape = runner.work_shape()
         key_name = name if not reflections else f"{name}-first{reflections}"
-        traffic = traffic_for(key_name, layout, shape["block"], shape["tile"], shape["group"],
-                              vsteps)
+        if not skip:
+            traffic = traffic_for(key_name, layout, shape["block"], shape["tile"],
+                                  shape["group"], vsteps)
         extra["work_shape"] = shape
     pairs = sum(len(w.coords) * len(w.omega) for w in wls)
     rec = {
@@ -599,8 +604,8 @@ def measure_plain(config: str, steps: int, warmup: int, cpu_budget: float,
         "voxel_steps_per_s": vsteps / (ms_per_step * 1e-3),
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                     "kernel": ("trace_kernel, one launch per sample" if config == "batched"
-                                else "trace_kernel"),
+                     "kernel": ("skip_kernel" if skip else "trace_kernel") +
+                               (", one launch per sample" if config == "batched" else ""),
                      "kernel_ms": k_ms, "bytes_per_launch": vsteps},
         "cpu_baseline": cpu,
         "speedup_vs_cpu": (value / cpu["value"]) if cpu else None,
@@ -646,12 +651,12 @@ def profile_shapes() -> None:
     of the 256^3 workload in a fixed order, printing one JSON line per launch
     so that the per-dispatch counters of a rocprofv3 --pmc run can be matched
     to work shapes (the figures of TRAFFIC_BYTES_PER_STEP)."""
-    from anacor_public_amd import autotune
+    from anacor_public_amd import _lib, autotune
     from anacor_public_amd import workload as W
     from anacor_public_amd.ray_tracing import Tracer
     wl = W.single_gpu_config()
     with Tracer.for_workload(wl) as t:
-        for lay in autotune.LAYOUTS:
+        for lay in (_lib.LAYOUT_RAW, _lib.LAYOUT_BRICK):
             t.set_layout(lay)
             for blk in autotune.BLOCKS:
                 t.set_voxel_block(*blk)
