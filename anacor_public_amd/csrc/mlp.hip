@@ -240,8 +240,8 @@ __global__ __launch_bounds__(256) void mlp_infer_kernel(
 // gradients, split over the rows) and reduce_kernel (the slices' sums, the
 // bias gradients and the loss, with Adam in place).  Layer by layer, with
 // pre-activations, activations and dZ in FP32 through memory, it was 22
-// launches and 270 us at 4,096 rows (66 us now: 38, 19 and 9), 566 us at 16,384
-// (162 us: 98, 57 and 7).  Every sum keeps the order it had there, so gradients
+// launches and 270 us at 4,096 rows (64 us now: 36, 19 and 9), 566 us at 16,384
+// (147 us: 84, 56 and 7).  Every sum keeps the order it had there, so gradients
 // and trained parameters carry the same bits: a training run multiplies a
 // difference of one rounding a hundredfold in 400 steps.  (In the orders that
 // suit the tiles, the input layer on the FP32 MFMA, bias and output gradients
@@ -262,7 +262,7 @@ constexpr size_t kActH = 2 * kPlaneX;                 // H(l), l = 0..3: + 2 l k
 constexpr size_t kActD = kActH + 8 * kPlane;          // dZ(l), l = 0..3: + 2 l kPlane
 constexpr size_t kActY = kActD + 8 * kPlane;
 constexpr size_t kActBlock = kActY + 2 * kRowBlock;
-constexpr size_t kDzBlock = 4 * kPlane;               // dZ1-dZ4 in FP32, for the biases
+constexpr size_t kDzBlock = 4 * kPlane;               // dZ1-dZ4 [32][256] in FP32, for the biases
 // A slice of gradients: W1 [256][64], W2, W3, W4 [256][256], b1-b4, w5.
 constexpr size_t kWsW2 = (size_t)kH * kInK;
 constexpr size_t kWsB = kWsW2 + 3 * (size_t)kH * kH;
@@ -301,8 +301,9 @@ __device__ __forceinline__ void lds_barrier() {
 // 16-byte fragments.  The input layer runs on FP32 VALU.
 //
 // What bounds it: the weights' 0.86 MB per workgroup out of L2, in rounds between
-// two barriers per layer (38 us for 256 workgroups of 16 rows, 98 us for 512 of
-// 32, some 6 and 24 us of it the input layer's chains).  SiLU' in registers and
+// two barriers per layer (36 us for 256 workgroups of 16 rows, 84 us for 512 of
+// 32, some 4 and 10 us of it the input layer's chains; with the inputs out of L1
+// rather than staged in LDS 38 and 98).  SiLU' in registers and
 // the layers unrolled, or a layer's fragments fetched ahead of its barrier,
 // changed nothing.  Rows per workgroup: the weights ask for more rows, a batch of
 // 4,096 for enough workgroups.
@@ -315,6 +316,7 @@ __global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
   __bf16 (*const Hl)[kHP] = hilo[1];
   float (*const h4)[kHP] = (float(*)[kHP])hilo;   // H4 in FP32, between two layers
   __shared__ floatx4 slope[3][2 * RT][512];       // SiLU' of layers 1-3, by thread
+  __shared__ __attribute__((aligned(16))) float xs[ROWS][kInK + 4];   // inputs, zero past kIn
   __shared__ float loss[ROWS], dys[ROWS];
   const int t = (int)threadIdx.x, lane = t & 63, wave = t >> 6;
   const int r16 = lane & 15, quad = lane >> 4, kg = quad * 8, q4 = quad * 4;
@@ -394,17 +396,20 @@ __global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
         }
     }
   };
+  for (int q = t; q < ROWS * kInK; q += 512) {
+    const int row = r0 + q / kInK, k = q % kInK;
+    xs[q / kInK][k] = k < kIn && row < a.n
+                          ? a.X[(size_t)(a.perm ? a.perm[row] : row) * kIn + k] : 0.f;
+  }
+  lds_barrier();
   // inputs as operand planes: 8 rows of one column per thread
   for (int q = t; q < kInK * (ROWS / 8); q += 512) {
     const int k = q % kInK, rg = q / kInK * 8;
     bf16x8 h, l;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const int row = r0 + rg + e;
-      float v = 0.f;
-      if (k < kIn && row < a.n) v = a.X[(size_t)(a.perm ? a.perm[row] : row) * kIn + k];
       __bf16 hr, lr;
-      split_bf16(v, hr, lr);
+      split_bf16(xs[rg + e][k], hr, lr);
       h[e] = hr;
       l[e] = lr;
     }
@@ -414,14 +419,6 @@ __global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
   }
   // input layer in FP32, one chain of multiply-adds per (row, unit)
   {
-    const float* x[RT][4];
-#pragma unroll
-    for (int j = 0; j < RT; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {     // rows past n: any row's, and zero below
-        const int row = min(r0 + j * 16 + q4 + r, a.n - 1);
-        x[j][r] = a.X + (size_t)(a.perm ? a.perm[row] : row) * kIn;
-      }
     const float* const w = a.P + kOffW1 + (size_t)(ub + r16) * kIn;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -429,7 +426,7 @@ __global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
 #pragma unroll
       for (int j = 0; j < RT; ++j) acc[i][j] = floatx4{bias, bias, bias, bias};
     }
-#pragma unroll 3
+#pragma unroll 5
     for (int k = 0; k < kIn; k += 4) {
       floatx4 wv[2];
 #pragma unroll
@@ -438,7 +435,7 @@ __global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
       for (int j = 0; j < RT; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const floatx4 xv = *(const floatx4*)(x[j][r] + k);
+          const floatx4 xv = *(const floatx4*)&xs[j * 16 + q4 + r][k];
 #pragma unroll
           for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -521,8 +518,9 @@ __global__ __launch_bounds__(512) void train_tile_kernel(TrainArgs a) {
 #pragma unroll
       for (int j = 0; j < RT; ++j) {
         put(i, j, dz[i][j], act + kActD + 2 * l * kPlane, l > 0);
-        *(floatx4*)(dzs + l * kPlane + (size_t)(ub + i * 16 + r16) * kRowBlock + rb + j * 16 +
-                    q4) = dz[i][j];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          dzs[l * kPlane + (size_t)(rb + j * 16 + q4 + r) * kH + ub + i * 16 + r16] = dz[i][j][r];
       }
     if (l == 0) break;
     lds_barrier();
@@ -557,17 +555,15 @@ __global__ __launch_bounds__(256) void weight_grad_kernel(WeightGradArgs g) {
   float* const ws = g.ws + (size_t)blockIdx.y * kWsStride;
   if (job >= 14) {
     const int layer = job - 14, unit = (int)threadIdx.x;
-    floatx4 s[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) s[q] = floatx4{0.f, 0.f, 0.f, 0.f};
+    float s[kRowBlock] = {};
     for (int b = b0; b < b1; ++b) {
-      const float* d = g.dz + (size_t)b * kDzBlock + layer * kPlane + (size_t)unit * kRowBlock;
+      const float* d = g.dz + (size_t)b * kDzBlock + layer * kPlane + unit;
 #pragma unroll
-      for (int q = 0; q < 8; ++q) s[q] += *(const floatx4*)(d + 4 * q);
+      for (int q = 0; q < kRowBlock; ++q) s[q] += d[q * kH];
     }
     float sum = 0.f;
 #pragma unroll
-    for (int q = 0; q < 32; ++q) sum += s[q >> 2][q & 3];
+    for (int q = 0; q < kRowBlock; ++q) sum += s[q];
     ws[kWsB + layer * kH + unit] = sum;
     return;
   }
