@@ -105,7 +105,8 @@ anacor_ctx *anacor_ctx_create(const uint8_t *volume, const int64_t shape[3],
 void anacor_ctx_destroy(anacor_ctx *ctx);
 
 /* Voxels per workgroup tile (0 = automatic: at most 1,024 in the raw
- * layout, 384 in the bricked ones). */
+ * layout, 384 in the bricked ones; over free distances 1,024, and 512 above
+ * 64 MB). */
 int anacor_ctx_set_tile(anacor_ctx *ctx, int voxels_per_tile);
 
 /* Launch order of the trace kernel (speed only, never results): reflections
@@ -126,13 +127,16 @@ int anacor_ctx_set_order(anacor_ctx *ctx, int refl_group, int direction_major);
 int anacor_ctx_get_work_shape(const anacor_ctx *ctx, int block[3], int *tile, int *refl_group,
                               int *direction_major);
 
-/* Volume layout of the trace kernel.  Never changes a result: every layout
+/* Volume layout of the trace kernel.  A requested layout never changes a result: each
  * yields the same labels along every ray (bit-identical results).  Bricks are
  * 8x8x8 voxels; 4-bit bricks store labels 0..4 as they are and any other value
  * as 5, which the boundary rule cannot tell apart (only 0, "changed" and
  * 0..4 matter to it).  The packed copy is built on the GPU on first use; the
- * raw volume stays resident (path records and the batched path use it). */
-#define ANACOR_LAYOUT_AUTO   (-1)  /* bricks above 64 MB; ANACOR_VOLUME_LAYOUT=raw|brick overrides */
+ * raw volume stays resident (path records and the batched path use it).  The
+ * automatic layout's means may differ from the others' in the last bits of a few
+ * FP64 operations per ray; a requested layout always steps. */
+#define ANACOR_LAYOUT_AUTO   (-1)  /* the walk over free distances where it applies, else
+                                     * bricks above 64 MB; ANACOR_VOLUME_LAYOUT=raw|brick overrides */
 #define ANACOR_LAYOUT_RAW    0     /* uint8 [z][y][x] */
 #define ANACOR_LAYOUT_BRICK  1     /* 2-bit bricks if every label is 0..3, else 4-bit */
 #define ANACOR_LAYOUT_BRICK2 2     /* 2-bit bricks (error unless every label is 0..3) */
