@@ -248,11 +248,15 @@ static_assert(sizeof(AxisLds) == 80, "AxisLds layout");
 // Whether the walk may leave along `axis`: the face's precondition holds, and
 // its deltas agree with the direction that chooses the face, so that every
 // origin leaving there keeps its stepped coordinates within a voxel of the
-// volume (ext: largest extent) and moves into the direction's octant.  A NaN
-// fails its comparison.  scale: 65536 / the largest move of a step along the
-// three axes, rounded down.
+// volume (ext: largest extent) and moves into the octant whose field is read:
+// bu, cu say whether that lies upward along the stepped axes.  (A component of
+// exactly zero can have a delta of either sign: the angles of a direction
+// without an x component are those of one 0.001 off, and the octant is the
+// zero's sign bit.)  A NaN fails its comparison.  scale: 65536 / the largest
+// move of a step along the three axes, rounded down.
 __device__ __forceinline__ bool exit_usable(const RayRule* __restrict__ rr, int axis,
-                                            const AxisExit& e, int ext, int& scale) {
+                                            const AxisExit& e, bool bu, bool cu, int ext,
+                                            int& scale) {
   const int b = axis == 0 ? 1 : 0, c = axis == 2 ? 1 : 2;
   const double sg = rr->neg ? -1.0 : 1.0;
   const double ea = __builtin_fabs(rr->dir[axis]), eb = sg * rr->dir[b], ec = sg * rr->dir[c];
@@ -264,7 +268,8 @@ __device__ __forceinline__ bool exit_usable(const RayRule* __restrict__ rr, int 
   if (mb <= 1.0 && mc <= 1.0) scale = 65536;
   return (rr->meta[e.face] & kMetaValid) && ea >= 0x1p-500 && ea <= 0x1p500 && mb <= 0x1p20 &&
          mc <= 0x1p20 && __builtin_fabs(db * ea - eb) <= slack &&
-         __builtin_fabs(dc * ea - ec) <= slack && db * eb >= 0.0 && dc * ec >= 0.0;
+         __builtin_fabs(dc * ea - ec) <= slack && (db == 0.0 || (db > 0.0) == bu) &&
+         (dc == 0.0 || (dc > 0.0) == cu);
 }
 
 // Offset of a stepped axis at m = RN(inc * d); `near` when some origin's
@@ -522,7 +527,8 @@ struct SkipRay {
       const double* d = rr->d[e.face];
       AxisLds& A = axes[tid];
       A.at = k.at[tid] * (int)sizeof(Words);
-      A.near = exit_usable(rr, tid, e, max(a.Z, max(a.Y, a.X)), A.scale) ? 0x7fffffff : 0;
+      A.near = exit_usable(rr, tid, e, tid == 0 ? ey.up : ez.up, tid == 2 ? ey.up : ex.up,
+                           max(a.Z, max(a.Y, a.X)), A.scale) ? 0x7fffffff : 0;
       A.add = e.add;
       A.hb = (tid == 0 ? a.Y : a.Z) - 1;
       A.hc = (tid == 2 ? a.Y : a.X) - 1;
