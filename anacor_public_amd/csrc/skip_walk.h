@@ -289,24 +289,6 @@ __device__ __forceinline__ unsigned bit_select(unsigned m, unsigned a, unsigned 
   return r;
 }
 
-// sqrt(S) / D for S zero or well inside the exponent range and D a small positive
-// integer: reciprocal and reciprocal root refined to an ulp or two, a third of
-// the instructions of the correctly rounded pair.  The FP64 mean keeps those.
-template <bool EXACT>
-__device__ __forceinline__ double root_over(double S, double D) {
-  if (EXACT) return __builtin_sqrt(S) / D;
-  double y = __builtin_amdgcn_rsq(S);
-  double g = S * y, h = 0.5 * y;
-  double e = __builtin_fma(-h, g, 0.5);
-  g = __builtin_fma(g, e, g);
-  h = __builtin_fma(h, e, h);
-  g = __builtin_fma(__builtin_fma(-g, g, S), h, g);
-  double q = __builtin_amdgcn_rcp(D);
-  q = __builtin_fma(__builtin_fma(-D, q, 1.0), q, q);
-  q = __builtin_fma(__builtin_fma(-D, q, 1.0), q, q);
-  return S > 0.0 ? g * q : 0.0;       // a ray held on its origin by the clamps
-}
-
 // How a walk reads its field.  Words: a position, or a table's entry, as words
 // whose sums are the position after a step.
 struct VoxelField {
@@ -581,7 +563,7 @@ struct SkipRay {
 
   // mu * length of one voxel's ray; kRayRedo in err where the walk does not
   // cover it.  col: this lane's step counters (zero before and after).
-  template <bool EXACT, class Args>
+  template <class Args>
   __device__ __forceinline__ double trace(const RayRule* __restrict__ rr, const int4 q,
                                           const Args& a, const SkipArgs& k, const AxisLds* axes,
                                           const Words* tbl, uint32_t* col, unsigned& err,
@@ -652,7 +634,9 @@ struct SkipRay {
         const double b_ = (double)(ib - cb) * A.vb;
         const double c_ = (double)(ic - cc) * A.vc;
         const double p_ = (double)dp * A.vp;
-        r = root_over<EXACT>(b_ * b_ + c_ * c_ + p_ * p_, D) * (W * 0.125);
+        r = ray_weight(__builtin_fma(b_, b_, __builtin_fma(c_, c_, p_ * p_)), W * 0.125, D,
+                       [](double v) { return __builtin_amdgcn_rsq(v); },
+                       [](double v) { return __builtin_amdgcn_rcp(v); });
       }
     }
     return r;
@@ -696,7 +680,7 @@ void skip_kernel(TraceArgs a, SkipArgs k) {
       const int s1 = min(v_end, s0 + kVox * kBlock);
 #pragma unroll 1
       for (int v = s0 + tid; v < s1; v += kBlock) {
-        double r = walk.template trace<F64>(rr, k.vox[v], a, k, axes, tbl, col, acc.err, steps);
+        double r = walk.trace(rr, k.vox[v], a, k, axes, tbl, col, acc.err, steps);
         double* const first = incident + (v - s0);
         if (ray == 0) {
           *first = r;
@@ -747,7 +731,7 @@ void skip_map_kernel(GridArgs a, SkipArgs k) {
   const int v_end = min(a.N, (tile + 1) * a.vox_per_tile);
 #pragma unroll 1
   for (int v = tile * a.vox_per_tile + (int)threadIdx.x; v < v_end; v += kBlock) {
-    const double r = walk.template trace<true>(rr, k.vox[v], a, k, axes, tbl, col, err, steps);
+    const double r = walk.trace(rr, k.vox[v], a, k, axes, tbl, col, err, steps);
     a.map[(size_t)d * a.N + k.index[v]] = (float)(a.is_exp ? exp(-r) : r);
   }
   if (err) atomicOr(&a.err[d], err);

@@ -39,6 +39,8 @@
 
 #include "errors.h"
 #include "geometry.h"
+#define ANACOR_DEVICE __device__
+#include "ray_weight.h"
 #include "../../include/anacor_mi355x.h"
 
 namespace anacor {
