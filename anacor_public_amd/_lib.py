@@ -29,6 +29,7 @@ LAYOUT_RAW = 0
 LAYOUT_BRICK = 1
 LAYOUT_BRICK2 = 2
 LAYOUT_BRICK4 = 4
+WALK_STEPS, WALK_VOXELS, WALK_CELLS = 0, 1, 2
 RAY_ERR_FACE = 1
 RAY_ERR_ASSERT = 2
 NOALLOC_MAX_REFLECTIONS = 16384
@@ -46,7 +47,7 @@ EXPORTED = (
     "anacor_ctx_set_voxel_block",
     "anacor_ctx_set_layout", "anacor_ctx_get_layout", "anacor_ctx_run",
     "anacor_ctx_run_noalloc", "anacor_ctx_paths",
-    "anacor_ctx_stats", "anacor_reflection_geometry", "anacor_batch_create",
+    "anacor_ctx_stats", "anacor_ctx_last_walk", "anacor_reflection_geometry", "anacor_batch_create",
     "anacor_batch_destroy", "anacor_batch_sample", "anacor_batch_run", "anacor_batch_stats",
     "anacor_batch_set_graph", "anacor_batch_last_graph",
     "anacor_mlp_create", "anacor_mlp_destroy", "anacor_mlp_num_params", "anacor_mlp_get_params",
@@ -148,6 +149,8 @@ def _prototypes(lib):
     lib.anacor_ctx_paths.argtypes = [vp, vp, vp, i64, vp, vp, vp, vp]
     lib.anacor_ctx_stats.restype = ct.c_int
     lib.anacor_ctx_stats.argtypes = [vp, ct.POINTER(Stats)]
+    lib.anacor_ctx_last_walk.restype = ct.c_int
+    lib.anacor_ctx_last_walk.argtypes = [vp, ct.POINTER(i64)]
     lib.anacor_batch_create.restype = vp
     lib.anacor_batch_create.argtypes = [ct.POINTER(Sample), i32, i32, i32]
     lib.anacor_batch_destroy.restype = None

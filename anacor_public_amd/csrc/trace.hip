@@ -1369,6 +1369,8 @@ struct Context {
   unsigned long long last_steps = 0;
   int64_t last_blocks = 0;
   double last_host_ms = 0.0;
+  int last_walk = ANACOR_WALK_STEPS;
+  int64_t last_retraced = 0;    // reflections (directions) the skip walk left to the stepping kernel
   std::mutex mu_run;
 };
 
@@ -1759,6 +1761,12 @@ static int launch_group(const Context* c, int layout) {
   return (layout == kLayoutBrick2 || layout == kLayoutBrick4) ? kBrickGroup : 1;
 }
 
+// What a trace reports of its kernel (anacor_ctx_last_walk).
+static void note_walk(Context* c, bool skip) {
+  c->last_walk = !skip ? ANACOR_WALK_STEPS : c->d_fine ? ANACOR_WALK_CELLS : ANACOR_WALK_VOXELS;
+  c->last_retraced = 0;
+}
+
 // The skip walk's arguments and the bytes of its tables.
 static SkipArgs skip_args(const Context* c, unsigned* lds) {
   SkipArgs k;
@@ -1888,6 +1896,7 @@ static int retrace_marked(Context* c, const RunBuffers& B, const ReflRule* h_rul
       guard = guard || h_rules[i].ray[0].guard || h_rules[i].ray[1].guard;
     }
   if (n == 0) return ANACOR_OK;
+  c->last_retraced = n;
   const bool f64 = (flags & ANACOR_FLAG_F64_MEAN) != 0;
   const unsigned words = (unsigned)((R + 255) / 256);
   HIP_TRY(hipMemcpyAsync(B.order, h_redo, (size_t)n * sizeof(int), hipMemcpyHostToDevice,
@@ -1948,6 +1957,7 @@ static int trace_call(Context* c, const RunBuffers& B, const ReflRule* h_rules,
   const bool f64 = (flags & ANACOR_FLAG_F64_MEAN) != 0;
   const bool paths = paths_out != nullptr;
   const bool skip = !paths && use_skip(c, R);
+  note_walk(c, skip);
   const int64_t tiles = (c->N + vpt - 1) / vpt;
   const int64_t nblk = R * tiles;
   const int64_t RA = (prepare_rest && first > 0 && first < R) ? first : R;
@@ -3150,6 +3160,7 @@ static int batch_run(Batch* b, const double* const* s1, const double* const* ome
   unsigned long long repeated = 0;
   for (int i = 0; i < S; ++i) {
     Context* c = b->samples[(size_t)i];
+    note_walk(c, use_skip(c, R[i]));
     if (R[i] == 0 || c->N == 0 || !use_skip(c, R[i])) continue;
     bool any = false;
     for (int64_t r = 0; r < R[i] && !any; ++r) any = out[i][r] != out[i][r];
@@ -3287,6 +3298,7 @@ static int grid_build(Context* c, int64_t n_theta, int64_t n_phi, const double* 
   std::vector<unsigned> h_err((size_t)D, 0u);
   // the skip walk as in use_skip; the unrounded map keeps the stepping kernel
   const bool skip = skip_ready(c) && !d_map64 && (int64_t)D * N > (1 << 20);
+  note_walk(c, skip);
   if (N > 0) {
     const int vpt = fit_tile(N, D, skip ? skip_map_tile(N, D) : choose_tile(c, D));
     if (vpt == 0) {
@@ -3336,6 +3348,7 @@ static int grid_build(Context* c, int64_t n_theta, int64_t n_phi, const double* 
         return fail(e, "skip_map_kernel");
       for (int d = 0; d < D; ++d)
         if (h_err[(size_t)d]) marked.push_back(d);
+      c->last_retraced = (int64_t)marked.size();
       if (!marked.empty()) {       // these directions by the stepping kernel
         if ((e = hipMalloc(&marked_buf.p, marked.size() * sizeof(int))) != hipSuccess ||
             (e = hipMemcpyAsync(marked_buf.p, marked.data(), marked.size() * sizeof(int),
@@ -4182,6 +4195,12 @@ int anacor_batch_set_graph(anacor_batch* batch, int use_graph) {
   std::lock_guard<std::mutex> lk(batch->b->mu);
   batch->b->use_graph = use_graph != 0;
   return ANACOR_OK;
+}
+
+int anacor_ctx_last_walk(const anacor_ctx* ctx, int64_t* retraced) {
+  if (!ctx || !ctx->c) return -1;
+  if (retraced) *retraced = ctx->c->last_retraced;
+  return ctx->c->last_walk;
 }
 
 int anacor_batch_last_graph(const anacor_batch* batch) {

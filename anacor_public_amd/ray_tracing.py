@@ -328,6 +328,13 @@ class Tracer:
                     workgroups=int(st.workgroups), n_voxels=int(st.n_voxels),
                     host_ms=st.host_ms, outside_reads=int(st.outside_reads))
 
+    def last_walk(self) -> tuple:
+        """(_lib.WALK_*, retraced): how the most recent trace or map went along
+        its rays, and how many reflections (directions) the walk by free
+        distances left to the stepping kernel."""
+        n = ct.c_int64()
+        return int(self._lib.anacor_ctx_last_walk(self.handle, ct.byref(n))), int(n.value)
+
     @classmethod
     def _borrow(cls, handle: int, n_voxels: int, shape) -> "Tracer":
         """A non-owning Tracer over a handle owned by a Batch."""

@@ -187,13 +187,13 @@ def volume_bytes(shape, layout: int) -> int:
     return bricks * (128 if layout == 2 else 256)
 
 
-def gather_ceiling(nbytes: int, achieved_gbs: float) -> dict:
+def gather_ceiling(nbytes: int, achieved_gbs) -> dict:
     """The device's one-byte gather rate with no arithmetic between loads
     (anacor_probe_gather), on a working set of the next power of two above
     the volume: every lane its own pseudo-random byte ("lanes"), and a wave's
     64 lanes one 64-byte row ("row", the shape of the walk's gathers).  At one
-    byte per load, in GB/s, with the kernel's algorithmic rate as a fraction
-    of each."""
+    byte per load, in GB/s, with the stepping kernel's algorithmic rate as a
+    fraction of each (null for the walk by free distances)."""
     import ctypes as ct
     from anacor_public_amd import _lib
     lib = _lib.load()
@@ -204,7 +204,7 @@ def gather_ceiling(nbytes: int, achieved_gbs: float) -> dict:
         _lib.check(lib.anacor_probe_gather(0, k, pattern, 1 << 34, ct.byref(rate)), lib)
         gbs = rate.value / 1e9
         out[f"{name}_GBps"] = gbs
-        out[f"frac_of_{name}"] = achieved_gbs / gbs if gbs > 0 else None
+        out[f"frac_of_{name}"] = achieved_gbs / gbs if achieved_gbs and gbs > 0 else None
     return out
 
 
@@ -490,6 +490,27 @@ def traffic_for(name: str, layout: int, block, tile: int, group: int, vsteps: in
     return None if per is None else per * vsteps
 
 
+def trace_roofline(walks, kernel_ms: float, vsteps: int, traffic, batched: bool) -> dict:
+    """Roofline position of a trace whose samples went along their rays as in
+    `walks` (_lib.WALK_*).  The stepping kernel reads one label, a byte, per
+    voxel step, which a full-size volume takes from memory.  The walk by free
+    distances answers a step from a byte read many steps before, out of the
+    caches, and is bound by VALU issue and the texture addresser: no rate of
+    bytes describes it, and none is reported."""
+    from anacor_public_amd import _lib
+    step = _lib.WALK_STEPS in walks
+    skip = bool(set(walks) - {_lib.WALK_STEPS})
+    rate = vsteps / (kernel_ms * 1e-3) / 1e9
+    return {"bound": "valu issue and texture addresser" if skip else "hbm",
+            "achieved": None if skip else rate, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+            "frac": None if skip else rate / HBM_PEAK_GBS,
+            "traffic": None if skip else traffic,
+            "kernel": " and ".join(["skip_kernel"] * skip + ["trace_kernel"] * step) +
+                      (", one launch per sample" if batched else ""),
+            "kernel_ms": kernel_ms, "bytes_per_launch": None if skip else vsteps,
+            "voxel_steps_per_launch": vsteps}
+
+
 def measure_plain(config: str, steps: int, warmup: int, cpu_budget: float,
                   reflections: int = 0, tile: int = 0, autotune_on: bool = True,
                   gather: bool = True) -> dict:
@@ -498,7 +519,7 @@ def measure_plain(config: str, steps: int, warmup: int, cpu_budget: float,
     every reflection's A_h.  Returns the record (value in A_h/s, roofline of
     the trace kernel, CPU baseline on a bounded sample of the same
     workload)."""
-    from anacor_public_amd import _lib, autotune
+    from anacor_public_amd import autotune
     from anacor_public_amd import workload as W
     from anacor_public_amd.ray_tracing import Batch, Tracer
     t0 = time.perf_counter()
@@ -515,9 +536,6 @@ def measure_plain(config: str, steps: int, warmup: int, cpu_budget: float,
     log(f"# workload {name}: volumes {[w.volume.shape for w in wls]}, N={N}, R={R} "
         f"(built in {time.perf_counter() - t0:.1f}s)")
     extra = {}
-    # the automatic layout walks by free distances (skip_kernel), for which no
-    # traffic per voxel step is on record
-    skip = "ANACOR_VOLUME_LAYOUT" not in os.environ
     if config == "batched":
         runner = Batch(wls)
         if autotune_on:
@@ -540,7 +558,6 @@ def measure_plain(config: str, steps: int, warmup: int, cpu_budget: float,
                                  trial=512, layouts=autotune.LAYOUTS, use_cache=False)
             extra["autotune"] = {"layout": pick["layout"], "block": pick["block"],
                                  "tile": pick["tile"]}
-            skip = skip and pick["layout"] == _lib.LAYOUT_AUTO
             log(f"# autotune ({time.perf_counter() - t1:.1f}s): {extra['autotune']}")
 
         def call():
@@ -561,7 +578,8 @@ def measure_plain(config: str, steps: int, warmup: int, cpu_budget: float,
     value = R * steps / elapsed
     k_ms = float(np.mean(kernel_ms))
     vsteps = int(vsteps_l[-1])
-    achieved = vsteps * 1.0 / (k_ms * 1e-3) / 1e9   # 1 algorithmic byte per voxel step
+    tracers = [runner.sample(i) for i in range(runner.n)] if config == "batched" else [runner]
+    walks = {t.last_walk()[0] for t in tracers}
     extra["host_setup_ms"] = float(np.mean(host_ms))
     log(f"# {name}: {steps} steps, {ms_per_step:.2f} ms/step, trace kernel {k_ms:.2f} ms, "
         f"host setup {extra['host_setup_ms']:.2f} ms, {vsteps} voxel steps per launch")
@@ -580,13 +598,12 @@ def measure_plain(config: str, steps: int, warmup: int, cpu_budget: float,
         log(f"# cpu baseline ({cpu['kind']}, {cpu['cores']} cores): {cpu['value']:.2f} A_h/s, "
             f"max rel diff vs GPU {rel:.2e}")
     layout = 0 if config == "batched" else runner.layout
-    traffic, shape = None, None
+    traffic = None
     if config != "batched":
         shape = runner.work_shape()
         key_name = name if not reflections else f"{name}-first{reflections}"
-        if not skip:
-            traffic = traffic_for(key_name, layout, shape["block"], shape["tile"],
-                                  shape["group"], vsteps)
+        traffic = traffic_for(key_name, layout, shape["block"], shape["tile"], shape["group"],
+                              vsteps)
         extra["work_shape"] = shape
     pairs = sum(len(w.coords) * len(w.omega) for w in wls)
     rec = {
@@ -602,11 +619,7 @@ def measure_plain(config: str, steps: int, warmup: int, cpu_budget: float,
         "volume_layout": {0: "raw", 2: "brick2", 4: "brick4"}[layout],
         "rays_per_s": 2.0 * pairs / (ms_per_step * 1e-3),
         "voxel_steps_per_s": vsteps / (ms_per_step * 1e-3),
-        "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                     "kernel": ("skip_kernel" if skip else "trace_kernel") +
-                               (", one launch per sample" if config == "batched" else ""),
-                     "kernel_ms": k_ms, "bytes_per_launch": vsteps},
+        "roofline": trace_roofline(walks, k_ms, vsteps, traffic, config == "batched"),
         "cpu_baseline": cpu,
         "speedup_vs_cpu": (value / cpu["value"]) if cpu else None,
     }
@@ -637,10 +650,10 @@ def measure_plain(config: str, steps: int, warmup: int, cpu_budget: float,
             f"(results identical: {same})")
     if config != "batched" and gather:
         rec["roofline"]["gather_ceiling"] = gather_ceiling(
-            volume_bytes(wls[0].volume.shape, layout), achieved)
+            volume_bytes(wls[0].volume.shape, layout), rec["roofline"]["achieved"])
         gc = rec["roofline"]["gather_ceiling"]
         log(f"# gather ceiling at {gc['working_set_bytes']} B: lanes {gc['lanes_GBps']:.0f} GB/s, "
-            f"row {gc['row_GBps']:.0f} GB/s; trace kernel at {achieved:.0f} GB/s")
+            f"row {gc['row_GBps']:.0f} GB/s")
     rec.update(extra)
     runner.close()
     return rec

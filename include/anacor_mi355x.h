@@ -209,6 +209,16 @@ typedef struct {
 } anacor_stats_t;
 int anacor_ctx_stats(const anacor_ctx *ctx, anacor_stats_t *stats);
 
+/* How the most recent trace, batch run or absorption map on ctx went along its
+ * rays: voxel by voxel, or by the free distances of single voxels or of cells
+ * of 4x4x4 voxels (ANACOR_LAYOUT_AUTO).  *retraced (may be NULL): the
+ * reflections, or directions of a map, that the walk by free distances left to
+ * the stepping kernel.  -1 for a null context. */
+#define ANACOR_WALK_STEPS  0
+#define ANACOR_WALK_VOXELS 1
+#define ANACOR_WALK_CELLS  2
+int anacor_ctx_last_walk(const anacor_ctx *ctx, int64_t *retraced);
+
 /* ----------------------------------------------------------- batched path */
 
 /* One independent sample of a batch: its label volume, crystal voxels,
