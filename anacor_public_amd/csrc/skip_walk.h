@@ -236,7 +236,8 @@ struct AxisExit {
 // What a lane needs of its exit axis, read from LDS by the axis.
 struct AxisLds {
   int at;                      // byte offset of its table
-  int near;                    // increments from here on are not tabulated (0: none)
+  int near;                    // increments from here on are not tabulated (0: none;
+                               // -1: the reference aborts on rays leaving here)
   int scale, add;
   int hb, hc;                  // extents - 1 of the two stepped axes
   int face, up;
@@ -510,7 +511,8 @@ struct SkipRay {
       AxisLds& A = axes[tid];
       A.at = k.at[tid] * (int)sizeof(Words);
       A.near = exit_usable(rr, tid, e, tid == 0 ? ey.up : ez.up, tid == 2 ? ey.up : ex.up,
-                           max(a.Z, max(a.Y, a.X)), A.scale) ? 0x7fffffff : 0;
+                           max(a.Z, max(a.Y, a.X)), A.scale) ? 0x7fffffff
+               : (rr->meta[e.face] & kMetaValid) ? 0 : -1;
       A.add = e.add;
       A.hb = (tid == 0 ? a.Y : a.Z) - 1;
       A.hc = (tid == 2 ? a.Y : a.X) - 1;
@@ -561,12 +563,14 @@ struct SkipRay {
     ox = ex.up ? a.X : 0;
   }
 
-  // mu * length of one voxel's ray; kRayRedo in err where the walk does not
-  // cover it.  col: this lane's step counters (zero before and after).
+  // mu * length of one voxel's ray; where the walk does not cover it, kRayRedo
+  // in err (in LDS: hardly a ray needs it) and 0, where the reference aborts the
+  // stepping kernel's error and NaN.  col: this lane's step counters (zero
+  // before and after).
   template <class Args>
   __device__ __forceinline__ double trace(const RayRule* __restrict__ rr, const int4 q,
                                           const Args& a, const SkipArgs& k, const AxisLds* axes,
-                                          const Words* tbl, uint32_t* col, unsigned& err,
+                                          const Words* tbl, uint32_t* col, unsigned* err,
                                           unsigned& steps) const {
     double r = 0.0;
     const int z = q.x & 0xffff, y = (int)((unsigned)q.x >> 16), x = q.y;
@@ -587,12 +591,25 @@ struct SkipRay {
                                        rr->neg != 0);
       p = (face == 2 || face == 3) ? 0 : (face == 4 || face == 5) ? 1 : 2;
       use = face - 1 == axes[p].face;
+      // a voxel on the lower plane that the reference finds first, at distance 0
+      // also for a ray that leaves it: one step, of length 0, whatever the deltas
+      const bool lower = face == 2 || face == 4 || face == 6;
+      if (lower && (p == 0 ? z : p == 1 ? y : x) == 0) {
+        if (rr->meta[face - 1] & kMetaValid) {
+          ++steps;
+          return 0.0;
+        }
+        atomicOr(err, ANACOR_RAY_ERR_ASSERT);
+        return __builtin_nan("");
+      }
     }
     const AxisLds& A = axes[p];
     const int kp = p == 0 ? kz : p == 1 ? ky : kx;
     const int limit = kp + A.add;
     if (!use || limit > A.near) {
-      err |= kRayRedo;
+      const bool abort = use && A.near < 0;
+      atomicOr(err, abort ? ANACOR_RAY_ERR_ASSERT : kRayRedo);
+      if (abort) r = __builtin_nan("");
     } else {
       const int scale = A.scale;
       const Words at = Field::origin(q);
@@ -654,6 +671,7 @@ void skip_kernel(TraceArgs a, SkipArgs k) {
   __shared__ AxisLds axes[3];
   __shared__ double incident[kVox * kBlock];  // the first ray's exponent per voxel
   __shared__ ReduceLds red;
+  __shared__ unsigned err;
 
   const int lb = xcd_logical_block((int)blockIdx.x, (int)gridDim.x);
   if (lb >= a.n_blocks) return;
@@ -666,6 +684,7 @@ void skip_kernel(TraceArgs a, SkipArgs k) {
   uint32_t* const col = hist + tid;
 #pragma unroll
   for (int l = 1; l < 5; ++l) col[l * kBlock] = 0;
+  if (tid == 0) err = 0;
   TileAcc acc = {0.f, 0.f, 0.0, 0ull, 0u};
   unsigned steps = 0;
   const int v_begin = tile * a.vox_per_tile;
@@ -677,10 +696,17 @@ void skip_kernel(TraceArgs a, SkipArgs k) {
       const RayRule* __restrict__ rr = &rule->ray[ray];
       __syncthreads();                          // the table's last readers are done
       const SkipRay<Field> walk(rr, a, k, axes, tbl);
+      // where the first ray aborts there is no second one (its voxels hold NaN)
+      const bool aborts = ray == 1 && __builtin_amdgcn_readfirstlane((int)err) != 0;
       const int s1 = min(v_end, s0 + kVox * kBlock);
 #pragma unroll 1
       for (int v = s0 + tid; v < s1; v += kBlock) {
-        double r = walk.trace(rr, k.vox[v], a, k, axes, tbl, col, acc.err, steps);
+        if (aborts) {
+          int w = v - s0;                         // its own address: no register across trace()
+          asm volatile("" : "+v"(w));
+          if (incident[w] != incident[w]) continue;
+        }
+        double r = walk.trace(rr, k.vox[v], a, k, axes, tbl, col, &err, steps);
         double* const first = incident + (v - s0);
         if (ray == 0) {
           *first = r;
@@ -703,6 +729,7 @@ void skip_kernel(TraceArgs a, SkipArgs k) {
   const int slot = pos * a.tiles + tile;
   reduce_tile<F64, false>(acc, red, &a.err[refl], a.steps, a.partial32 + slot,
                           a.partial64 + slot);
+  if (tid == 0 && err) atomicOr(&a.err[refl], err);   // behind reduce_tile's barrier
 }
 
 // The absorption map (grid_map_kernel) by the skip walk: one direction per
@@ -718,6 +745,7 @@ void skip_map_kernel(GridArgs a, SkipArgs k) {
   typename Field::Words* const tbl = (typename Field::Words*)tables;
   __shared__ uint32_t hist[5 * kBlock];
   __shared__ AxisLds axes[3];
+  __shared__ unsigned err;
   const int lb = xcd_logical_block((int)blockIdx.x, (int)gridDim.x);
   if (lb >= a.n_blocks) return;
   const int d = lb / a.tiles;
@@ -726,13 +754,15 @@ void skip_map_kernel(GridArgs a, SkipArgs k) {
 #pragma unroll
   for (int l = 1; l < 5; ++l) col[l * kBlock] = 0;
   const RayRule* __restrict__ rr = a.rays + d;
+  if (threadIdx.x == 0) err = 0;
   const SkipRay<Field> walk(rr, a, k, axes, tbl);
-  unsigned err = 0, steps = 0;
+  unsigned steps = 0;
   const int v_end = min(a.N, (tile + 1) * a.vox_per_tile);
 #pragma unroll 1
   for (int v = tile * a.vox_per_tile + (int)threadIdx.x; v < v_end; v += kBlock) {
-    const double r = walk.trace(rr, k.vox[v], a, k, axes, tbl, col, err, steps);
+    const double r = walk.trace(rr, k.vox[v], a, k, axes, tbl, col, &err, steps);
     a.map[(size_t)d * a.N + k.index[v]] = (float)(a.is_exp ? exp(-r) : r);
   }
-  if (err) atomicOr(&a.err[d], err);
+  __syncthreads();
+  if (threadIdx.x == 0 && err) atomicOr(&a.err[d], err);
 }

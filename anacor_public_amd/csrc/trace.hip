@@ -1841,6 +1841,15 @@ __global__ void clear_run_kernel(unsigned* __restrict__ err, int R,
                                  unsigned long long* __restrict__ steps) {
   const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   if (i < R) err[i] = 0u;
+  if (i == 0) *steps = 0ull;
+}
+
+// The same for the listed reflections' error words only.
+__global__ void clear_listed_kernel(const int* __restrict__ list, int n,
+                                    unsigned* __restrict__ err,
+                                    unsigned long long* __restrict__ steps) {
+  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (i < n) err[list[i]] = 0u;
   if (i == 0 && steps) *steps = 0ull;
 }
 
@@ -1878,8 +1887,17 @@ static TraceArgs trace_args(const Context* c, const RunBuffers& B, int vpt, int 
   return a;
 }
 
-// The reflections that the skip walk marked (kRayRedo in h_err[R], downloaded
-// by the caller with their means NaN) once more with the stepping kernel:
+// Whether the stepping kernel has to trace a reflection that the skip walk left
+// with the error word err: marked, or aborted on the first ray where the second,
+// which the walk then did not look at, may have no exit face to report.
+static bool needs_stepping(unsigned err, const ReflRule& r) {
+  if (err & kRayRedo) return true;
+  const double* d = r.ray[1].dir;
+  return err && !(std::isfinite(d[0]) && std::isfinite(d[1]) && std::isfinite(d[2]));
+}
+
+// The reflections that the skip walk did not cover (needs_stepping; their error
+// words in h_err[R], downloaded by the caller with their means NaN) once more with the stepping kernel:
 // their means into out, their error words into h_err, and the step count in
 // *steps corrected (the marked reflections' blocks had counted what they
 // walked, which a second skip walk of them alone counts again; *repeated sums
@@ -1891,25 +1909,25 @@ static int retrace_marked(Context* c, const RunBuffers& B, const ReflRule* h_rul
   int n = 0;
   bool guard = false;
   for (int64_t i = 0; i < R; ++i)
-    if (h_err[i] & kRayRedo) {
+    if (needs_stepping(h_err[i], h_rules[i])) {
       h_redo[n++] = (int)i;
       guard = guard || h_rules[i].ray[0].guard || h_rules[i].ray[1].guard;
     }
   if (n == 0) return ANACOR_OK;
   c->last_retraced = n;
   const bool f64 = (flags & ANACOR_FLAG_F64_MEAN) != 0;
-  const unsigned words = (unsigned)((R + 255) / 256);
+  const unsigned words = (unsigned)((n + 255) / 256);
   HIP_TRY(hipMemcpyAsync(B.order, h_redo, (size_t)n * sizeof(int), hipMemcpyHostToDevice,
                          c->stream));
   TraceArgs a = trace_args(c, B, vpt, layout, flags, nullptr);
   const int per_launch = (int)std::max<int64_t>(1, kMaxBlocks / a.tiles);
-  hipLaunchKernelGGL(clear_run_kernel, dim3(words), dim3(256), 0, c->stream, B.err, (int)R,
+  hipLaunchKernelGGL(clear_listed_kernel, dim3(words), dim3(256), 0, c->stream, B.order, n, B.err,
                      B.steps + 1);
   HIP_TRY(hipGetLastError());
   for (int pass = 0; pass < 2; ++pass) {
     if (pass == 1) {     // the error words the stepping kernel will set
-      hipLaunchKernelGGL(clear_run_kernel, dim3(words), dim3(256), 0, c->stream, B.err, (int)R,
-                         (unsigned long long*)nullptr);
+      hipLaunchKernelGGL(clear_listed_kernel, dim3(words), dim3(256), 0, c->stream, B.order, n,
+                         B.err, (unsigned long long*)nullptr);
       HIP_TRY(hipGetLastError());
     }
     a.steps = pass == 0 ? B.steps + 1 : B.steps;
@@ -3347,14 +3365,18 @@ static int grid_build(Context* c, int64_t n_theta, int64_t n_phi, const double* 
           (e = hipStreamSynchronize(c->stream)) != hipSuccess)
         return fail(e, "skip_map_kernel");
       for (int d = 0; d < D; ++d)
-        if (h_err[(size_t)d]) marked.push_back(d);
+        if (h_err[(size_t)d] & kRayRedo) marked.push_back(d);
       c->last_retraced = (int64_t)marked.size();
       if (!marked.empty()) {       // these directions by the stepping kernel
+        const int n = (int)marked.size();
         if ((e = hipMalloc(&marked_buf.p, marked.size() * sizeof(int))) != hipSuccess ||
             (e = hipMemcpyAsync(marked_buf.p, marked.data(), marked.size() * sizeof(int),
-                                hipMemcpyHostToDevice, c->stream)) != hipSuccess ||
-            (e = hipMemsetAsync(d_err, 0, (size_t)D * sizeof(unsigned), c->stream)) != hipSuccess)
+                                hipMemcpyHostToDevice, c->stream)) != hipSuccess)
           return fail(e, "marked directions");
+        hipLaunchKernelGGL(clear_listed_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
+                           c->stream, (const int*)marked_buf.p, n, d_err,
+                           (unsigned long long*)nullptr);
+        if ((e = hipGetLastError()) != hipSuccess) return fail(e, "marked directions");
         a.dirs = (const int*)marked_buf.p;
         a.vox_per_tile = fit_tile(N, D, choose_tile(c, (int64_t)marked.size()));
         a.tiles = (N + a.vox_per_tile - 1) / a.vox_per_tile;
