@@ -695,6 +695,10 @@ void skip_kernel(TraceArgs a, SkipArgs k) {
     for (int ray = 0; ray < 2; ++ray) {
       const RayRule* __restrict__ rr = &rule->ray[ray];
       __syncthreads();                          // the table's last readers are done
+      if (__builtin_amdgcn_readfirstlane((int)err) & kRayRedo) {   // traced again anyway
+        s0 = v_end;
+        break;
+      }
       const SkipRay<Field> walk(rr, a, k, axes, tbl);
       // where the first ray aborts there is no second one (its voxels hold NaN)
       const bool aborts = ray == 1 && __builtin_amdgcn_readfirstlane((int)err) != 0;
@@ -727,9 +731,16 @@ void skip_kernel(TraceArgs a, SkipArgs k) {
   }
   acc.steps = steps;
   const int slot = pos * a.tiles + tile;
-  reduce_tile<F64, false>(acc, red, &a.err[refl], a.steps, a.partial32 + slot,
+  reduce_tile<F64, false>(acc, red, &a.err[refl], a.steps + refl, a.partial32 + slot,
                           a.partial64 + slot);
-  if (tid == 0 && err) atomicOr(&a.err[refl], err);   // behind reduce_tile's barrier
+  if (tid == 0 && err) {                        // behind reduce_tile's barrier
+    // a second ray that the walk did not look at behind an aborting first one may
+    // have no exit face, which is then the error to report
+    const double* const d = rule->ray[1].dir;
+    const bool face = __builtin_isfinite(d[0]) && __builtin_isfinite(d[1]) &&
+                      __builtin_isfinite(d[2]);
+    atomicOr(&a.err[refl], face ? err : err | kRayRedo);
+  }
 }
 
 // The absorption map (grid_map_kernel) by the skip walk: one direction per

@@ -132,7 +132,7 @@ struct TraceArgs {
   float2* partial32;           // [R * tiles] (sum, compensation)
   double* partial64;           // [R * tiles]
   unsigned* err;               // [R]
-  unsigned long long* steps;   // sum of len_path_2
+  unsigned long long* steps;   // sum of len_path_2 (skip_kernel: [R], per reflection)
   PathRecord* paths;           // [R * N] in original voxel order (paths kernel)
   const int* order;            // [R] caller's index of the reflection at each processing position
   const double* incd;          // (double)i for i = 0 .. incd_last
@@ -955,28 +955,48 @@ struct GridArgs {
 
 #include "skip_walk.h"
 
+// Adds a wave's voxel steps (st: this lane's reflection) to *total, or writes them
+// to out[wave] where out is set; every lane of every wave comes here.
+__device__ __forceinline__ void add_steps(unsigned long long st, unsigned long long* total,
+                                          unsigned long long* out) {
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) st += __shfl_xor(st, off);
+  const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t % kWave) return;
+  if (out) out[t / kWave] = st;
+  else if (st) atomicAdd(total, st);
+}
+
 // Per reflection: combine the tile partials in tile order and divide by N.
+// refl_steps: the skip walk's steps per reflection (may be `out` itself: a
+// reflection's mean replaces its count), added to *steps but for those that it
+// left to the stepping kernel; null where *steps is the whole call's already.
+// steps_out: the sums by wave instead of *steps.
 __global__ void finish_kernel(const float2* __restrict__ p32, const double* __restrict__ p64,
                               const unsigned* __restrict__ err, const int* __restrict__ order,
-                              int R, int tiles, int N, int f64, double* __restrict__ out,
-                              const unsigned long long* __restrict__ steps = nullptr,
-                              unsigned long long* __restrict__ steps_out = nullptr) {
+                              int R, int tiles, int N, int f64, double* out,
+                              const unsigned long long* refl_steps, unsigned long long* steps,
+                              unsigned long long* __restrict__ steps_out) {
   const int r = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (r >= R) return;
-  if (r == 0 && steps_out) *steps_out = *steps;
-  double sum = 0.0;
-  if (f64) {
-    for (int t = 0; t < tiles; ++t) sum += p64[(size_t)r * tiles + t];
-  } else {
-    float s = 0.f, c = 0.f;
-    for (int t = 0; t < tiles; ++t) {
-      const float2 q = p32[(size_t)r * tiles + t];
-      merge_pair(s, c, q.x, q.y);
+  unsigned long long st = 0;
+  if (r < R) {
+    double sum = 0.0;
+    if (f64) {
+      for (int t = 0; t < tiles; ++t) sum += p64[(size_t)r * tiles + t];
+    } else {
+      float s = 0.f, c = 0.f;
+      for (int t = 0; t < tiles; ++t) {
+        const float2 q = p32[(size_t)r * tiles + t];
+        merge_pair(s, c, q.x, q.y);
+      }
+      sum = (double)s - (double)c;
     }
-    sum = (double)s - (double)c;
+    const int refl = order[r];
+    if (refl_steps && !(err[refl] & kRayRedo)) st = refl_steps[refl];
+    if (!refl_steps && r == 0 && steps_out) st = *steps;
+    out[refl] = err[refl] ? __builtin_nan("") : sum / (double)N;
   }
-  const int refl = order[r];
-  out[refl] = err[refl] ? __builtin_nan("") : sum / (double)N;
+  if (refl_steps || steps_out) add_steps(st, steps, steps_out);
 }
 
 // ------------------------------------------------------------ batched path
@@ -1000,6 +1020,7 @@ __global__ void finish_kernel(const float2* __restrict__ p32, const double* __re
 struct BatchSample {
   const int* order;            // processing position -> reflection
   int N, R, tiles, vpt;
+  int skip;                    // by the skip walk: `out` counts its steps until the means
   float2* p32;                 // tile partials [R][tiles]
   double* p64;
   unsigned* err;               // [R]
@@ -1014,33 +1035,42 @@ __global__ void batch_clear_kernel(const BatchSample* __restrict__ samples, int 
   if (t == 0) *steps = 0ull;
   for (int s = 0; s < S; ++s) {
     const BatchSample& B = samples[s];
-    for (int r = t; r < B.R; r += (int)(gridDim.x * blockDim.x)) B.err[r] = 0u;
+    for (int r = t; r < B.R; r += (int)(gridDim.x * blockDim.x)) {
+      B.err[r] = 0u;
+      if (B.skip) B.out[r] = 0.0;
+    }
   }
 }
 
-// Per (sample, reflection): merge the tile partials in order, divide by N.
+// Per (sample, reflection): merge the tile partials in order, divide by N
+// (finish_kernel).
 __global__ void batch_finish_kernel(const BatchSample* __restrict__ samples, int S, int f64,
-                                    long long total_refl) {
+                                    long long total_refl, unsigned long long* steps) {
   const long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= total_refl) return;
-  long long base = 0;
-  int s = 0;
-  while (s < S && g >= base + samples[s].R) { base += samples[s].R; ++s; }
-  const BatchSample& B = samples[s];
-  const int r = (int)(g - base);
-  double sum = 0.0;
-  if (f64) {
-    for (int t = 0; t < B.tiles; ++t) sum += B.p64[(size_t)r * B.tiles + t];
-  } else {
-    float a = 0.f, c = 0.f;
-    for (int t = 0; t < B.tiles; ++t) {
-      const float2 q = B.p32[(size_t)r * B.tiles + t];
-      merge_pair(a, c, q.x, q.y);
+  unsigned long long st = 0;
+  if (g < total_refl) {
+    long long base = 0;
+    int s = 0;
+    while (s < S && g >= base + samples[s].R) { base += samples[s].R; ++s; }
+    const BatchSample& B = samples[s];
+    const int r = (int)(g - base);
+    double sum = 0.0;
+    if (f64) {
+      for (int t = 0; t < B.tiles; ++t) sum += B.p64[(size_t)r * B.tiles + t];
+    } else {
+      float a = 0.f, c = 0.f;
+      for (int t = 0; t < B.tiles; ++t) {
+        const float2 q = B.p32[(size_t)r * B.tiles + t];
+        merge_pair(a, c, q.x, q.y);
+      }
+      sum = (double)a - (double)c;
     }
-    sum = (double)a - (double)c;
+    const int refl = B.order[r];
+    if (B.skip && !(B.err[refl] & kRayRedo))
+      st = (unsigned long long)__double_as_longlong(B.out[refl]);
+    B.out[refl] = B.err[refl] ? __builtin_nan("") : sum / (double)B.N;
   }
-  const int refl = B.order[r];
-  B.out[refl] = B.err[refl] ? __builtin_nan("") : sum / (double)B.N;
+  add_steps(st, steps, nullptr);
 }
 
 // ------------------------------------------------------------- gridding
@@ -1419,8 +1449,7 @@ static int ensure_run_buffers(Context* c, int64_t R, int64_t n_partials, bool f6
     HIP_TRY(hipMalloc(&c->d_order, (size_t)R * sizeof(int)));
     c->refl_cap = (size_t)R;
   }
-  // two counters: the call's steps, and those of a repeated reflection's first trace
-  if (!c->d_steps) HIP_TRY(hipMalloc(&c->d_steps, 2 * sizeof(unsigned long long)));
+  if (!c->d_steps) HIP_TRY(hipMalloc(&c->d_steps, sizeof(unsigned long long)));
   return ANACOR_OK;
 }
 
@@ -1803,20 +1832,22 @@ static void launch_skip(const Context* c, const TraceArgs& a, int grid, bool f64
 
 // A call of few reflections as one record, in page-locked memory and on the
 // device: the rules, the processing order, the cleared error words and step
-// counters go up in one copy, and the finish kernel writes the means and the
-// step count into the record's page-locked end: three operations on the
-// stream instead of seven. 64^3, one reflection: 93 us per call
+// counters (the call's, and each reflection's) go up in one copy, and the finish
+// kernel writes the means and the step counts of its waves into the record's
+// page-locked end: three operations on the stream instead of seven. 64^3, one reflection: 93 us per call
 // before, 50 so; 256: 205 and 155 us.
 struct CallRecord {
   size_t order, err, steps, up, out, steps_out, total;   // byte offsets; up: bytes copied
+  size_t waves;                                          // of the finish kernel
   explicit CallRecord(int64_t R) {
     order = (size_t)R * sizeof(ReflRule);
     err = order + (size_t)R * sizeof(int);
     steps = (err + (size_t)R * sizeof(unsigned) + 15) / 16 * 16;
-    up = steps + 2 * sizeof(unsigned long long);
+    up = steps + (1 + (size_t)R) * sizeof(unsigned long long);
     out = (up + 63) / 64 * 64;
     steps_out = out + (size_t)R * sizeof(double);
-    total = steps_out + sizeof(unsigned long long);
+    waves = (size_t)(R + 255) / 256 * (256 / kWave);
+    total = steps_out + waves * sizeof(unsigned long long);
   }
   size_t records() const { return (total + sizeof(ReflRule) - 1) / sizeof(ReflRule); }
 };
@@ -1830,17 +1861,20 @@ struct RunBuffers {
   unsigned* err = nullptr;             // [R] per-reflection error bits
   double* out = nullptr;               // [R] means
   void* partial = nullptr;             // [R * tiles] float2 or double
-  unsigned long long* steps = nullptr; // [2] voxel-step counter, repeated steps
-  unsigned long long* h_steps = nullptr;   // CallRecord: its page-locked step count; then
+  unsigned long long* steps = nullptr; // voxel-step counter
+  unsigned long long* refl_steps = nullptr;   // [R] the skip walk's, per reflection
+  unsigned long long* h_steps = nullptr;   // CallRecord: its page-locked step counts; then
                                            // out is page-locked too
 };
 
 // Clears what a trace call accumulates into (a fill kernel rather than
 // hipMemsetAsync, so the sequence holds no memset node if it is captured).
 __global__ void clear_run_kernel(unsigned* __restrict__ err, int R,
-                                 unsigned long long* __restrict__ steps) {
+                                 unsigned long long* __restrict__ steps,
+                                 unsigned long long* __restrict__ refl_steps) {
   const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   if (i < R) err[i] = 0u;
+  if (i < R && refl_steps) refl_steps[i] = 0ull;
   if (i == 0) *steps = 0ull;
 }
 
@@ -1887,32 +1921,25 @@ static TraceArgs trace_args(const Context* c, const RunBuffers& B, int vpt, int 
   return a;
 }
 
-// Whether the stepping kernel has to trace a reflection that the skip walk left
-// with the error word err: marked, or aborted on the first ray where the second,
-// which the walk then did not look at, may have no exit face to report.
-static bool needs_stepping(unsigned err, const ReflRule& r) {
-  if (err & kRayRedo) return true;
-  const double* d = r.ray[1].dir;
-  return err && !(std::isfinite(d[0]) && std::isfinite(d[1]) && std::isfinite(d[2]));
-}
-
-// The reflections that the skip walk did not cover (needs_stepping; their error
-// words in h_err[R], downloaded by the caller with their means NaN) once more with the stepping kernel:
-// their means into out, their error words into h_err, and the step count in
-// *steps corrected (the marked reflections' blocks had counted what they
-// walked, which a second skip walk of them alone counts again; *repeated sums
-// those over the calls that share a counter).  h_redo: R words of work space.  Synchronous; nothing to do is the usual case.
+// The reflections that the skip walk marked (kRayRedo in h_err[R], downloaded by
+// the caller with their means NaN) once more with the stepping kernel: their
+// means into out, their error words into h_err, their steps added to *steps.
+// h_redo: the call's processing order, of which the marked ones are kept.
+// Synchronous; nothing to do is the usual case.  A call of nothing else costs
+// the tables and a walk that stops at the first mark of a workgroup beside the
+// stepping: 256^3, 6,000 reflections at 270 degrees, 26.9 ms with the walk
+// carried through and repeated for its step count, 21.0 so, 18.8 stepping only.
 static int retrace_marked(Context* c, const RunBuffers& B, const ReflRule* h_rules, int64_t R,
                           int vpt, int layout, int flags, double* out, unsigned* h_err,
-                          int* h_redo, unsigned long long* steps,
-                          unsigned long long* repeated) {
+                          int* h_redo, unsigned long long* steps) {
   int n = 0;
   bool guard = false;
-  for (int64_t i = 0; i < R; ++i)
-    if (needs_stepping(h_err[i], h_rules[i])) {
-      h_redo[n++] = (int)i;
-      guard = guard || h_rules[i].ray[0].guard || h_rules[i].ray[1].guard;
-    }
+  for (int64_t i = 0; i < R; ++i) {
+    const int r = h_redo[i];
+    if (!(h_err[r] & kRayRedo)) continue;
+    h_redo[n++] = r;
+    guard = guard || h_rules[r].ray[0].guard || h_rules[r].ray[1].guard;
+  }
   if (n == 0) return ANACOR_OK;
   c->last_retraced = n;
   const bool f64 = (flags & ANACOR_FLAG_F64_MEAN) != 0;
@@ -1922,38 +1949,27 @@ static int retrace_marked(Context* c, const RunBuffers& B, const ReflRule* h_rul
   TraceArgs a = trace_args(c, B, vpt, layout, flags, nullptr);
   const int per_launch = (int)std::max<int64_t>(1, kMaxBlocks / a.tiles);
   hipLaunchKernelGGL(clear_listed_kernel, dim3(words), dim3(256), 0, c->stream, B.order, n, B.err,
-                     B.steps + 1);
+                     B.steps);
   HIP_TRY(hipGetLastError());
-  for (int pass = 0; pass < 2; ++pass) {
-    if (pass == 1) {     // the error words the stepping kernel will set
-      hipLaunchKernelGGL(clear_listed_kernel, dim3(words), dim3(256), 0, c->stream, B.order, n,
-                         B.err, (unsigned long long*)nullptr);
-      HIP_TRY(hipGetLastError());
-    }
-    a.steps = pass == 0 ? B.steps + 1 : B.steps;
-    for (int p0 = 0; p0 < n; p0 += per_launch) {
-      a.R = std::min(per_launch, n - p0);
-      a.pos0 = p0;
-      a.n_blocks = a.R * a.tiles;
-      const int grid = (a.n_blocks + 7) / 8 * 8;
-      if (pass == 0) launch_skip(c, a, grid, f64, c->stream);
-      else dispatch_trace(a, grid, guard, c->full != 0, layout, f64, false, !c->labels_over4,
-                          c->stream);
-      HIP_TRY(hipGetLastError());
-    }
+  for (int p0 = 0; p0 < n; p0 += per_launch) {
+    a.R = std::min(per_launch, n - p0);
+    a.pos0 = p0;
+    a.n_blocks = a.R * a.tiles;
+    dispatch_trace(a, (a.n_blocks + 7) / 8 * 8, guard, c->full != 0, layout, f64, false,
+                   !c->labels_over4, c->stream);
+    HIP_TRY(hipGetLastError());
   }
-  hipLaunchKernelGGL(finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream,
+  hipLaunchKernelGGL(finish_kernel, dim3(words), dim3(256), 0, c->stream,
                      (const float2*)B.partial, (const double*)B.partial, B.err, B.order, n,
-                     a.tiles, c->N, f64 ? 1 : 0, B.out);
+                     a.tiles, c->N, f64 ? 1 : 0, B.out, nullptr, nullptr, nullptr);
   HIP_TRY(hipGetLastError());
-  unsigned long long count[2] = {0, 0};
+  unsigned long long count = 0;
   HIP_TRY(hipMemcpyAsync(out, B.out, (size_t)R * sizeof(double), hipMemcpyDefault, c->stream));
   HIP_TRY(hipMemcpyAsync(h_err, B.err, (size_t)R * sizeof(unsigned), hipMemcpyDeviceToHost,
                          c->stream));
-  HIP_TRY(hipMemcpyAsync(count, B.steps, sizeof(count), hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(hipMemcpyAsync(&count, B.steps, sizeof(count), hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
-  *repeated += count[1];
-  *steps = count[0] - *repeated;
+  *steps += count;
   return ANACOR_OK;
 }
 
@@ -1967,7 +1983,7 @@ static int retrace_marked(Context* c, const RunBuffers& B, const ReflRule* h_rul
 // rules and order of positions [0, first) (reflections [0, first)) go up and
 // their trace is launched, then prepare_rest() fills h_rules and h_order for
 // [first, R) on the host while the GPU traces the first part, and those go
-// up and are traced behind it.  h_redo: R words of host work space.
+// up and are traced behind it.  h_redo: the processing order, work space afterwards.
 static int trace_call(Context* c, const RunBuffers& B, const ReflRule* h_rules,
                       const int* h_order, int64_t R, int vpt, int layout, int flags, double* out,
                       PathRecord* d_paths, PathRecord* paths_out, unsigned* h_err, int* h_redo,
@@ -1994,11 +2010,12 @@ static int trace_call(Context* c, const RunBuffers& B, const ReflRule* h_rules,
     HIP_TRY(hipMemcpyAsync(B.order, h_order, (size_t)RA * sizeof(int), hipMemcpyHostToDevice,
                            c->stream));
     hipLaunchKernelGGL(clear_run_kernel, dim3((unsigned)((R + 255) / 256)), dim3(256), 0,
-                       c->stream, B.err, (int)R, B.steps);
+                       c->stream, B.err, (int)R, B.steps, skip ? B.refl_steps : nullptr);
     HIP_TRY(hipGetLastError());
   }
 
   TraceArgs a = trace_args(c, B, vpt, layout, flags, d_paths);
+  if (skip) a.steps = B.refl_steps;
 
   // a dispatch holds at most kMaxBlocks workgroups: a longer call runs as
   // several launches of whole reflections (consecutive processing positions)
@@ -2039,7 +2056,7 @@ static int trace_call(Context* c, const RunBuffers& B, const ReflRule* h_rules,
     hipLaunchKernelGGL(finish_kernel, dim3((unsigned)((R + 255) / 256)), dim3(256), 0, c->stream,
                        (const float2*)B.partial, (const double*)B.partial, B.err, B.order,
                        (int)R, (int)tiles, c->N, f64 ? 1 : 0, B.out,
-                       (const unsigned long long*)B.steps, B.h_steps);
+                       skip ? B.refl_steps : nullptr, B.steps, B.h_steps);
     HIP_TRY(hipGetLastError());
     if (!B.h_steps)
       HIP_TRY(hipMemcpyAsync(out, B.out, (size_t)R * sizeof(double), hipMemcpyDeviceToHost,
@@ -2054,7 +2071,8 @@ static int trace_call(Context* c, const RunBuffers& B, const ReflRule* h_rules,
   HIP_TRY(hipStreamSynchronize(c->stream));
   if (B.h_steps) {
     std::memcpy(out, B.out, (size_t)R * sizeof(double));
-    c->last_steps = *B.h_steps;
+    c->last_steps = 0;
+    for (size_t w = 0; w < CallRecord(R).waves; ++w) c->last_steps += B.h_steps[w];
   }
   HIP_TRY(hipEventElapsedTime(&c->last_kernel_ms, c->ev0, c->ev1));
   c->last_blocks = nblk;
@@ -2072,9 +2090,8 @@ static int trace_call(Context* c, const RunBuffers& B, const ReflRule* h_rules,
   }
   HIP_TRY(hipMemcpy(h_err, B.err, (size_t)R * sizeof(unsigned), hipMemcpyDeviceToHost));
   if (skip) {
-    unsigned long long repeated = 0;
-    rc = retrace_marked(c, B, h_rules, R, vpt, layout, flags, out, h_err, h_redo, &c->last_steps,
-                        &repeated);
+    rc = retrace_marked(c, B, h_rules, R, vpt, layout, flags, out, h_err, h_redo,
+                        &c->last_steps);
     if (rc) return rc;
   }
   for (int64_t i = 0; i < R; ++i)
@@ -2136,6 +2153,7 @@ static int run_rules(Context* c, const ReflRule* h_rules, int64_t R, int flags, 
     B.order = (int*)(d + r.order);
     B.err = (unsigned*)(d + r.err);
     B.steps = (unsigned long long*)(d + r.steps);
+    B.refl_steps = B.steps + 1;
     B.out = (double*)(h + r.out);
     B.partial = c->d_partial;
     B.h_steps = (unsigned long long*)(h + r.steps_out);
@@ -2172,6 +2190,7 @@ static int run_rules(Context* c, const ReflRule* h_rules, int64_t R, int flags, 
   B.out = c->d_out;
   B.partial = c->d_partial;
   B.steps = c->d_steps;
+  B.refl_steps = (unsigned long long*)c->d_out;
   if (RA < R)
     return trace_call(c, B, h_rules, c->h_order_pin.data(), R, vpt, layout, flags, out,
                       (PathRecord*)paths_buf.p, paths_out, nullptr, c->h_order_pin.data(), RA,
@@ -2758,6 +2777,7 @@ static int ctx_run_noalloc(Context* c, const double* s1, const double* omega, in
   B.err = (unsigned*)(base + kScratchErr);
   B.out = (double*)(base + kScratchOut);
   B.steps = (unsigned long long*)(base + kScratchSteps);
+  B.refl_steps = (unsigned long long*)B.out;
   return trace_call(c, B, g_noalloc_rules, g_noalloc_order, R, (int)vpt, c->layout, flags, out,
                     nullptr, nullptr, g_noalloc_err, g_noalloc_order);
 }
@@ -2897,7 +2917,7 @@ static int batch_create(const anacor_sample_t* in, int n, int full, int device, 
   BATCH_TRY(hipEventCreateWithFlags(&b->fork, hipEventDisableTiming));
   BATCH_TRY(hipEventCreate(&b->ev0));
   BATCH_TRY(hipEventCreate(&b->ev1));
-  BATCH_TRY(hipMalloc(&b->d_counters, 2 * sizeof(unsigned long long)));
+  BATCH_TRY(hipMalloc(&b->d_counters, sizeof(unsigned long long)));
 #undef BATCH_TRY
   *out = b;
   return ANACOR_OK;
@@ -2971,7 +2991,8 @@ static int batch_enqueue(Batch* b, bool capture, bool f64, int is_exp, long long
     t.partial32 = d.p32;
     t.partial64 = d.p64;
     t.err = d.err;
-    t.steps = b->d_counters;
+    const bool skip = use_skip(c, job.R);
+    t.steps = skip ? (unsigned long long*)d.out : b->d_counters;
     t.paths = nullptr;
     t.order = d.order;
     t.incd = c->d_incd;
@@ -2982,7 +3003,7 @@ static int batch_enqueue(Batch* b, bool capture, bool f64, int is_exp, long long
     // kernel, and a run whose rays need the guard is traced again without it
     const bool guard = !capture && job.guard;
     const int grid = (t.n_blocks + 7) / 8 * 8;
-    if (use_skip(c, job.R)) launch_skip(c, t, grid, f64, b->stream);
+    if (skip) launch_skip(c, t, grid, f64, b->stream);
     else dispatch_trace(t, grid, guard, b->full != 0,
                         raw_needs_wide(c) ? kLayoutWide : kLayoutRaw, f64, false,
                         !c->labels_over4, b->stream);
@@ -2993,7 +3014,7 @@ static int batch_enqueue(Batch* b, bool capture, bool f64, int is_exp, long long
   HIP_TRY(hipStreamWaitEvent(b->stream, b->fork, 0));
   if (total_refl > 0) {
     hipLaunchKernelGGL(batch_finish_kernel, dim3((unsigned)((total_refl + 255) / 256)),
-                       dim3(256), 0, b->stream, b->d_desc, S, f64 ? 1 : 0, total_refl);
+                       dim3(256), 0, b->stream, b->d_desc, S, f64 ? 1 : 0, total_refl, b->d_counters);
     HIP_TRY(hipGetLastError());
   }
   return ANACOR_OK;
@@ -3062,6 +3083,7 @@ static int batch_run(Batch* b, const double* const* s1, const double* const* ome
     d.R = (int)Ri;
     d.tiles = std::max(tiles, 1);
     d.vpt = vpt;
+    d.skip = c->N > 0 && use_skip(c, Ri) ? 1 : 0;
     d.p32 = (float2*)c->d_partial;
     d.p64 = (double*)c->d_partial;
     d.err = c->d_err;
@@ -3175,7 +3197,6 @@ static int batch_run(Batch* b, const double* const* s1, const double* const* ome
   }
   // reflections the skip walk marked: retraced sample by sample, on the
   // sample's own stream (the batch's has been waited for)
-  unsigned long long repeated = 0;
   for (int i = 0; i < S; ++i) {
     Context* c = b->samples[(size_t)i];
     note_walk(c, use_skip(c, R[i]));
@@ -3195,7 +3216,7 @@ static int batch_run(Batch* b, const double* const* s1, const double* const* ome
     B.steps = b->d_counters;
     rc = retrace_marked(c, B, c->h_rules.data(), R[i], b->h_desc[(size_t)i].vpt,
                         raw_needs_wide(c) ? kLayoutWide : kLayoutRaw, flags, out[i], err.data(),
-                        c->h_order_pin.data(), &b->last_steps, &repeated);
+                        c->h_order_pin.data(), &b->last_steps);
     if (rc != ANACOR_OK) return rc;
   }
   // report the first reflection the reference would have aborted on
@@ -4010,7 +4031,8 @@ static int ib_run(Context* c, int64_t R, int num_cls, int flags, double* out, do
   HIP_TRY(hipEventRecord(c->ev1, c->stream));
   hipLaunchKernelGGL(finish_kernel, dim3((unsigned)((R + 255) / 256)), dim3(256), 0, c->stream,
                      (const float2*)c->d_partial, (const double*)c->d_partial, c->d_err,
-                     c->d_order, (int)R, (int)tiles, c->N, f64 ? 1 : 0, c->d_out);
+                     c->d_order, (int)R, (int)tiles, c->N, f64 ? 1 : 0, c->d_out, nullptr,
+                     nullptr, nullptr);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipMemcpyAsync(out, c->d_out, (size_t)R * sizeof(double), hipMemcpyDeviceToHost,
                          c->stream));
