@@ -79,7 +79,7 @@ __device__ __forceinline__ int padded_label(const uint8_t* __restrict__ vol, int
   return vol[((size_t)cz * (Y + 2) + cy) * (X + 2) + cx];   // the raw layout's zero shell
 }
 
-// flag |= 1 when some listed voxel's label is not 3.
+// flag |= 4 when some listed voxel's label is not 3.
 __global__ void origin_label_kernel(const uint8_t* __restrict__ vol, int Y, int X,
                                     const int4* __restrict__ coords, int n,
                                     unsigned* __restrict__ flag) {
@@ -89,7 +89,7 @@ __global__ void origin_label_kernel(const uint8_t* __restrict__ vol, int Y, int 
     const int4 c = coords[i];
     other = vol[((size_t)(c.x + 1) * (Y + 2) + c.y + 1) * (X + 2) + c.z + 1] != 3;
   }
-  if (__any(other) && (threadIdx.x & (kWave - 1)) == 0) atomicOr(flag, 1u);
+  if (__any(other) && (threadIdx.x & (kWave - 1)) == 0) atomicOr(flag, 4u);
 }
 
 // Level 1: one wave per 64 voxels of a padded row; bits past the row are 1.

@@ -1353,7 +1353,9 @@ struct Context {
   bool labels_over4 = true;              // some label outside 0..4
   int4* d_coords = nullptr;
   int N = 0;
-  // skip walk: eight octants of free distances, the voxel list in its order
+  bool labels_listed3 = false;           // every listed voxel has label 3
+  // skip walk: eight octants of free distances and the voxel list in its order, all
+  // in one allocation at d_field
   uint8_t* d_field = nullptr;
   FieldShape field{};
   uint8_t* d_fine = nullptr;             // by cells: single labels; null: by voxels
@@ -1796,6 +1798,16 @@ static void note_walk(Context* c, bool skip) {
   c->last_retraced = 0;
 }
 
+// The skip walk's tables: entries per exit axis, and bytes in all.
+static int skip_table_entries(const Context* c, int axis) {
+  const int ext = axis == 0 ? c->Z : axis == 1 ? c->Y : c->X;
+  return std::max(ext - c->box_lo[axis], c->box_hi[axis]) + 1;
+}
+static unsigned skip_table_bytes(const Context* c, bool cells) {
+  const int n = skip_table_entries(c, 0) + skip_table_entries(c, 1) + skip_table_entries(c, 2);
+  return (unsigned)(n * (cells ? sizeof(CellField::Words) : sizeof(VoxelField::Words)));
+}
+
 // The skip walk's arguments and the bytes of its tables.
 static SkipArgs skip_args(const Context* c, unsigned* lds) {
   SkipArgs k;
@@ -1809,15 +1821,14 @@ static SkipArgs skip_args(const Context* c, unsigned* lds) {
   k.fine_shift = c->cells.shift;
   k.vox = c->d_skip_vox;
   k.index = c->d_skip_index;
-  const int ext[3] = {c->Z, c->Y, c->X};
   int entries = 0;
   for (int i = 0; i < 3; ++i) {
     k.lo[i] = c->box_lo[i];
     k.hi[i] = c->box_hi[i];
     k.at[i] = entries;
-    entries += std::max(ext[i] - k.lo[i], k.hi[i]) + 1;
+    entries += skip_table_entries(c, i);
   }
-  *lds = (unsigned)(entries * (cells ? sizeof(CellField::Words) : sizeof(VoxelField::Words)));
+  *lds = skip_table_bytes(c, cells);
   return k;
 }
 
@@ -2256,17 +2267,6 @@ static int upload_voxel_order(Context* c, int bz, int by, int bx) {
 // the caller asked for.
 static int upload_skip_voxels(Context* c) {
   const size_t n = c->h_coords.size();
-  for (int i = 0; i < 3; ++i) {
-    c->box_lo[i] = kSkipMaxExtent;
-    c->box_hi[i] = 0;
-  }
-  for (const int4& q : c->h_coords) {
-    const int p[3] = {q.x, q.y, q.z};
-    for (int i = 0; i < 3; ++i) {
-      c->box_lo[i] = std::min(c->box_lo[i], p[i]);
-      c->box_hi[i] = std::max(c->box_hi[i], p[i]);
-    }
-  }
   std::vector<int4> v(n);
   if (c->block[0] > 0 && !c->auto_block) {
     HIP_TRY(hipMemcpy(v.data(), c->d_coords, n * sizeof(int4), hipMemcpyDeviceToHost));
@@ -2308,9 +2308,7 @@ static int upload_skip_voxels(Context* c) {
     q = make_int4(z | (y << 16), x, (int)dilate_x(x + 1),
                   (int)(dilate_y(y + 1, f.hx) + (unsigned)((z + 1) * f.zs)));
   }
-  if (!c->d_skip_vox) HIP_TRY(hipMalloc(&c->d_skip_vox, n * sizeof(int4)));
   HIP_TRY(hipMemcpy(c->d_skip_vox, v.data(), n * sizeof(int4), hipMemcpyHostToDevice));
-  if (!c->d_skip_index) HIP_TRY(hipMalloc(&c->d_skip_index, n * sizeof(int)));
   HIP_TRY(hipMemcpy(c->d_skip_index, index.data(), n * sizeof(int), hipMemcpyHostToDevice));
   return ANACOR_OK;
 }
@@ -2347,128 +2345,145 @@ static int field_planes(Context* c, const uint8_t* vol, int Z, int Y, int X, int
   return ANACOR_OK;
 }
 
-// The field of voxels (planes in P) or, with its labels, of cells; false when
-// the offsets or the device memory do not allow it.
-static int voxel_field(Context* c, DeviceTemp& planes, bool* built) {
+// What the skip walk's field of a context takes.
+struct FieldPlan {
+  bool by_cells;
   FieldShape f;
-  f.Z = c->Z; f.Y = c->Y; f.X = c->X;
-  const int Z2 = c->Z + 2, Y2 = c->Y + 2, X2 = c->X + 2;
-  f.nbx = (X2 + 7) / 8;
-  f.nby = (Y2 + 15) / 16;
-  f.hx = 0;
-  while ((1 << f.hx) < f.nbx) ++f.hx;
-  const int64_t zs = (int64_t)f.nby << (7 + f.hx);
-  if (zs * Z2 >= (1ll << 31)) return ANACOR_OK;
-  f.zs = (int)zs;
-  f.bytes = zs * Z2;
-  f.wx = (X2 + 31) / 32;
-  const long long plane = (long long)Z2 * Y2 * f.wx;
-  if (hipMalloc(&planes.p, (size_t)plane * kLevels * sizeof(uint32_t)) != hipSuccess ||
-      hipMalloc(&c->d_field, (size_t)f.bytes * 8) != hipSuccess) {
-    (void)hipGetLastError();
-    c->d_field = nullptr;
-    return ANACOR_OK;
-  }
-  uint32_t* const P = (uint32_t*)planes.p;
-  const int rc = field_planes(c, c->d_vol, c->Z, c->Y, c->X, f.wx, P);
-  if (rc) return rc;
-  const long long threads = (long long)Z2 * f.nby * f.nbx * 16;
-  hipLaunchKernelGGL(field_pack_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
-                     c->stream, c->d_vol, f, P, plane, c->d_field);
-  HIP_TRY(hipGetLastError());
-  c->field = f;
-  *built = true;
-  return ANACOR_OK;
-}
+  CellShape cells;
+  size_t plane;                      // words of one bit plane
+  size_t fine, vox, index, bytes;    // the kept allocation: offsets behind the octants, size
+  size_t labels, work;               // the building's: offset behind the planes, size
+};
 
-static int cell_field(Context* c, DeviceTemp& planes, DeviceTemp& labels, bool* built) {
-  CellShape s;
-  s.Z = (c->Z + 5) / 4; s.Y = (c->Y + 5) / 4; s.X = (c->X + 5) / 4;   // of the padded volume
-  s.shift = c->labels_over3 ? 1 : 2;
-  const int nxt = (s.X + 7) / 8, nyt = (s.Y + 3) / 4, nzt = (s.Z + 3) / 4;
-  s.hx = 0;
-  while ((1 << s.hx) < nxt) ++s.hx;
-  s.tiles = nyt << s.hx;
-  const int64_t slots = (int64_t)nzt * s.tiles << 13;
-  if (slots >= (1ll << 32)) return ANACOR_OK;
-  FieldShape f{};
-  f.bytes = slots >> 6;
-  f.wx = (s.X + 2 + 31) / 32;
-  const long long ncell = (long long)(s.Z + 2) * (s.Y + 2) * (s.X + 2);
-  const long long plane = (long long)(s.Z + 2) * (s.Y + 2) * f.wx;
-  uint8_t* fine = nullptr;
-  if (hipMalloc(&planes.p, (size_t)plane * kLevels * sizeof(uint32_t)) != hipSuccess ||
-      hipMalloc(&labels.p, (size_t)ncell) != hipSuccess ||
-      hipMalloc(&c->d_field, (size_t)f.bytes * 8) != hipSuccess ||
-      hipMalloc(&fine, (size_t)(slots >> s.shift)) != hipSuccess) {
-    (void)hipGetLastError();
-    if (c->d_field) (void)hipFree(c->d_field);
-    c->d_field = nullptr;
-    return ANACOR_OK;
-  }
-  c->d_fine = fine;
-  c->fine_bytes = (size_t)(slots >> s.shift);
-  hipLaunchKernelGGL(cell_label_kernel, dim3((unsigned)((ncell + 255) / 256)), dim3(256), 0,
-                     c->stream, c->d_vol, c->Z, c->Y, c->X, s, (uint8_t*)labels.p,
-                     (uint32_t*)c->d_fine);
-  HIP_TRY(hipGetLastError());
-  uint32_t* const P = (uint32_t*)planes.p;
-  const int rc = field_planes(c, (const uint8_t*)labels.p, s.Z, s.Y, s.X, f.wx, P);
-  if (rc) return rc;
-  const long long threads = (long long)s.Z * s.Y * s.X;
-  hipLaunchKernelGGL(cell_pack_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
-                     c->stream, (const uint8_t*)labels.p, s, f.wx, P, plane, c->d_field, f.bytes);
-  HIP_TRY(hipGetLastError());
-  c->field = f;
-  c->cells = s;
-  *built = true;
-  return ANACOR_OK;
-}
-
-// The skip walk's field, where the walk's rules hold: no full_iteration, every
-// label in 0..4, every listed voxel of label 3, finite coefficients and voxel
-// edges whose squares are normal, extents within the tables and offsets.
-// Without the device memory for it the stepping kernels trace as before.
+// Whether the skip walk's rules hold, and the field's shape and sizes, before
+// anything is allocated: no full_iteration, every label in 0..4, every listed
+// voxel of label 3, finite coefficients and voxel edges whose squares are normal,
+// extents within the tables and offsets.
 // By cells in volumes past 160 MB, whose voxel field outgrows the caches by too
 // much (450x460x440, 20,000 voxels, 3,000 reflections: 6.3 ms by voxels, 7.6 by
 // cells; 700x640x680: 12.4 and 9.7 ms; 1000x1000x800: 53.9 and 29.7 ms).
 constexpr long long kCellVolume = 160ll << 20;
-static int field_build(Context* c) {
-  if (c->N == 0 || c->full || c->labels_over4 ||
+static bool plan_field(Context* c, FieldPlan* p) {
+  if (c->N == 0 || c->full || c->labels_over4 || !c->labels_listed3 ||
       std::max(c->Z, std::max(c->Y, c->X)) > kSkipMaxExtent)
-    return ANACOR_OK;
+    return false;
   for (double v : c->mu)
-    if (!(std::fabs(v) < 0x1p300)) return ANACOR_OK;
+    if (!(std::fabs(v) < 0x1p300)) return false;
   for (double v : c->vs)
-    if (!(std::fabs(v) > 0x1p-300 && std::fabs(v) < 0x1p300)) return ANACOR_OK;
-  // at most a quarter of the free memory (eight bytes per voxel, or a cell's
-  // eight and its labels), so that contexts created later still find theirs
+    if (!(std::fabs(v) > 0x1p-300 && std::fabs(v) < 0x1p300)) return false;
+  for (int i = 0; i < 3; ++i) {
+    c->box_lo[i] = kSkipMaxExtent;
+    c->box_hi[i] = 0;
+  }
+  for (const int4& q : c->h_coords) {
+    const int v[3] = {q.x, q.y, q.z};
+    for (int i = 0; i < 3; ++i) {
+      c->box_lo[i] = std::min(c->box_lo[i], v[i]);
+      c->box_hi[i] = std::max(c->box_hi[i], v[i]);
+    }
+  }
+  p->by_cells = c->vol_bytes > kCellVolume;
+  if (skip_table_bytes(c, p->by_cells) > kSkipTableBytes) return false;
+  const size_t n = c->h_coords.size();
+  FieldShape& f = p->f;
+  f = FieldShape{};
+  int64_t octants;
+  if (p->by_cells) {
+    CellShape& s = p->cells;
+    s.Z = (c->Z + 5) / 4; s.Y = (c->Y + 5) / 4; s.X = (c->X + 5) / 4;   // of the padded volume
+    s.shift = c->labels_over3 ? 1 : 2;
+    const int nxt = (s.X + 7) / 8, nyt = (s.Y + 3) / 4, nzt = (s.Z + 3) / 4;
+    s.hx = 0;
+    while ((1 << s.hx) < nxt) ++s.hx;
+    s.tiles = nyt << s.hx;
+    const int64_t slots = (int64_t)nzt * s.tiles << 13;
+    if (slots >= (1ll << 32)) return false;
+    f.bytes = slots >> 6;
+    f.wx = (s.X + 2 + 31) / 32;
+    p->plane = (size_t)(s.Z + 2) * (s.Y + 2) * f.wx;
+    octants = f.bytes * 8;
+    p->fine = (size_t)octants;
+    p->vox = p->fine + (size_t)(slots >> s.shift);
+    p->labels = p->plane * kLevels * sizeof(uint32_t);
+    p->work = p->labels + (size_t)(s.Z + 2) * (s.Y + 2) * (s.X + 2);
+  } else {
+    f.Z = c->Z; f.Y = c->Y; f.X = c->X;
+    const int Z2 = c->Z + 2, Y2 = c->Y + 2, X2 = c->X + 2;
+    f.nbx = (X2 + 7) / 8;
+    f.nby = (Y2 + 15) / 16;
+    f.hx = 0;
+    while ((1 << f.hx) < f.nbx) ++f.hx;
+    const int64_t zs = (int64_t)f.nby << (7 + f.hx);
+    if (zs * Z2 >= (1ll << 31)) return false;
+    f.zs = (int)zs;
+    f.bytes = zs * Z2;
+    f.wx = (X2 + 31) / 32;
+    p->plane = (size_t)Z2 * Y2 * f.wx;
+    octants = f.bytes * 8;
+    p->fine = 0;
+    p->vox = (size_t)octants;
+    p->labels = 0;
+    p->work = p->plane * kLevels * sizeof(uint32_t);
+  }
+  p->vox = (p->vox + 255) / 256 * 256;
+  p->index = p->vox + n * sizeof(int4);
+  p->bytes = p->index + n * sizeof(int);
+  return true;
+}
+
+// The skip walk's field, where its rules hold and it takes at most a quarter of
+// the free memory (eight octants at a byte per voxel, up to twice that where x
+// tiles are rounded up, or per cell with the single labels, and the building's bit
+// planes), so that contexts created later still find theirs.  Otherwise, or
+// without the memory, the stepping kernels trace as before.
+static int field_build(Context* c) {
+  FieldPlan p;
+  if (!plan_field(c, &p)) return ANACOR_OK;
   size_t free_bytes = 0, total = 0;
   if (hipMemGetInfo(&free_bytes, &total) != hipSuccess) {
     (void)hipGetLastError();
     return ANACOR_OK;
   }
-  const bool by_cells = c->vol_bytes > kCellVolume;
-  if ((size_t)c->vol_bytes * (by_cells ? 1 : 10) > free_bytes / 4) return ANACOR_OK;
-  DeviceTemp planes, labels, flag;
-  HIP_TRY(hipMalloc(&flag.p, sizeof(unsigned)));
-  HIP_TRY(hipMemsetAsync(flag.p, 0, sizeof(unsigned), c->stream));
-  hipLaunchKernelGGL(origin_label_kernel, dim3((unsigned)((c->N + 255) / 256)), dim3(256), 0,
-                     c->stream, c->d_vol, c->Y, c->X, c->d_coords, c->N, (unsigned*)flag.p);
-  HIP_TRY(hipGetLastError());
-  bool built = false;
-  int rc = by_cells ? cell_field(c, planes, labels, &built) : voxel_field(c, planes, &built);
-  if (!rc && built) rc = upload_skip_voxels(c);   // host work beside the kernels
-  if (rc) return rc;
-  unsigned other = 0;
-  HIP_TRY(hipMemcpyAsync(&other, flag.p, sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  unsigned lds = 0;
-  if (built) (void)skip_args(c, &lds);
-  if (built && (other || lds > kSkipTableBytes)) {
-    HIP_TRY(hipFree(c->d_field));
+  if (p.bytes + p.work > free_bytes / 4) return ANACOR_OK;
+  DeviceTemp work;
+  if (hipMalloc(&work.p, p.work) != hipSuccess ||
+      hipMalloc(&c->d_field, p.bytes) != hipSuccess) {
+    (void)hipGetLastError();
     c->d_field = nullptr;
+    return ANACOR_OK;
   }
+  c->field = p.f;
+  c->d_skip_vox = (int4*)(c->d_field + p.vox);
+  c->d_skip_index = (int*)(c->d_field + p.index);
+  uint32_t* const P = (uint32_t*)work.p;
+  const long long plane = (long long)p.plane;
+  int rc;
+  if (p.by_cells) {
+    const CellShape& s = p.cells;
+    c->cells = s;
+    c->d_fine = c->d_field + p.fine;
+    c->fine_bytes = (size_t)((long long)p.f.bytes << 6 >> s.shift);
+    uint8_t* const labels = (uint8_t*)work.p + p.labels;
+    const long long ncell = (long long)(s.Z + 2) * (s.Y + 2) * (s.X + 2);
+    hipLaunchKernelGGL(cell_label_kernel, dim3((unsigned)((ncell + 255) / 256)), dim3(256), 0,
+                       c->stream, c->d_vol, c->Z, c->Y, c->X, s, labels, (uint32_t*)c->d_fine);
+    HIP_TRY(hipGetLastError());
+    rc = field_planes(c, labels, s.Z, s.Y, s.X, p.f.wx, P);
+    if (rc) return rc;
+    const long long threads = (long long)s.Z * s.Y * s.X;
+    hipLaunchKernelGGL(cell_pack_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
+                       c->stream, labels, s, p.f.wx, P, plane, c->d_field, p.f.bytes);
+  } else {
+    rc = field_planes(c, c->d_vol, c->Z, c->Y, c->X, p.f.wx, P);
+    if (rc) return rc;
+    const long long threads = (long long)(c->Z + 2) * p.f.nby * p.f.nbx * 16;
+    hipLaunchKernelGGL(field_pack_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
+                       c->stream, c->d_vol, p.f, P, plane, c->d_field);
+  }
+  HIP_TRY(hipGetLastError());
+  rc = upload_skip_voxels(c);        // host work beside the kernels
+  if (rc) return rc;
+  HIP_TRY(hipStreamSynchronize(c->stream));
   return ANACOR_OK;
 }
 
@@ -2532,36 +2547,6 @@ static int ctx_create(const uint8_t* vol, const int64_t shape[3], const int64_t*
     for (int i = 0; i < 4; ++i) c->mu[i] = mu ? mu[i] : 0.0;
     c->full = full;
     c->N = (int)n;
-    {  // upload, scan which label ranges the volume holds (layout choice, walk
-       // variant), and lay it out with its zero shell
-      DeviceTemp in, flag;   // freed on every way out of this block
-      unsigned h_flag = 0;
-      HIP_TRY(hipMalloc(&in.p, nvox));
-      HIP_TRY(hipMemcpy(in.p, vol, nvox, hipMemcpyHostToDevice));
-      HIP_TRY(hipMalloc(&flag.p, sizeof(unsigned)));
-      HIP_TRY(hipMemsetAsync(flag.p, 0, sizeof(unsigned), c->stream));
-      hipLaunchKernelGGL(label_scan_kernel, dim3(2048), dim3(256), 0, c->stream,
-                         (const uint8_t*)in.p, (long long)nvox, (unsigned*)flag.p);
-      HIP_TRY(hipGetLastError());
-      HIP_TRY(hipMalloc(&c->d_vol, npad));
-      c->vol_bytes = (long long)npad;
-      hipLaunchKernelGGL(shell_volume_kernel, dim3(4096), dim3(256), 0, c->stream,
-                         (const uint8_t*)in.p, c->Z, c->Y, c->X, (long long)npad, c->d_vol);
-      HIP_TRY(hipGetLastError());
-      HIP_TRY(hipMemcpyAsync(&h_flag, flag.p, sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
-      HIP_TRY(hipStreamSynchronize(c->stream));
-      c->labels_over3 = (h_flag & 1u) != 0;
-      c->labels_over4 = (h_flag & 2u) != 0;
-    }
-    {  // increments as doubles: a walk reaches at most extent + 1 plus one
-       // unrolled group; 32 spare entries
-      const int m = std::max(c->Z, std::max(c->Y, c->X)) + 32;
-      std::vector<double> h((size_t)m);
-      for (int i = 0; i < m; ++i) h[(size_t)i] = (double)i;
-      HIP_TRY(hipMalloc(&c->d_incd, (size_t)m * sizeof(double)));
-      HIP_TRY(hipMemcpy(c->d_incd, h.data(), (size_t)m * sizeof(double), hipMemcpyHostToDevice));
-      c->incd_last = m - 1;
-    }
     c->h_coords.resize((size_t)n);
     for (int64_t i = 0; i < n; ++i) {
       const int64_t z = coords ? coords[3 * i] : coords32[3 * i];
@@ -2577,8 +2562,44 @@ static int ctx_create(const uint8_t* vol, const int64_t shape[3], const int64_t*
     if (const char* e = std::getenv("ANACOR_VOXEL_BLOCK"))
       if (std::sscanf(e, "%d,%d,%d", &blk[0], &blk[1], &blk[2]) != 3) blk[0] = blk[1] = blk[2] = 0;
     c->auto_block = std::getenv("ANACOR_VOXEL_BLOCK") == nullptr;
-    const int rc = upload_voxel_order(c, blk[0], blk[1], blk[2]);
-    if (rc) return rc;
+    {  // upload, scan which label ranges the volume and the listed voxels hold
+       // (layout choice, walk variant), and lay it out with its zero shell
+      DeviceTemp in, flag;   // freed on every way out of this block
+      unsigned h_flag = 0;
+      HIP_TRY(hipMalloc(&in.p, nvox));
+      HIP_TRY(hipMemcpy(in.p, vol, nvox, hipMemcpyHostToDevice));
+      HIP_TRY(hipMalloc(&flag.p, sizeof(unsigned)));
+      HIP_TRY(hipMemsetAsync(flag.p, 0, sizeof(unsigned), c->stream));
+      hipLaunchKernelGGL(label_scan_kernel, dim3(2048), dim3(256), 0, c->stream,
+                         (const uint8_t*)in.p, (long long)nvox, (unsigned*)flag.p);
+      HIP_TRY(hipGetLastError());
+      HIP_TRY(hipMalloc(&c->d_vol, npad));
+      c->vol_bytes = (long long)npad;
+      hipLaunchKernelGGL(shell_volume_kernel, dim3(4096), dim3(256), 0, c->stream,
+                         (const uint8_t*)in.p, c->Z, c->Y, c->X, (long long)npad, c->d_vol);
+      HIP_TRY(hipGetLastError());
+      const int rc = upload_voxel_order(c, blk[0], blk[1], blk[2]);   // beside the kernels
+      if (rc) return rc;
+      if (c->N > 0) {
+        hipLaunchKernelGGL(origin_label_kernel, dim3((unsigned)((c->N + 255) / 256)), dim3(256), 0,
+                           c->stream, c->d_vol, c->Y, c->X, c->d_coords, c->N, (unsigned*)flag.p);
+        HIP_TRY(hipGetLastError());
+      }
+      HIP_TRY(hipMemcpyAsync(&h_flag, flag.p, sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
+      HIP_TRY(hipStreamSynchronize(c->stream));
+      c->labels_over3 = (h_flag & 1u) != 0;
+      c->labels_over4 = (h_flag & 2u) != 0;
+      c->labels_listed3 = (h_flag & 4u) == 0;
+    }
+    {  // increments as doubles: a walk reaches at most extent + 1 plus one
+       // unrolled group; 32 spare entries
+      const int m = std::max(c->Z, std::max(c->Y, c->X)) + 32;
+      std::vector<double> h((size_t)m);
+      for (int i = 0; i < m; ++i) h[(size_t)i] = (double)i;
+      HIP_TRY(hipMalloc(&c->d_incd, (size_t)m * sizeof(double)));
+      HIP_TRY(hipMemcpy(c->d_incd, h.data(), (size_t)m * sizeof(double), hipMemcpyHostToDevice));
+      c->incd_last = m - 1;
+    }
     // a one-shot call builds the field where its steps (about a third of the
     // extents' sum per pair) cost more than the field and its allocations do,
     // some 1.3 ms: 150x201x187, 6.5e8 steps 1.6 ms per call without it and 2.4
@@ -2606,9 +2627,6 @@ static void ctx_destroy(Context* c) {
   if (c->d_pack) (void)hipFree(c->d_pack);
   if (c->d_coords) (void)hipFree(c->d_coords);
   if (c->d_field) (void)hipFree(c->d_field);
-  if (c->d_fine) (void)hipFree(c->d_fine);
-  if (c->d_skip_vox) (void)hipFree(c->d_skip_vox);
-  if (c->d_skip_index) (void)hipFree(c->d_skip_index);
   if (c->d_rules) (void)hipFree(c->d_rules);
   if (c->d_partial) (void)hipFree(c->d_partial);
   if (c->d_err) (void)hipFree(c->d_err);
