@@ -63,10 +63,6 @@ __device__ __forceinline__ float sigmoidf_(float z) {
   return __builtin_amdgcn_rcpf(1.0f + __expf(-z));
 }
 __device__ __forceinline__ float silu(float z) { return z * sigmoidf_(z); }
-__device__ __forceinline__ float silu_grad(float z) {
-  const float s = sigmoidf_(z);
-  return s * (1.0f + z * (1.0f - s));
-}
 
 // MFMA 16x16x32 operand layout: lane l supplies row (A) / column (B) l % 16
 // and the 8 k values 8 (l / 16) .. 8 (l / 16) + 7; the accumulator of lane l

@@ -3884,9 +3884,11 @@ static void launch_ib(const IbArgs& a, int grid, hipStream_t s) {
 static void dispatch_ib(const IbArgs& a, int grid, int layout, bool f64, bool lengths, bool exact,
                         hipStream_t s) {
   using Fn = void (*)(const IbArgs&, int, hipStream_t);
-#define IB_ROW(LAYOUT, F64)                                               \
-  {{launch_ib<LAYOUT, F64, false, false>, launch_ib<LAYOUT, F64, false, true>}, \
-   {launch_ib<LAYOUT, F64, true, false>, launch_ib<LAYOUT, F64, true, true>}}
+  // (extents of the exact search never need the wide layout)
+#define IB_ROW(LAYOUT, F64)                                                                     \
+  {{launch_ib<LAYOUT, F64, false, false>, launch_ib<LAYOUT, F64, false, LAYOUT != kLayoutWide>}, \
+   {launch_ib<LAYOUT, F64, true, false>, launch_ib<LAYOUT, F64, true, LAYOUT != kLayoutWide>}}
+  static_assert((int64_t)(kIbExactExtent + 2) * (kIbExactExtent + 2) < (1 << 23), "raw_needs_wide");
   static const Fn table[4][2][2][2] = {
       {IB_ROW(kLayoutRaw, false), IB_ROW(kLayoutRaw, true)},
       {IB_ROW(kLayoutWide, false), IB_ROW(kLayoutWide, true)},
