@@ -14,6 +14,19 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an MI355X (HIP device)")
 
 
+def pytest_collection_modifyitems(config, items):
+    """Tests against the reference's own C build are skipped, with the reason, where
+    it is neither built nor can be (its sources are not there to compile)."""
+    from oracle.oracle import REF_SO, REF_SRC
+    if os.path.exists(REF_SO) or os.path.isdir(REF_SRC):
+        return
+    skip = pytest.mark.skip(reason=f"needs the reference's own build: {REF_SO} is missing and so "
+                                   f"are the sources of `make -C oracle ref` ({REF_SRC})")
+    for item in items:
+        if "reference" in getattr(item, "fixturenames", ()):
+            item.add_marker(skip)
+
+
 def load_npz(name):
     return np.load(os.path.join(GOLDEN, name), allow_pickle=False)
 
