@@ -4414,13 +4414,15 @@ static double single_impl(int64_t* coord_list, int64_t len_coord_list, const dou
   const int flags = ((char)IsExp == 1) ? 0 : ANACOR_FLAG_NO_EXP;
   {
     std::lock_guard<std::mutex> lk(c->mu_run);
-    if (hipSetDevice(c->device) == hipSuccess &&
-        c->h_rules.reserve(CallRecord(1).records()) == hipSuccess) {
+    auto trace = [&]() -> int {
+      HIP_TRY(hipSetDevice(c->device));
+      HIP_TRY(c->h_rules.reserve(CallRecord(1).records()));
       host_setup_rotated(rotated_s1, xray, max_dim(c), c->h_rules.data(), nullptr);
-      const int rc = run_rules(c, c->h_rules.data(), 1, flags, &out, nullptr);
-      if (rc != ANACOR_OK && rc != ANACOR_ERR_GEOMETRY)
-        fprintf(stderr, "anacor: ray_tracing_single: %s\n", g_err);
-    }
+      return run_rules(c, c->h_rules.data(), 1, flags, &out, nullptr);
+    };
+    const int rc = trace();
+    if (rc != ANACOR_OK && rc != ANACOR_ERR_GEOMETRY)
+      fprintf(stderr, "anacor: ray_tracing_single: %s\n", g_err);
   }
   ctx_destroy(c);
   return out;
