@@ -21,7 +21,8 @@
 // them in LDS for its reflection and notes the first increment of each face
 // that is too close to call.  A lane that would use it, or whose geometry the
 // table does not cover in any other way, marks its reflection (kRayRedo), and
-// the host traces such reflections with the stepping kernels.
+// the host traces such reflections with the stepping kernels.  Where the
+// reference aborts, the walk raises the same error itself.
 //
 // Layout of one octant's field: the volume with a one-voxel replicated shell
 // (the reference clamps a stepped coordinate to the volume), tiles of 8 (x) by
@@ -32,14 +33,14 @@
 // words fill with ones so that carries run through, and one bit select merges
 // them.
 //
-// What bounds it: VALU issue (71% of one instruction per SIMD every 4 cycles)
-// and the texture addresser (79% busy, 20 cycles per 64-lane byte gather), at
+// What bounds it: VALU issue (75% of one instruction per SIMD every 4 cycles)
+// and the texture addresser (81% busy, 20 cycles per 64-lane byte gather), at
 // once.  256^3, 25,323 voxels, 20,000 reflections: 62.5 ms stepping, 21.6 ms
 // with the first form of this kernel (507 VALU instructions per wave and ray,
 // five waves per SIMD), 17.7 ms with nine instructions per gather and eight
 // waves, 13.8 ms with the diffracted ray leading the sort and rows of lanes
-// within cubes.  181x203x227, 5,003 voxels, 4,001 reflections, FP64 mean: 5.1
-// and 0.95 ms.
+// within cubes, 13.4 ms with the errors in LDS.  181x203x227, 5,003 voxels, 4,001
+// reflections, FP64 mean: 5.1 and 0.95 ms.
 
 constexpr unsigned kRayRedo = 1u << 30;   // err bit: trace with the stepping kernels
 constexpr int kSkipMaxExtent = 2046;      // coordinates in 16 bits, tables in LDS

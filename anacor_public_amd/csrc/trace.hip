@@ -2602,9 +2602,9 @@ static int ctx_create(const uint8_t* vol, const int64_t shape[3], const int64_t*
     }
     // a one-shot call builds the field where its steps (about a third of the
     // extents' sum per pair) cost more than the field and its allocations do,
-    // some 1.3 ms: 150x201x187, 6.5e8 steps 1.6 ms per call without it and 2.4
-    // with it, 1.6e9 steps 3.0 and 2.7; 100^3, 2e8 steps 0.67 and 0.84; 256^3,
-    // 1.3e9 steps 4.0 and 2.4, 5.1e9 steps 14.2 and 3.9
+    // some 1.1 ms: 150x201x187, 6.5e8 steps 1.9 ms per call without it and 2.5
+    // with it, 1.6e9 steps 3.3 and 2.6; 100^3, 2e8 steps 0.84 and 0.80; 256^3,
+    // 1.3e9 steps 4.4 and 2.4, 5.1e9 steps 14.6 and 3.6
     const double steps = (double)reflections * (double)n * (c->Z + c->Y + c->X) / 3.0;
     if (reflections > 0 && steps < 1e9 + 30.0 * (double)nvox) return ANACOR_OK;
     return field_build(c);

@@ -257,8 +257,8 @@ class Tracer:
         return int(self._lib.anacor_ctx_get_layout(self.handle))
 
     def set_voxel_block(self, bz: int, by: int, bx: int):
-        """Group crystal voxels into waves by (bz, by, bx) voxel blocks
-        ((0, 0, 0): Morton order)."""
+        """Group crystal voxels into waves by (bz, by, bx) voxel blocks ((0, 0, 0):
+        Morton order, of voxels or, in the walk over free distances, of small cubes)."""
         _lib.check(self._lib.anacor_ctx_set_voxel_block(self.handle, int(bz), int(by), int(bx)),
                    self._lib)
 

@@ -134,7 +134,10 @@ int anacor_ctx_get_work_shape(const anacor_ctx *ctx, int block[3], int *tile, in
  * 0..4 matter to it).  The packed copy is built on the GPU on first use; the
  * raw volume stays resident (path records and the batched path use it).  The
  * automatic layout's means may differ from the others' in the last bits of a few
- * FP64 operations per ray; a requested layout always steps. */
+ * FP64 operations per ray; a requested layout always steps.  The automatic one
+ * also steps in calls of at most 2^20 (reflection, voxel) pairs on volumes with
+ * Z + Y + X <= 256, so there a part of a call may differ from the whole in those
+ * bits (anacor_ctx_last_walk tells which way a call went). */
 #define ANACOR_LAYOUT_AUTO   (-1)  /* the walk over free distances where it applies, else
                                      * bricks above 64 MB; ANACOR_VOLUME_LAYOUT=raw|brick overrides */
 #define ANACOR_LAYOUT_RAW    0     /* uint8 [z][y][x] */
@@ -147,7 +150,9 @@ int anacor_ctx_get_layout(const anacor_ctx *ctx);
 
 /* Grouping of the crystal voxels into waves: blocks of bz x by x bx voxels in
  * z, y, x order, lanes along x inside a block; (0, 0, 0) selects Morton
- * order.  Affects speed only, never results beyond the FP32 summation order. */
+ * order, in the walk over free distances Morton-ordered cubes of about a wave's
+ * voxels with rows along x inside.  Affects speed only, never results beyond the
+ * summation order of the voxels' terms. */
 int anacor_ctx_set_voxel_block(anacor_ctx *ctx, int bz, int by, int bx);
 
 /* Mean absorption factor of R reflections (s1 [R][3], omega [R], DIALS frame)
